@@ -114,15 +114,61 @@ void upload(DevBuf& buf, const std::vector<T>& host) {
   }
 }
 
+// Passes of the row FFT kernels for scalar fields: primes above 13 first, largest first (the
+// first pass of such a radix shares its sums between outputs and has no
+// twiddles), then the radices 2..16 of least modelled cost.  A pass costs its
+// LDS round trip (~100 wave instructions) plus, per round of 64 butterflies,
+// ~20 R for addresses, twiddles and LDS accesses and its DFT (direct for 5,
+// 7, 11, 13, ~5 R log2 R otherwise); with N = 1152 this takes 12 x 12 x 8
+// over 4 x 4 x 4 x 2 x 3 x 3.
+double pass_cost(int n, int r) {
+  const int rounds = (n / r + 63) / 64;
+  double dft = 5.0 * r * std::log2((double)r);
+  for (int p : {5, 7, 11, 13})
+    if (r % p == 0) dft += (r / p) * 2.0 * (p - 1) * (p - 1);
+  return 100.0 + rounds * (20.0 * r + dft);
+}
+
+void best_passes(int n, int rest, int largest, std::vector<int>& now, double cost,
+                 std::vector<int>& best, double& least) {
+  if (cost >= least) return;
+  if (rest == 1) {
+    best = now;
+    least = cost;
+    return;
+  }
+  for (int r = largest; r >= 2; --r) {
+    if (rest % r) continue;
+    now.push_back(r);
+    best_passes(n, rest / r, r, now, cost + pass_cost(n, r), best, least);
+    now.pop_back();
+  }
+}
+
 std::vector<int> factor_radices(int n) {
   std::vector<int> r;
+  int rest = n;
+  for (int p = 2; p <= rest; ++p)
+    while (rest % p == 0) {
+      if (p > 13) r.insert(r.begin(), p);
+      rest /= p;
+    }
+  int smooth = n;
+  for (int p : r) smooth /= p;
+  std::vector<int> now, best;
+  double least = 1e300;
+  best_passes(n, smooth, 16, now, 0.0, best, least);
+  r.insert(r.end(), best.begin(), best.end());
+  return r;
+}
+
+// Passes for the vector operators' rows: fours, a two, threes and the other
+// primes in rising order.
+std::vector<int> plain_radices(int n) {
+  std::vector<int> r;
   while (n % 4 == 0) { r.push_back(4); n /= 4; }
-  while (n % 2 == 0) { r.push_back(2); n /= 2; }
-  while (n % 3 == 0) { r.push_back(3); n /= 3; }
-  for (int p = 5; n > 1; p += 2) {
+  for (int p = 2; n > 1; ++p)
     while (n % p == 0) { r.push_back(p); n /= p; }
-    if (p * p > n && n > 1) { r.push_back(n); n = 1; }
-  }
   return r;
 }
 
@@ -156,8 +202,6 @@ struct arwen_sht_plan {
   DevBuf scale_fold_vec64_cos, scale_inv_acos64;
   DevBuf low_syn[3], low_ana[3];
   sht::FftPlan fft{};
-  int rp_fold = 4, rp_fold_vec = 4, rp_unfold = 4;  // folded rows (wavefronts) per FFT block
-  int fft_gpb = 2;                                   // row groups walked by one FFT block
   // single-operation batches by (op, count, stream), most recent first
   std::list<std::pair<std::tuple<int, int, void*>, arwen_sht_batch*>> cache;
   std::mutex cache_mu;
@@ -282,11 +326,15 @@ void build_plan(arwen_sht_plan* P, const arwen_sht_plan_desc* d) {
             "legendre_tables launch");
 
   // FFT plan.
-  std::vector<int> rad = factor_radices(P->nlon);
-  if ((int)rad.size() > sht::kMaxStages) fail(ARWEN_SHT_EINVAL, "nlon has too many factors");
   P->fft.N = P->nlon;
-  P->fft.nstages = (int)rad.size();
-  for (size_t s = 0; s < rad.size(); ++s) P->fft.radix[s] = rad[s];
+  for (auto* passes : {&P->fft.scalar, &P->fft.vector}) {
+    const bool direct = passes == &P->fft.vector;
+    const std::vector<int> rad = direct ? plain_radices(P->nlon) : factor_radices(P->nlon);
+    if ((int)rad.size() > sht::kMaxStages) fail(ARWEN_SHT_EINVAL, "nlon has too many factors");
+    passes->n = (int)rad.size();
+    passes->direct = direct;
+    for (size_t s = 0; s < rad.size(); ++s) passes->radix[s] = rad[s];
+  }
   std::vector<float2> tw(P->nlon);
   for (int k = 0; k < P->nlon; ++k) {
     double ang = -2.0 * M_PI * (double)k / (double)P->nlon;
@@ -303,26 +351,13 @@ void build_plan(arwen_sht_plan* P, const arwen_sht_plan_desc* d) {
     upload(P->d_tw64, tw64);
     P->fft.tw64 = P->d_tw64.as<double2>();
   }
-  // Wavefronts (folded rows) per FFT block: as many as fit 80 KiB, so two
-  // blocks share a CU; one row per block up to the device's whole LDS where
-  // a single row needs more (nlon = 3072: 96 KiB for a u,v row pair).
   {
     int lds_max = 65536;
     (void)hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, P->device);
-    const size_t budget = std::min<size_t>((size_t)lds_max, 81920);
-    size_t need = budget;
-    auto pick = [&](auto bytes) {
-      int rp = 4;
-      while (rp > 1 && bytes(rp) > budget) rp /= 2;
-      if (bytes(rp) > (size_t)lds_max)
-        fail(ARWEN_SHT_EINVAL, "nlon=" + std::to_string(P->nlon) + " needs more LDS than the device has");
-      need = std::max(need, bytes(rp));
-      return rp;
-    };
-    P->rp_fold = pick([&](int rp) { return sht_fold_lds_bytes(P->nlon, T, 0, rp); });
-    P->rp_fold_vec = pick([&](int rp) { return sht_fold_lds_bytes(P->nlon, T, 1, rp); });
-    P->rp_unfold = pick([&](int rp) { return sht_unfold_lds_bytes(P->nlon, T, rp); });
-    hip_check(sht_fft_allow_lds(need, (size_t)lds_max), "FFT LDS attribute");
+    // the longest row a plan takes: 32 bytes of LDS per longitude
+    if ((size_t)P->nlon * 4 * sizeof(float2) > (size_t)lds_max)
+      fail(ARWEN_SHT_EINVAL, "nlon=" + std::to_string(P->nlon) + " needs more LDS than the device has");
+    hip_check(sht_fft_allow_lds((size_t)lds_max), "FFT LDS attribute");
     if (P->m0 > 0) hip_check(sht_low_allow_lds((size_t)lds_max), "low-order LDS attribute");
     // wave-resident FFTs (N = 64 L) when their LDS fits the device
     const int L = sht_fft_wave_L(P->nlon);
@@ -803,10 +838,6 @@ void setup_job(arwen_sht_batch* B, JobState* js, bool prepare) {
       ua.nlat = P->nlat;
       ua.JH = P->JH;
       ua.JHP = P->JHP;
-      ua.rp = P->rp_unfold;
-      ua.ngroups = (P->JH + ua.rp - 1) / ua.rp;
-      ua.gpb = P->fft_gpb;
-      ua.nchunks = (ua.ngroups + ua.gpb - 1) / ua.gpb;
       ua.job.waist = waist.as<float>();
       ua.job.grid = static_cast<float*>(grid);
       ua.job.rowscale = sc.as<float>();
@@ -846,6 +877,8 @@ void setup_job(arwen_sht_batch* B, JobState* js, bool prepare) {
     } else if (J.op == ARWEN_SHT_OP_UV_FROM_VORDIV) {
       unfold(js->waist_a, J.out0, 0, 4, P->scale_inv_a, 0);
       unfold(js->waist_a, J.out1, 2, 4, P->scale_inv_a, 0);
+      for (size_t k = B->unfolds.size() - 2; k < B->unfolds.size(); ++k)
+        B->unfolds[k].job.wind = 1;
       if (recp)  // the recurrence form's orders: a cos(phi) (u, v)
         for (size_t k = B->unfolds.size() - 2; k < B->unfolds.size(); ++k) {
           B->unfolds[k].job.rowscale_hi = P->scale_inv_acos.as<float>();
@@ -893,10 +926,6 @@ void setup_job(arwen_sht_batch* B, JobState* js, bool prepare) {
     fa.nlat = P->nlat;
     fa.JH = P->JH;
     fa.JHP = P->JHP;
-    fa.rp = vec ? P->rp_fold_vec : P->rp_fold;
-    fa.ngroups = P->JHP / fa.rp;
-    fa.gpb = P->fft_gpb;
-    fa.nchunks = (fa.ngroups + fa.gpb - 1) / fa.gpb;
     fa.job.grid0 = static_cast<const float*>(J.in0);
     fa.job.grid1 = static_cast<const float*>(J.in1);
     fa.job.waist0 = js->waist_a.as<float>();
@@ -905,6 +934,7 @@ void setup_job(arwen_sht_batch* B, JobState* js, bool prepare) {
     fa.job.col0 = 0;
     fa.job.ldw = P->ldw;
     fa.job.vector = vec ? 1 : 0;
+    fa.job.fstride = ncol;
     fa.job.goff = J.grid_offset;
     const bool low = J.op == ARWEN_SHT_OP_VORDIV_FROM_UV && P->m0 > 0;
     // without FP64 low orders (plain FP32) on a wave-resident grid: the
@@ -948,7 +978,20 @@ void setup_job(arwen_sht_batch* B, JobState* js, bool prepare) {
       la.nlev = n;
       B->low_anas.push_back(la);
     } else if (!from_waist(J.op)) {
-      B->folds.push_back(fa);
+      if (vec && !P->fft.wave_L) {
+        // one component per launch: i U to level columns 2, 3, i V to 0, 1
+        for (int f = 0; f < 2; ++f) {
+          sht::FoldArgs fh = fa;
+          fh.job.grid0 = static_cast<const float*>(f == 0 ? J.in0 : J.in1);
+          fh.job.grid1 = nullptr;
+          fh.job.vector = 0;
+          fh.job.imul = 1;
+          fh.job.col0 = f == 0 ? 2 : 0;
+          B->folds.push_back(fh);
+        }
+      } else {
+        B->folds.push_back(fa);
+      }
       if (prepare) B->fft_bytes += (vec ? 2.0 : 1.0) * n * fftb;
     }
     const DataRef wst{js->waist_a.as<char>()};

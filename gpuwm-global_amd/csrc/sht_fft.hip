@@ -5,11 +5,11 @@
 // (2*field + re/im), fp32 in every precision mode (the split modes cut the
 // analysis waist into bf16 pieces as the GEMM loads it).
 //
-// A block holds `rp` wavefronts; wavefront w owns folded row i0 + w (the
-// mirror pair north = nlat-1-i, south = i) and runs its own FFT in its own
-// LDS slice, so rp FFTs advance together between the block barriers of the
-// Stockham passes.  Neighbouring wavefronts write neighbouring runs of each
-// m-tile (4 orders per latitude), which meet in L2 as whole sectors.
+// One wavefront transforms one mirror row pair (north = nlat-1-i, south = i)
+// in its own LDS slice; a block holds up to eight consecutive rows, so that
+// a waist run of rows x 4 orders is one whole line.  N = 64 L runs
+// wave-resident (registers and two LDS transposes), any other N in Stockham
+// passes in LDS.
 //
 // Two real rows ride one complex FFT of length N = nlon:
 //   z = north + i*south,  X_N[m] = (Z[m] + conj Z[N-m]) / 2,
@@ -20,9 +20,8 @@
 // zero-padded spectrum scaled by nlon (transform.py:1654-1702), i.e.
 // f = Re G_0 + 2 Re sum_{m>=1} G_m e^{i m lambda}.
 //
-// Stockham autosort, radix 4/2/3 butterflies and a generic-radix DFT for any
-// other prime factor, twiddles from a table of e^{-2 pi i k/N} computed in
-// FP64 and rounded once.
+// Twiddles come from a table of e^{-2 pi i k/N} computed in FP64 and rounded
+// once.
 #include <algorithm>
 #include <map>
 #include <mutex>
@@ -58,363 +57,8 @@ __device__ __forceinline__ C twiddle(const C* tw, int k, int sign) {
   return sign < 0 ? t : cconj(t);
 }
 
-template <int R>
-__device__ __forceinline__ void dft_small(float2* v, int sign) {
-  if constexpr (R == 2) {
-    float2 a = v[0], b = v[1];
-    v[0] = cadd(a, b);
-    v[1] = csub(a, b);
-  } else if constexpr (R == 4) {
-    float2 a0 = cadd(v[0], v[2]), a1 = csub(v[0], v[2]);
-    float2 a2 = cadd(v[1], v[3]), a3 = csub(v[1], v[3]);
-    // a3 times -i (forward) or +i (inverse)
-    float2 a3r = sign < 0 ? make_float2(a3.y, -a3.x) : make_float2(-a3.y, a3.x);
-    v[0] = cadd(a0, a2);
-    v[2] = csub(a0, a2);
-    v[1] = cadd(a1, a3r);
-    v[3] = csub(a1, a3r);
-  } else if constexpr (R == 3) {
-    const float c = -0.5f;
-    const float s = (sign < 0 ? -1.0f : 1.0f) * 0.86602540378443864676f;
-    float2 t1 = cadd(v[1], v[2]);
-    float2 t2 = csub(v[1], v[2]);
-    float2 m1 = make_float2(v[0].x + c * t1.x, v[0].y + c * t1.y);
-    float2 m2 = make_float2(-s * t2.y, s * t2.x);  // i*s*t2
-    v[0] = cadd(v[0], t1);
-    v[1] = cadd(m1, m2);
-    v[2] = csub(m1, m2);
-  }
-}
-
-// One Stockham pass of radix R over one wavefront's N points.
-template <int R>
-__device__ void stockham_pass(const float2* __restrict__ in, float2* __restrict__ out, int N,
-                              int Ns, const float2* tw, int sign, int lane) {
-  const int nb = N / R;
-  const int tstep = N / (Ns * R);
-  for (int j = lane; j < nb; j += kWave) {
-    const int k = j % Ns;
-    float2 v[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      float2 x = in[j + r * nb];
-      v[r] = (r == 0 || k == 0) ? x : cmul(x, twiddle(tw, r * k * tstep, sign));
-    }
-    dft_small<R>(v, sign);
-    const int d = (j / Ns) * Ns * R + k;
-#pragma unroll
-    for (int r = 0; r < R; ++r) out[d + r * Ns] = v[r];
-  }
-}
-
-__device__ void stockham_pass_generic(const float2* __restrict__ in, float2* __restrict__ out,
-                                      int N, int Ns, int R, const float2* tw, int sign,
-                                      int lane) {
-  const int nb = N / R;
-  const int rstep = N / R;  // twiddle stride of the R-point DFT
-  const int tstep = N / (Ns * R);
-  for (int j = lane; j < nb; j += kWave) {
-    const int k = j % Ns;
-    const int d = (j / Ns) * Ns * R + k;
-    for (int q = 0; q < R; ++q) {
-      float2 acc = make_float2(0.f, 0.f);
-      for (int r = 0; r < R; ++r) {
-        float2 x = in[j + r * nb];
-        if (r > 0 && k > 0) x = cmul(x, twiddle(tw, r * k * tstep, sign));
-        if (r > 0 && q > 0) x = cmul(x, twiddle(tw, ((r * q) % R) * rstep, sign));
-        acc = cadd(acc, x);
-      }
-      out[d + q * Ns] = acc;
-    }
-  }
-}
-
-// FFT of N points in buf0 (one wavefront's slice); every wavefront of the
-// block runs the same pass sequence, so block barriers separate the passes.
-// Returns the buffer holding the result.
-__device__ float2* wave_fft(float2* buf0, float2* buf1, const FftPlan& plan, const float2* tw,
-                            int sign, int lane) {
-  float2* in = buf0;
-  float2* out = buf1;
-  int Ns = 1;
-  for (int s = 0; s < plan.nstages; ++s) {
-    const int R = plan.radix[s];
-    if (R == 4) stockham_pass<4>(in, out, plan.N, Ns, tw, sign, lane);
-    else if (R == 2) stockham_pass<2>(in, out, plan.N, Ns, tw, sign, lane);
-    else if (R == 3) stockham_pass<3>(in, out, plan.N, Ns, tw, sign, lane);
-    else stockham_pass_generic(in, out, plan.N, Ns, R, tw, sign, lane);
-    __syncthreads();
-    Ns *= R;
-    float2* t = in;
-    in = out;
-    out = t;
-  }
-  return in;
-}
-
 __device__ __forceinline__ size_t waist_index(int c, int ldw, int JHP, int m, int p, int i) {
   return (size_t)c * ldw + ((size_t)((m / kMT) * 2 + p) * JHP + i) * kMT + (m % kMT);
-}
-
-// ---------------------------------------------------------------------------
-// Analysis: grid rows -> folded, weighted waist.
-// ---------------------------------------------------------------------------
-// A block walks `gpb` consecutive row groups of one field; each wavefront
-// fetches its next mirror pair's rows into registers (PF floats per lane and
-// row, PF * 64 >= N) while it transforms the current pair.  PF = 0 reads the
-// rows straight into LDS instead.  LDS: the N twiddles, then per wavefront
-// two N-point buffers plus a third holding the u spectrum while v is
-// transformed (vector jobs).
-template <int PF>
-__global__ void __launch_bounds__(kFftThreads) rfft_fold_kernel(FoldArgs a) {
-  extern __shared__ float2 lds[];
-  const int N = a.fft.N;
-  const int T1 = a.T + 1;
-  const int lane = threadIdx.x & (kWave - 1);
-  const int w = threadIdx.x / kWave;
-  const int chunk = blockIdx.x % a.nchunks;
-  const int item = blockIdx.x / a.nchunks;  // field (scalar) or level (vector)
-  if (item >= a.job.nfields) return;        // block-uniform
-  const int nsrc = a.job.vector ? 2 : 1;
-  const int nbuf = a.job.vector ? 3 : 2;
-  float2* tw = lds;
-  float2* base = lds + N + (size_t)w * nbuf * N;
-  for (int k = threadIdx.x; k < N; k += blockDim.x) tw[k] = a.fft.tw[k];
-  const size_t plane = (size_t)a.nlat * N;
-  const float* gsrc[2] = {a.job.grid0 + (size_t)item * plane,
-                          a.job.vector ? a.job.grid1 + (size_t)item * plane : nullptr};
-  const int g0 = chunk * a.gpb;
-  const int g1 = min(g0 + a.gpb, a.ngroups);
-  const int Tpad = ((T1 + kMT - 1) / kMT) * kMT;
-
-  float rn[2][PF > 0 ? PF : 1], rs[2][PF > 0 ? PF : 1];
-  auto fetch = [&](int g) {
-    if constexpr (PF > 0) {
-      const int i = g * a.rp + w;
-      if (i >= a.JH) return;
-#pragma unroll
-      for (int src = 0; src < 2; ++src) {
-        if (src >= nsrc) break;
-        const float* n_ = gsrc[src] + (size_t)(a.nlat - 1 - i) * N;
-        const float* s_ = gsrc[src] + (size_t)i * N;
-#pragma unroll
-        for (int j = 0; j < PF; ++j) {
-          const int k = lane + kWave * j;
-          rn[src][j] = k < N ? n_[k] : 0.f;
-          rs[src][j] = k < N ? s_[k] : 0.f;
-        }
-      }
-    }
-  };
-  // a scalar field's grid offset is subtracted as its rows enter the FFT
-  // (x - 0 = x exactly, so no offset changes no bit)
-  const float goff = (!a.job.vector && a.job.goff) ? a.job.goff[item] : 0.f;
-  auto put = [&](int g, int src, float2* b) {
-    const int i = g * a.rp + w;
-    if (i >= a.JH) return;
-    if constexpr (PF > 0) {
-#pragma unroll
-      for (int j = 0; j < PF; ++j) {
-        const int k = lane + kWave * j;
-        if (k < N) b[k] = make_float2(rn[src][j] - goff, rs[src][j] - goff);
-      }
-    } else {
-      const float* n_ = gsrc[src] + (size_t)(a.nlat - 1 - i) * N;
-      const float* s_ = gsrc[src] + (size_t)i * N;
-      for (int k = lane; k < N; k += kWave) b[k] = make_float2(n_[k] - goff, s_[k] - goff);
-    }
-  };
-
-  fetch(g0);
-  for (int g = g0; g < g1; ++g) {
-    const int i = g * a.rp + w;
-    const bool live = i < a.JH;
-    const float s = live ? a.job.rowscale[i] : 0.f;
-    put(g, 0, base);
-    float vreg[PF > 0 ? PF : 1], vsreg[PF > 0 ? PF : 1];  // v rows wait in registers
-    if constexpr (PF > 0) {
-#pragma unroll
-      for (int j = 0; j < PF; ++j) {
-        vreg[j] = rn[1][j];
-        vsreg[j] = rs[1][j];
-      }
-    }
-    if (g + 1 < g1) fetch(g + 1);  // next pair's rows load during these FFTs
-    __syncthreads();
-    float2* Zsrc[2] = {nullptr, nullptr};
-    float2* Z = wave_fft(base, base + N, a.fft, tw, -1, lane);
-    Zsrc[0] = Z;
-    if (nsrc == 2) {
-      if (Z != base) {
-        // keep the u spectrum in buffer 0 while v is transformed in 1 and 2
-        for (int k = lane; k < N; k += kWave) base[k] = Z[k];
-        Zsrc[0] = base;
-      }
-      if (live) {
-        if constexpr (PF > 0) {
-#pragma unroll
-          for (int j = 0; j < PF; ++j) {
-            const int k = lane + kWave * j;
-            if (k < N) base[N + k] = make_float2(vreg[j], vsreg[j]);
-          }
-        } else {
-          put(g, 1, base + N);
-        }
-      }
-      __syncthreads();
-      Zsrc[1] = wave_fft(base + N, base + 2 * N, a.fft, tw, -1, lane);
-    }
-    // Fold and write: E = (X_N + X_S) s, O = (X_N - X_S) s for m = 0..T,
-    // zeros for the padding rows and the padding orders of the last m-tile.
-    for (int m = lane; m < Tpad; m += kWave) {
-      float2 e[2], o[2];
-#pragma unroll
-      for (int src = 0; src < 2; ++src) {
-        e[src] = make_float2(0.f, 0.f);
-        o[src] = make_float2(0.f, 0.f);
-        if (src < nsrc && live && m < T1) {
-          const float2* Zs = Zsrc[src];
-          float2 zm = Zs[m];
-          float2 zc = cconj(Zs[(N - m) % N]);
-          float2 xn = make_float2(0.5f * (zm.x + zc.x), 0.5f * (zm.y + zc.y));
-          float2 d = csub(zm, zc);
-          float2 xs = make_float2(0.5f * d.y, -0.5f * d.x);
-          e[src] = make_float2((xn.x + xs.x) * s, (xn.y + xs.y) * s);
-          o[src] = make_float2((xn.x - xs.x) * s, (xn.y - xs.y) * s);
-        }
-      }
-      auto put_w = [&](int c, int p, float v) {
-        a.job.waist0[waist_index(c, a.job.ldw, a.JHP, m, p, i)] = v;
-      };
-      if (!a.job.vector) {
-        const int c = a.job.col0 + 2 * item;
-        put_w(c, 0, e[0].x);
-        put_w(c + 1, 0, e[0].y);
-        put_w(c, 1, o[0].x);
-        put_w(c + 1, 1, o[0].y);
-      } else {
-        // level columns [iV, iU] = [-V.im, V.re, -U.im, U.re] (fold p); the
-        // dP/dphi segment reads [U, -V] = [a3, -a2, -a1, a0] of the same
-        // columns through the GEMM's column map.
-        const int c = a.job.col0 + 4 * item;
-#pragma unroll
-        for (int p = 0; p < 2; ++p) {
-          const float2 U = p == 0 ? e[0] : o[0];
-          const float2 V = p == 0 ? e[1] : o[1];
-          const float va[4] = {-V.y, V.x, -U.y, U.x};
-#pragma unroll
-          for (int cl = 0; cl < 4; ++cl) put_w(c + cl, p, va[cl]);
-        }
-      }
-    }
-    __syncthreads();  // buffers are rewritten by the next group
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Synthesis: folded waist -> grid rows.
-// ---------------------------------------------------------------------------
-// A block walks `gpb` consecutive row groups of one field; each wavefront
-// fetches its next row's E/O values (PF per lane and quantity) while it
-// transforms the current one.  LDS: the N twiddles, then two N-point buffers
-// per wavefront.
-template <int PF>
-__global__ void __launch_bounds__(kFftThreads) irfft_unfold_kernel(UnfoldArgs a) {
-  extern __shared__ float2 lds[];
-  const int N = a.fft.N;
-  const int T1 = a.T + 1;
-  const int lane = threadIdx.x & (kWave - 1);
-  const int w = threadIdx.x / kWave;
-  const int chunk = blockIdx.x % a.nchunks;
-  const int f = blockIdx.x / a.nchunks;
-  if (f >= a.job.nfields) return;  // block-uniform
-  float2* tw = lds;
-  float2* b0 = lds + N + (size_t)w * 2 * N;
-  float2* b1 = b0 + N;
-  for (int k = threadIdx.x; k < N; k += blockDim.x) tw[k] = a.fft.tw[k];
-  const int c = a.job.col0 + a.job.fstride * f;
-  const float* W = a.job.waist;
-  const int g0 = chunk * a.gpb;
-  const int g1 = min(g0 + a.gpb, a.ngroups);
-  // orders per lane, m = lane + 64 j < T+1 <= N/2: half the row depth
-  constexpr int MP = PF > 0 ? PF / 2 : 1;
-  float er[MP], ei[MP], orr[MP], oi[MP];
-  auto fetch = [&](int g) {
-    if constexpr (PF > 0) {
-      const int i = g * a.rp + w;
-      if (i >= a.JH) return;
-#pragma unroll
-      for (int j = 0; j < MP; ++j) {
-        const int m = lane + kWave * j;
-        const bool ok = m < T1;
-        er[j] = ok ? W[waist_index(c, a.job.ldw, a.JHP, m, 0, i)] : 0.f;
-        ei[j] = ok ? W[waist_index(c + 1, a.job.ldw, a.JHP, m, 0, i)] : 0.f;
-        orr[j] = ok ? W[waist_index(c, a.job.ldw, a.JHP, m, 1, i)] : 0.f;
-        oi[j] = ok ? W[waist_index(c + 1, a.job.ldw, a.JHP, m, 1, i)] : 0.f;
-      }
-    }
-  };
-  // spectrum value Z at order m from E, O
-  auto zval = [&](float2 E, float2 O, float s, int m, bool lower) {
-    float2 A = make_float2((E.x + O.x) * s, (E.y + O.y) * s);
-    float2 B = make_float2((E.x - O.x) * s, (E.y - O.y) * s);
-    if (a.job.imul) {
-      const float k = a.job.imul == 2 ? (float)m : 1.f;  // i m or i
-      A = make_float2(-k * A.y, k * A.x);
-      B = make_float2(-k * B.y, k * B.x);
-    }
-    if (m == 0) {
-      A.y = 0.f;
-      B.y = 0.f;
-    }
-    return lower ? make_float2(A.x - B.y, A.y + B.x)     // A + iB
-                 : make_float2(A.x + B.y, -A.y + B.x);   // conj(A) + i conj(B)
-  };
-
-  fetch(g0);
-  for (int g = g0; g < g1; ++g) {
-    const int i = g * a.rp + w;
-    const bool live = i < a.JH;
-    if (live) {
-      const float s = a.job.rowscale[i];
-      // Z[k] = A + iB at k = m <= N/2, conj(A) + i conj(B) at k = N - m; zero above T
-      for (int k = lane; k < N; k += kWave) b0[k] = make_float2(0.f, 0.f);
-      if constexpr (PF > 0) {
-#pragma unroll
-        for (int j = 0; j < MP; ++j) {
-          const int m = lane + kWave * j;
-          if (m < T1) {
-            const float2 E = make_float2(er[j], ei[j]), O = make_float2(orr[j], oi[j]);
-            b0[m] = zval(E, O, s, m, true);
-            if (m > 0) b0[N - m] = zval(E, O, s, m, false);
-          }
-        }
-      } else {
-        for (int m = lane; m < T1; m += kWave) {
-          const float2 E = make_float2(W[waist_index(c, a.job.ldw, a.JHP, m, 0, i)],
-                                       W[waist_index(c + 1, a.job.ldw, a.JHP, m, 0, i)]);
-          const float2 O = make_float2(W[waist_index(c, a.job.ldw, a.JHP, m, 1, i)],
-                                       W[waist_index(c + 1, a.job.ldw, a.JHP, m, 1, i)]);
-          b0[m] = zval(E, O, s, m, true);
-          if (m > 0) b0[N - m] = zval(E, O, s, m, false);
-        }
-      }
-    }
-    if (g + 1 < g1) fetch(g + 1);  // next row's E/O load during this FFT
-    __syncthreads();
-    float2* x = wave_fft(b0, b1, a.fft, tw, +1, lane);
-    if (live) {
-      const size_t plane = (size_t)a.nlat * N;
-      float* rn = a.job.grid + (size_t)f * plane + (size_t)(a.nlat - 1 - i) * N;
-      float* rs = a.job.grid + (size_t)f * plane + (size_t)i * N;
-      for (int k = lane; k < N; k += kWave) {
-        float2 v = x[k];
-        rn[k] = a.job.post_exp ? expf(v.x) : v.x;
-        rs[k] = a.job.post_exp ? expf(v.y) : v.y;
-      }
-    }
-    __syncthreads();  // buffers are rewritten by the next group
-  }
 }
 
 // ---------------------------------------------------------------------------
@@ -470,6 +114,9 @@ constexpr Ring48<R> make_ring48() {
 constexpr Ring48<float> kRing48 = make_ring48<float>();
 constexpr Ring48<double> kRing48d = make_ring48<double>();
 
+// Lambdas of the unrolled loops are inlined whatever their size: their
+// captured arrays must stay in registers.
+#define SHT_INLINE __attribute__((always_inline))
 template <class Fn, int... I>
 __device__ __forceinline__ void static_for_impl(Fn&& fn, std::integer_sequence<int, I...>) {
   (fn(std::integral_constant<int, I>{}), ...);
@@ -480,7 +127,11 @@ __device__ __forceinline__ void static_for(Fn&& fn) {
   static_for_impl(fn, std::make_integer_sequence<int, N>{});
 }
 
-// x * e^(S 2 pi i E / R), R | 48; C is float2 or double2
+// cos and sin of 2 pi e / R in FP64 (rings that do not divide 48: fp32 FFTs)
+constexpr double ring_cos(int e, int R) { return taylor_cos(kTwoPi * (e % R) / R); }
+constexpr double ring_sin(int e, int R) { return taylor_sin(kTwoPi * (e % R) / R); }
+
+// x * e^(S 2 pi i E / R); C is float2, or double2 where R | 48
 template <int E, int R, int S, class C>
 __device__ __forceinline__ C rot(C x) {
   constexpr int e = ((E % R) + R) % R;
@@ -492,6 +143,9 @@ __device__ __forceinline__ C rot(C x) {
     return S > 0 ? cmk(-x.y, x.x) : cmk(x.y, -x.x);
   } else if constexpr (4 * e == 3 * R) {  // -S i
     return S > 0 ? cmk(x.y, -x.x) : cmk(-x.y, x.x);
+  } else if constexpr (48 % R != 0) {
+    constexpr float c = (float)ring_cos(e, R), sn = S * (float)ring_sin(e, R);
+    return make_float2(x.x * c - x.y * sn, x.x * sn + x.y * c);
   } else if constexpr (std::is_same<C, float2>::value) {
     constexpr int j = e * (48 / R);
     constexpr float c = kRing48.c[j], sn = S * kRing48.s[j];
@@ -533,28 +187,53 @@ __device__ __forceinline__ void dft(C (&v)[R]) {
     v[2] = csub(a0, a2);
     v[1] = cadd(a1, a3);
     v[3] = csub(a1, a3);
+  } else if constexpr (R == 5 || R == 7 || R == 11 || R == 13) {
+    // x_r +- x_{R-r}: outputs q and R-q share their sums of cosines and sines
+    constexpr int H = (R - 1) / 2;
+    const C x0 = v[0];
+    C p[H], d[H], sum = x0;
+    static_for<H>([&](auto h_) SHT_INLINE {
+      constexpr int h = decltype(h_)::value;
+      p[h] = cadd(v[h + 1], v[R - 1 - h]);
+      d[h] = csub(v[h + 1], v[R - 1 - h]);
+      sum = cadd(sum, p[h]);
+    });
+    v[0] = sum;
+    static_for<H>([&](auto q_) SHT_INLINE {
+      constexpr int q = decltype(q_)::value + 1;
+      C c = x0, t = cmk(0.f, 0.f);
+      static_for<H>([&](auto h_) SHT_INLINE {
+        constexpr int h = decltype(h_)::value;
+        constexpr float co = (float)ring_cos(q * (h + 1), R);
+        constexpr float si = S * (float)ring_sin(q * (h + 1), R);
+        c = cmk(c.x + co * p[h].x, c.y + co * p[h].y);
+        t = cmk(t.x + si * d[h].x, t.y + si * d[h].y);
+      });
+      v[q] = cmk(c.x - t.y, c.y + t.x);
+      v[R - q] = cmk(c.x + t.y, c.y - t.x);
+    });
   } else {
     // n = Q n1 + n2, k = k1 + P k2:
     // X[k1 + P k2] = sum_n2 w_Q^(n2 k2) w_R^(n2 k1) sum_n1 x[Q n1 + n2] w_P^(n1 k1)
     constexpr int P = (R % 4 == 0) ? 4 : ((R % 3 == 0) ? 3 : 2);
     constexpr int Q = R / P;
     C y[R];
-    static_for<Q>([&](auto n2_) {
+    static_for<Q>([&](auto n2_) SHT_INLINE {
       constexpr int n2 = decltype(n2_)::value;
       C t[P];
-      static_for<P>([&](auto n1_) { t[n1_] = v[Q * decltype(n1_)::value + n2]; });
+      static_for<P>([&](auto n1_) SHT_INLINE { t[n1_] = v[Q * decltype(n1_)::value + n2]; });
       dft<P, S>(t);
-      static_for<P>([&](auto k1_) {
+      static_for<P>([&](auto k1_) SHT_INLINE {
         constexpr int k1 = decltype(k1_)::value;
         y[n2 * P + k1] = rot<n2 * k1, R, S>(t[k1]);
       });
     });
-    static_for<P>([&](auto k1_) {
+    static_for<P>([&](auto k1_) SHT_INLINE {
       constexpr int k1 = decltype(k1_)::value;
       C t[Q];
-      static_for<Q>([&](auto n2_) { t[n2_] = y[decltype(n2_)::value * P + k1]; });
+      static_for<Q>([&](auto n2_) SHT_INLINE { t[n2_] = y[decltype(n2_)::value * P + k1]; });
       dft<Q, S>(t);
-      static_for<Q>([&](auto k2_) { v[k1 + P * decltype(k2_)::value] = t[k2_]; });
+      static_for<Q>([&](auto k2_) SHT_INLINE { v[k1 + P * decltype(k2_)::value] = t[k2_]; });
     });
   }
 }
@@ -599,10 +278,10 @@ __device__ __forceinline__ void fill_wave_twiddles(C* tw, const C* table) {
 template <int L, int F, int S, class C>
 __device__ __forceinline__ void wave_fft64(C (&v)[F][L], C* buf, const C* tw, int lane) {
   constexpr int SP = wave_span<L>();
-  static_for<F>([&](auto f_) {
+  static_for<F>([&](auto f_) SHT_INLINE {
     constexpr int f = decltype(f_)::value;
     dft<L, S>(v[f]);
-    static_for<L>([&](auto k1_) {
+    static_for<L>([&](auto k1_) SHT_INLINE {
       constexpr int k1 = decltype(k1_)::value;
       C x = v[f][k1];
       if constexpr (k1 > 0) x = cmul(x, twiddle(tw, 64 * k1 + lane, S));
@@ -613,15 +292,15 @@ __device__ __forceinline__ void wave_fft64(C (&v)[F][L], C* buf, const C* tw, in
   constexpr int U = F * L * 8, RND = (U + 63) / 64;
   C w[RND][8];
   // B: units (f, k1, b)
-  static_for<RND>([&](auto r_) {
+  static_for<RND>([&](auto r_) SHT_INLINE {
     constexpr int r = decltype(r_)::value;
     const int u = lane + 64 * r;
     if (u < U) {
       const int f = u / (8 * L), k1 = (u >> 3) % L, b = u & 7;
       const C* row = buf + f * SP + k1 * kRowSpan + b;
-      static_for<8>([&](auto a_) { w[r][a_] = row[8 * decltype(a_)::value]; });
+      static_for<8>([&](auto a_) SHT_INLINE { w[r][a_] = row[8 * decltype(a_)::value]; });
       dft<8, S>(w[r]);
-      static_for<8>([&](auto c_) {
+      static_for<8>([&](auto c_) SHT_INLINE {
         constexpr int c = decltype(c_)::value;
         if constexpr (c > 0) w[r][c] = cmul(w[r][c], twiddle(tw, 64 * L + 8 * c + b, S));
       });
@@ -630,13 +309,13 @@ __device__ __forceinline__ void wave_fft64(C (&v)[F][L], C* buf, const C* tw, in
   wave_sync();
   // S2[k1][c][b ^ c]: the B writes (lanes over b) and the C reads (lanes
   // over c) both hit distinct banks (measured)
-  static_for<RND>([&](auto r_) {
+  static_for<RND>([&](auto r_) SHT_INLINE {
     constexpr int r = decltype(r_)::value;
     const int u = lane + 64 * r;
     if (u < U) {
       const int f = u / (8 * L), k1 = (u >> 3) % L, b = u & 7;
       C* row = buf + f * SP + k1 * kRowSpan;
-      static_for<8>([&](auto c_) {
+      static_for<8>([&](auto c_) SHT_INLINE {
         constexpr int c = decltype(c_)::value;
         row[8 * c + (b ^ c)] = w[r][c];
       });
@@ -644,24 +323,24 @@ __device__ __forceinline__ void wave_fft64(C (&v)[F][L], C* buf, const C* tw, in
   });
   wave_sync();
   // C: units (f, k1, c)
-  static_for<RND>([&](auto r_) {
+  static_for<RND>([&](auto r_) SHT_INLINE {
     constexpr int r = decltype(r_)::value;
     const int u = lane + 64 * r;
     if (u < U) {
       const int f = u / (8 * L), k1 = (u >> 3) % L, c = u & 7;
       const C* row = buf + f * SP + k1 * kRowSpan + 8 * c;
-      static_for<8>([&](auto b_) { w[r][b_] = row[decltype(b_)::value ^ c]; });
+      static_for<8>([&](auto b_) SHT_INLINE { w[r][b_] = row[decltype(b_)::value ^ c]; });
       dft<8, S>(w[r]);
     }
   });
   wave_sync();
-  static_for<RND>([&](auto r_) {
+  static_for<RND>([&](auto r_) SHT_INLINE {
     constexpr int r = decltype(r_)::value;
     const int u = lane + 64 * r;
     if (u < U) {
       const int f = u / (8 * L), k1 = (u >> 3) % L, c = u & 7;
       C* out = buf + f * SP + k1 + L * c;
-      static_for<8>([&](auto d_) { out[8 * L * decltype(d_)::value] = w[r][d_]; });
+      static_for<8>([&](auto d_) SHT_INLINE { out[8 * L * decltype(d_)::value] = w[r][d_]; });
     }
   });
   wave_sync();
@@ -716,14 +395,14 @@ __global__ void __launch_bounds__(64 * kWaveBlock, (fold_waves_per_simd<L, F, kW
     const int item = grp * kWaveBlock + w;
     const int fld = item / a.JHP, i = item % a.JHP;
     if (i >= a.JH) return;
-    static_for<F>([&](auto f_) {
+    static_for<F>([&](auto f_) SHT_INLINE {
       constexpr int f = decltype(f_)::value;
       const float* gp = (f == 0 ? a.job.grid0 : a.job.grid1) + (size_t)fld * plane;
       const float* rn = gp + (size_t)(a.nlat - 1 - i) * N;
       const float* rs = gp + (size_t)i * N;
       // a scalar field's grid offset (x - 0 = x exactly)
       const float off = (F == 1 && a.job.goff) ? a.job.goff[fld] : 0.f;
-      static_for<L>([&](auto n1_) {
+      static_for<L>([&](auto n1_) SHT_INLINE {
         constexpr int n1 = decltype(n1_)::value;
         v[f][n1] = make_float2(rn[64 * n1 + lane] - off, rs[64 * n1 + lane] - off);
       });
@@ -924,13 +603,13 @@ __global__ void __launch_bounds__(64 * kWaveBlock,
       }
       wave_sync();
       float2 v[1][L];
-      static_for<L>([&](auto n1_) { v[0][n1_] = buf[64 * decltype(n1_)::value + lane]; });
+      static_for<L>([&](auto n1_) SHT_INLINE { v[0][n1_] = buf[64 * decltype(n1_)::value + lane]; });
       wave_sync();
       wave_fft64<L, 1, +1>(v, buf, tw, lane);
       float* rn = a.job.grid + (size_t)fld * plane + (size_t)(a.nlat - 1 - i) * N;
       float* rs = a.job.grid + (size_t)fld * plane + (size_t)i * N;
       const bool post_exp = a.job.post_exp != 0;
-      static_for<L>([&](auto q_) {
+      static_for<L>([&](auto q_) SHT_INLINE {
         const int k = lane + 64 * decltype(q_)::value;
         const float2 x = buf[k];
         rn[k] = post_exp ? expf(x.x) : x.x;
@@ -980,7 +659,7 @@ __global__ void __launch_bounds__(64 * kWaveBlock) rfft_fold_wave64_kernel(FoldA
     const float* gp = a.job.grid0 + (size_t)fld * plane;
     const float* rn = gp + (size_t)(a.nlat - 1 - i) * N;
     const float* rs = gp + (size_t)i * N;
-    static_for<L>([&](auto n1_) {
+    static_for<L>([&](auto n1_) SHT_INLINE {
       constexpr int n1 = decltype(n1_)::value;
       pre[n1] = make_float2(rn[64 * n1 + lane], rs[64 * n1 + lane]);
     });
@@ -994,7 +673,7 @@ __global__ void __launch_bounds__(64 * kWaveBlock) rfft_fold_wave64_kernel(FoldA
     const bool live = i < a.JH;
     if (live) {
       double2 v[1][L];
-      static_for<L>([&](auto n1_) {
+      static_for<L>([&](auto n1_) SHT_INLINE {
         constexpr int n1 = decltype(n1_)::value;
         v[0][n1] = make_double2((double)pre[n1].x, (double)pre[n1].y);
       });
@@ -1155,12 +834,12 @@ __global__ void __launch_bounds__(64 * kWaveBlock) irfft_unfold_wave64_kernel(Un
       }
       wave_sync();
       double2 v[1][L];
-      static_for<L>([&](auto n1_) { v[0][n1_] = buf[64 * decltype(n1_)::value + lane]; });
+      static_for<L>([&](auto n1_) SHT_INLINE { v[0][n1_] = buf[64 * decltype(n1_)::value + lane]; });
       wave_sync();
       wave_fft64<L, 1, +1>(v, buf, tw, lane);
       float* rn = a.job.grid + (size_t)fld * plane + (size_t)(a.nlat - 1 - i) * N;
       float* rs = a.job.grid + (size_t)fld * plane + (size_t)i * N;
-      static_for<L>([&](auto q_) {
+      static_for<L>([&](auto q_) SHT_INLINE {
         const int k = lane + 64 * decltype(q_)::value;
         const double2 x = buf[k];
         rn[k] = (float)x.x;
@@ -1168,6 +847,361 @@ __global__ void __launch_bounds__(64 * kWaveBlock) irfft_unfold_wave64_kernel(Un
       });
     }
     __syncthreads();  // every span is consumed before the next group's runs land
+  }
+}
+
+// ---------------------------------------------------------------------------
+// FFTs of any other even N: Stockham passes of one wavefront in LDS
+// ---------------------------------------------------------------------------
+// A wavefront transforms a mirror row pair in two LDS buffers, one pass per
+// factor of N chosen by the host, with no block barrier.  Bound: LDS latency
+// and bandwidth of the passes, a read and a write of the row each, so scalar
+// fields take few, large radices (2..16 with a butterfly in registers, a
+// larger prime by shared cosine and sine sums).  The vector operators' rows
+// take radices 4, 2, 3 and direct sums of the other primes: vorticity and
+// divergence multiply a wind's last-bit rounding by up to the truncation, and
+// that sequence of roundings is the one their results have always had.
+// Points sit at padded
+// positions i + i/16, which spreads the stride-R stores of the first pass over
+// the banks.  Quotients by Ns come from an fp32 reciprocal:
+// floor((j + 1/2) / Ns) is exact for j < 2^20 (the product is within
+// N/(R Ns) 2^-22 of the quotient, the nearest integer at least 1/(2 Ns) away).
+// Rows per block as in the wave-resident kernels (8 where they fit), so the
+// waist moves in whole lines; launch positions are dealt to the XCDs in runs
+// of neighbouring groups, so that where fewer rows fit the parts of a line
+// meet in one L2.
+// Measured (19 fields of gradients, T106 on 161 x 322, two launches): 402 us
+// in the former passes (a block barrier each, a modulo per term), 19.7 us here.
+
+// float2 per buffer, even: the staged runs are 16-byte vectors
+__host__ __device__ inline int gen_span(int N) { return (N + N / 16 + 9) & ~1; }
+__device__ __forceinline__ int gp(int i) { return i + (i >> 4); }
+
+template <int R, int S, bool FIRST>
+__device__ __forceinline__ void gen_pass(const float2* in, float2* out, int N, int Ns,
+                                         const float2* tw, int lane) {
+  // opaque, so that each pass's addresses are formed in it rather than held
+  // in registers across the kernel's group loop (256 VGPRs and spills)
+  asm volatile("" : "+v"(lane), "+s"(N));
+  const int nb = N / R;
+  const int tstep = FIRST ? 0 : nb / Ns;
+  const float inv_ns = 1.0f / (float)Ns;
+  for (int j = lane; j < nb; j += kWave) {
+    int k = 0, q = j;
+    if constexpr (!FIRST) {
+      q = (int)(((float)j + 0.5f) * inv_ns);
+      k = j - q * Ns;
+    }
+    const int t = k * tstep;
+    float2 v[R];
+    static_for<R>([&](auto r_) SHT_INLINE {
+      constexpr int r = decltype(r_)::value;
+      v[r] = in[gp(j + r * nb)];
+      if constexpr (!FIRST && r > 0) v[r] = cmul(v[r], twiddle(tw, r * t, S));
+    });
+    dft<R, S>(v);
+    const int d = q * Ns * R + k;
+    static_for<R>([&](auto r_) SHT_INLINE {
+      constexpr int r = decltype(r_)::value;
+      out[gp(d + r * Ns)] = v[r];
+    });
+  }
+}
+
+// First pass (Ns = 1) of a prime radix R > 13: x_r and x_{R-r} are replaced
+// by their sum and difference in place, then outputs q and R-q come from the
+// same h = (R-1)/2 cosine and sine sums.  A lane takes one j and up to four
+// q, so each sum and difference read feeds eight accumulators.
+template <int S>
+__device__ __forceinline__ void gen_prime_first(float2* in, float2* out, int N, int R,
+                                                const float2* tw, int lane) {
+  asm volatile("" : "+v"(lane), "+s"(N));
+  const int nb = N / R, h = (R - 1) / 2;
+  const float inv_nb = 1.0f / (float)nb;
+  for (int u = lane; u < nb * h; u += kWave) {
+    const int r = (int)(((float)u + 0.5f) * inv_nb), j = u - r * nb;
+    const int ia = gp(j + (r + 1) * nb), ib = gp(j + (R - 1 - r) * nb);
+    const float2 a = in[ia], b = in[ib];
+    in[ia] = cadd(a, b);
+    in[ib] = csub(a, b);
+  }
+  wave_sync();
+  const int QG = (h + 4) / 4;  // q = 0..h in four groups
+  for (int u = lane; u < nb * QG; u += kWave) {
+    const int qg = (int)(((float)u + 0.5f) * inv_nb), j = u - qg * nb;
+    const float2 x0 = in[gp(j)];
+    float2 c[4], t[4];
+    int inc[4], idx[4];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      c[g] = x0;
+      t[g] = make_float2(0.f, 0.f);
+      idx[g] = 0;
+      inc[g] = min(qg + g * QG, h) * nb;  // index step of q in the w_N table
+    }
+    for (int r = 1; r <= h; ++r) {
+      const float2 a = in[gp(j + r * nb)], b = in[gp(j + (R - r) * nb)];
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        idx[g] += inc[g];
+        idx[g] -= idx[g] >= N ? N : 0;
+        const float2 w = tw[idx[g]];  // cos, -sin
+        c[g] = make_float2(c[g].x + w.x * a.x, c[g].y + w.x * a.y);
+        t[g] = make_float2(t[g].x + w.y * b.x, t[g].y + w.y * b.y);
+      }
+    }
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int q = qg + g * QG;
+      if (q > h) continue;
+      // sum x_r e^{S i theta} = c + S i sum b sin = c - S i t
+      const float2 p = make_float2(c[g].x + t[g].y, c[g].y - t[g].x);
+      const float2 m = make_float2(c[g].x - t[g].y, c[g].y + t[g].x);
+      out[gp(j * R + q)] = S > 0 ? p : m;
+      if (q > 0) out[gp(j * R + R - q)] = S > 0 ? m : p;
+    }
+  }
+}
+
+// A pass of any radix R by direct sums in the order of the inputs: twiddled in
+// place (passes after the first), then up to four outputs q of one j per
+// lane, so each input read feeds four accumulators.
+template <int S>
+__device__ __forceinline__ void gen_direct_pass(float2* in, float2* out, int N, int Ns, int R,
+                                                const float2* tw, int lane) {
+  asm volatile("" : "+v"(lane), "+s"(N));
+  const int nb = N / R, tstep = nb / Ns;
+  const float inv_nb = 1.0f / (float)nb, inv_ns = 1.0f / (float)Ns;
+  if (Ns > 1) {
+    for (int u = lane + nb; u < N; u += kWave) {
+      const int r = (int)(((float)u + 0.5f) * inv_nb), j = u - r * nb;
+      const int k = j - (int)(((float)j + 0.5f) * inv_ns) * Ns;
+      in[gp(u)] = cmul(in[gp(u)], twiddle(tw, r * k * tstep, S));
+    }
+    wave_sync();
+  }
+  const int QG = (R + 3) / 4;
+  for (int u = lane; u < nb * QG; u += kWave) {
+    const int qg = (int)(((float)u + 0.5f) * inv_nb), j = u - qg * nb;
+    const int g = (int)(((float)j + 0.5f) * inv_ns), d = g * Ns * R + (j - g * Ns);
+    float2 acc[4];
+    int inc[4], idx[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      acc[e] = in[gp(j)];
+      idx[e] = 0;
+      inc[e] = min(qg + e * QG, R - 1) * nb;  // step of q in the w_N table
+    }
+    for (int r = 1; r < R; ++r) {
+      const float2 x = in[gp(j + r * nb)];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        idx[e] += inc[e];
+        idx[e] -= idx[e] >= N ? N : 0;
+        acc[e] = cadd(acc[e], cmul(x, twiddle(tw, idx[e], S)));
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (qg + e * QG < R) out[gp(d + (qg + e * QG) * Ns)] = acc[e];
+  }
+}
+
+// The transform of the N points in b0 (padded positions) in the given
+// passes; returns the buffer that holds the result.
+template <int S>
+__device__ __forceinline__ float2* gen_fft(float2* b0, float2* b1, int N, const FftPasses& passes,
+                                           const float2* tw, int lane) {
+  float2 *in = b0, *out = b1;
+  int Ns = 1;
+  for (int s = 0; s < passes.n; ++s) {
+    const int R = passes.radix[s];
+#define SHT_GEN_PASS(RR)                                                     \
+  case RR:                                                                   \
+    if (s == 0) gen_pass<RR, S, true>(in, out, N, 1, tw, lane);              \
+    else gen_pass<RR, S, false>(in, out, N, Ns, tw, lane);                   \
+    break;
+    switch (passes.direct && R > 4 ? 0 : R) {
+      SHT_GEN_PASS(2) SHT_GEN_PASS(3) SHT_GEN_PASS(4) SHT_GEN_PASS(5) SHT_GEN_PASS(6)
+      SHT_GEN_PASS(7) SHT_GEN_PASS(8) SHT_GEN_PASS(9) SHT_GEN_PASS(10) SHT_GEN_PASS(11)
+      SHT_GEN_PASS(12) SHT_GEN_PASS(13) SHT_GEN_PASS(14) SHT_GEN_PASS(15) SHT_GEN_PASS(16)
+      default:
+        if (s == 0 && !passes.direct) gen_prime_first<S>(in, out, N, R, tw, lane);
+        else gen_direct_pass<S>(in, out, N, Ns, R, tw, lane);
+    }
+#undef SHT_GEN_PASS
+    wave_sync();
+    Ns *= R;
+    float2* t = in;
+    in = out;
+    out = t;
+  }
+  return in;
+}
+
+// Logical position of this block, neighbours on one XCD (grid a multiple of
+// 8: launch position b runs on XCD b % 8).
+__device__ __forceinline__ int xcd_position() {
+  const int G = gridDim.x;
+  return G % 8 ? (int)blockIdx.x : (int)(blockIdx.x % 8) * (G / 8) + (int)(blockIdx.x / 8);
+}
+
+constexpr int kGenBatch = 8;  // row loads in flight per lane
+
+// One row (or mirror row pair) into an LDS buffer at padded positions:
+// get(k), k < N, in batches of kGenBatch loads per lane.
+template <class Get>
+__device__ __forceinline__ void gen_load_row(float2* buf, int N, int lane, Get&& get) {
+  for (int k0 = lane; k0 < N; k0 += kWave * kGenBatch) {
+    float2 x[kGenBatch];
+#pragma unroll
+    for (int u = 0; u < kGenBatch; ++u) x[u] = get(min(k0 + kWave * u, N - 1));
+#pragma unroll
+    for (int u = 0; u < kGenBatch; ++u)
+      if (k0 + kWave * u < N) buf[gp(k0 + kWave * u)] = x[u];
+  }
+}
+
+// Analysis of one field per (field, folded row); with job.imul the columns of
+// i X (the vector operators' [iV, iU] arrangement, one launch per component).
+__global__ void __launch_bounds__(512) rfft_fold_rows_kernel(FoldArgs a) {
+  extern __shared__ float2 lds[];
+  typedef __attribute__((ext_vector_type(4))) float f4;
+  const int N = a.fft.N, T1 = a.T + 1;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int rb = blockDim.x >> 6, lrb = 31 - __clz(rb);  // rows per block, a power of two
+  const int span = gen_span(N), WS = 2 * span + kSpanPad;
+  float2* tw = lds;
+  float2* rows = lds + N;
+  float2* b0 = rows + (size_t)w * WS;
+  // after an odd number of passes the spectrum is in the second buffer; the
+  // folded values are staged in the other one
+  const FftPasses& passes = a.job.imul ? a.fft.vector : a.fft.scalar;
+  const int z_at = passes.n & 1 ? span : 0, stage_at = span - z_at;
+  for (int k = threadIdx.x; k < N; k += blockDim.x) tw[k] = a.fft.tw[k];
+  const int rgroups = a.JHP >> lrb, ngroups = a.job.nfields * rgroups;
+  const int MT = (T1 + kMT - 1) / kMT, MO = MT * kMT;
+  const size_t plane = (size_t)a.nlat * N;
+  const float inv_mt = 1.0f / (float)MT;
+  __syncthreads();
+  for (int g = xcd_position(); g < ngroups; g += gridDim.x) {
+    const int fld = g / rgroups, i0 = (g % rgroups) << lrb, i = i0 + w;
+    const bool live = i < a.JH;
+    if (live) {
+      const float* rn = a.job.grid0 + (size_t)fld * plane + (size_t)(a.nlat - 1 - i) * N;
+      const float* rs = a.job.grid0 + (size_t)fld * plane + (size_t)i * N;
+      const float off = a.job.goff ? a.job.goff[fld] : 0.f;  // x - 0 = x exactly
+      gen_load_row(b0, N, lane, [&](int k) { return make_float2(rn[k] - off, rs[k] - off); });
+      wave_sync();
+      gen_fft<-1>(b0, b0 + span, N, passes, tw, lane);
+    }
+    // E = (X_N + X_S) s, O = (X_N - X_S) s to stage[2 column + parity][m],
+    // zeros for the padding rows and the padding orders of the last m-tile
+    const float s = live ? a.job.rowscale[i] : 0.f;
+    const float2* Z = b0 + z_at;
+    float* stage = reinterpret_cast<float*>(b0 + stage_at);
+    for (int m = lane; m < MO; m += kWave) {
+      float2 e = make_float2(0.f, 0.f), o = e;
+      if (live && m < T1) {
+        const float2 zm = Z[gp(m)];
+        const float2 zc = cconj(Z[gp(m ? N - m : 0)]);
+        const float2 xn = make_float2(0.5f * (zm.x + zc.x), 0.5f * (zm.y + zc.y));
+        const float2 d = csub(zm, zc);
+        const float2 xs = make_float2(0.5f * d.y, -0.5f * d.x);
+        e = make_float2((xn.x + xs.x) * s, (xn.y + xs.y) * s);
+        o = make_float2((xn.x - xs.x) * s, (xn.y - xs.y) * s);
+      }
+      stage[m] = a.job.imul ? -e.y : e.x;
+      stage[MO + m] = a.job.imul ? -o.y : o.x;
+      stage[2 * MO + m] = a.job.imul ? e.x : e.y;
+      stage[3 * MO + m] = a.job.imul ? o.x : o.y;
+    }
+    __syncthreads();
+    // run (e, mt) = rows i0 .. i0+rb-1 x orders 4 mt .. 4 mt + 3, one contiguous
+    // piece, as in rfft_fold_wave_kernel (the quotient is exact: e <= 3)
+    for (int u = threadIdx.x; u < (4 * MT) << lrb; u += blockDim.x) {
+      const int ww = u & (rb - 1), rn = u >> lrb;
+      const int e = (int)(((float)rn + 0.5f) * inv_mt), mt = rn - e * MT;
+      const int c = a.job.col0 + a.job.fstride * fld + (e >> 1), p = e & 1;
+      *reinterpret_cast<f4*>(a.job.waist0 + waist_index(c, a.job.ldw, a.JHP, mt * kMT, p, i0 + ww)) =
+          *reinterpret_cast<const f4*>(
+              reinterpret_cast<const float*>(rows + (size_t)ww * WS + stage_at) +
+              ((size_t)e * MT + mt) * 4);
+    }
+    __syncthreads();  // the buffers are rewritten by the next group
+  }
+}
+
+// Synthesis of one field per (field, folded row): the waist's runs are staged
+// in the second buffer, the spectrum is built in the first.
+__global__ void __launch_bounds__(512) irfft_unfold_rows_kernel(UnfoldArgs a) {
+  extern __shared__ float2 lds[];
+  typedef __attribute__((ext_vector_type(4))) float f4;
+  const int N = a.fft.N, T1 = a.T + 1;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int rb = blockDim.x >> 6, lrb = 31 - __clz(rb);
+  const int span = gen_span(N), WS = 2 * span + kSpanPad;
+  float2* tw = lds;
+  float2* rows = lds + N;
+  float2* b0 = rows + (size_t)w * WS;
+  for (int k = threadIdx.x; k < N; k += blockDim.x) tw[k] = a.fft.tw[k];
+  const int rgroups = (a.JH + rb - 1) >> lrb, ngroups = a.job.nfields * rgroups;
+  const int MT = (T1 + kMT - 1) / kMT, MO = MT * kMT;
+  const size_t plane = (size_t)a.nlat * N;
+  const float inv_mt = 1.0f / (float)MT;
+  for (int g = xcd_position(); g < ngroups; g += gridDim.x) {
+    const int fld = g / rgroups, i0 = (g % rgroups) << lrb, i = i0 + w;
+    const float* W = a.job.waist + (size_t)(a.job.col0 + a.job.fstride * fld) * a.job.ldw;
+    const int runs = (4 * MT) << lrb;
+    for (int u0 = threadIdx.x; u0 < runs; u0 += 4 * blockDim.x) {
+      f4 x[4];
+      int at[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {  // past the end: the last run again
+        const int u = min(u0 + q * (int)blockDim.x, runs - 1);
+        const int ww = u & (rb - 1), rn = u >> lrb;
+        const int e = (int)(((float)rn + 0.5f) * inv_mt), mt = rn - e * MT;
+        x[q] = *reinterpret_cast<const f4*>(
+            W + waist_index(e >> 1, a.job.ldw, a.JHP, mt * kMT, e & 1, i0 + ww));
+        at[q] = 2 * (ww * WS + span) + 4 * rn;
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) *reinterpret_cast<f4*>(reinterpret_cast<float*>(rows) + at[q]) = x[q];
+    }
+    __syncthreads();  // the runs (and, the first time, the twiddles) are in LDS
+    if (i < a.JH) {
+      const float s = a.job.rowscale[i];
+      const float* stage = reinterpret_cast<const float*>(b0 + span);
+      // Z[k] = A + iB at k = m, conj(A) + i conj(B) at k = N - m; zero above T
+      for (int k = T1 + lane; k < N - a.T; k += kWave) b0[gp(k)] = make_float2(0.f, 0.f);
+      for (int m = lane; m < T1; m += kWave) {
+        const float er = stage[m], orr = stage[MO + m], ei = stage[2 * MO + m], oi = stage[3 * MO + m];
+        float2 A = make_float2((er + orr) * s, (ei + oi) * s);
+        float2 B = make_float2((er - orr) * s, (ei - oi) * s);
+        if (a.job.imul) {
+          const float k = a.job.imul == 2 ? (float)m : 1.f;  // i m or i
+          A = make_float2(-k * A.y, k * A.x);
+          B = make_float2(-k * B.y, k * B.x);
+        }
+        if (m == 0) {
+          A.y = 0.f;
+          B.y = 0.f;
+        }
+        b0[gp(m)] = make_float2(A.x - B.y, A.y + B.x);
+        if (m > 0) b0[gp(N - m)] = make_float2(A.x + B.y, -A.y + B.x);
+      }
+      wave_sync();
+      const float2* x = gen_fft<+1>(b0, b0 + span, N, a.job.wind ? a.fft.vector : a.fft.scalar, tw, lane);
+      float* rn = a.job.grid + (size_t)fld * plane + (size_t)(a.nlat - 1 - i) * N;
+      float* rs = a.job.grid + (size_t)fld * plane + (size_t)i * N;
+      const bool post_exp = a.job.post_exp != 0;
+      for (int k = lane; k < N; k += kWave) {
+        const float2 v = x[gp(k)];
+        rn[k] = post_exp ? expf(v.x) : v.x;
+        rs[k] = post_exp ? expf(v.y) : v.y;
+      }
+    }
+    __syncthreads();  // every row is consumed before the next group's runs land
   }
 }
 
@@ -1239,13 +1273,16 @@ constexpr size_t kWaveLdsMax = 160 * 1024;  // LDS of one gfx950 workgroup
 // rows per block: 8 when their LDS fits, else 4
 int wave_rb(size_t lds8) { return lds8 <= kWaveLdsMax ? 8 : 4; }
 
-size_t fold_lds_bytes(int N, int T, int vector, int rp) {
-  (void)T;
-  return (size_t)(1 + rp * (vector ? 3 : 2)) * N * sizeof(float2);
+// LDS of the row kernels (any other N): twiddles and two buffers per row.
+size_t gen_lds_bytes(int N, int rb) {
+  return ((size_t)N + (size_t)rb * (2 * gen_span(N) + kSpanPad)) * sizeof(float2);
 }
-size_t unfold_lds_bytes(int N, int T, int rp) {
-  (void)T;
-  return (size_t)(1 + rp * 2) * N * sizeof(float2);
+// Rows per block: the most, up to 8, that fit (a single row needs 131 KB at
+// N = 5120, the longest a plan accepts).
+int gen_rb(int N) {
+  int rb = 8;
+  while (rb > 1 && gen_lds_bytes(N, rb) > kWaveLdsMax) rb /= 2;
+  return rb;
 }
 
 // ---- the reference's Fourier waist (*lead, nlat, T+1) complex ----
@@ -1274,7 +1311,7 @@ __global__ void __launch_bounds__(64 * kRowWaves) waist_from_rows_kernel(WaistRo
   if (r >= a.nlead * a.nrows) return;  // no block barrier below
   const float* x = a.rows_in + (size_t)r * N;
   float2 v[1][L];
-  static_for<L>([&](auto n1_) {
+  static_for<L>([&](auto n1_) SHT_INLINE {
     constexpr int n1 = decltype(n1_)::value;
     v[0][n1] = make_float2(x[64 * n1 + lane], 0.f);
   });
@@ -1314,46 +1351,61 @@ __global__ void __launch_bounds__(64 * kRowWaves) rows_from_waist_kernel(WaistRo
   }
   wave_sync();
   float2 v[1][L];
-  static_for<L>([&](auto n1_) { v[0][n1_] = buf[64 * decltype(n1_)::value + lane]; });
+  static_for<L>([&](auto n1_) SHT_INLINE { v[0][n1_] = buf[64 * decltype(n1_)::value + lane]; });
   wave_sync();
   wave_fft64<L, 1, +1>(v, buf, tw, lane);
   float* out = a.rows_out + (size_t)r * N;
   for (int k = lane; k < N; k += 64) out[k] = buf[k].x;
 }
 
-// The same two maps for an nlon that is not 64 L: direct sums against the
-// twiddle table, one thread per output value.
-__global__ void waist_from_rows_dft_kernel(WaistRowsArgs a) {
-  const int N = a.fft.N, T1 = a.T + 1;
-  const long long total = (long long)a.nlead * a.nrows * T1;
-  for (long long e = blockIdx.x * (long long)blockDim.x + threadIdx.x; e < total;
-       e += (long long)gridDim.x * blockDim.x) {
-    const int r = (int)(e / T1), m = (int)(e % T1);
-    const float* x = a.rows_in + (size_t)r * N;
-    float2 acc = make_float2(0.f, 0.f);
-    for (int j = 0; j < N; ++j) {
-      const float2 t = a.fft.tw[(int)(((long long)j * m) % N)];  // e^{-2 pi i j m / N}
-      acc.x += x[j] * t.x;
-      acc.y += x[j] * t.y;
-    }
-    a.waist_out[waist_row(a, r) + m] = make_float2(acc.x / (float)N, acc.y / (float)N);
+// The same two maps for any other N, by the LDS passes of the row kernels.
+__global__ void __launch_bounds__(64 * kRowWaves) waist_from_rows_gen_kernel(WaistRowsArgs a) {
+  extern __shared__ float2 lds[];
+  const int N = a.fft.N, span = gen_span(N);
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  float2* tw = lds;
+  float2* b0 = lds + N + (size_t)w * (2 * span);
+  for (int k = threadIdx.x; k < N; k += blockDim.x) tw[k] = a.fft.tw[k];
+  __syncthreads();
+  const int r = blockIdx.x * (int)(blockDim.x >> 6) + w;
+  if (r >= a.nlead * a.nrows) return;  // no block barrier below
+  const float* x = a.rows_in + (size_t)r * N;
+  gen_load_row(b0, N, lane, [&](int k) { return make_float2(x[k], 0.f); });
+  wave_sync();
+  const float2* Z = gen_fft<-1>(b0, b0 + span, N, a.fft.scalar, tw, lane);
+  const float inv = 1.0f / (float)N;
+  float2* out = a.waist_out + waist_row(a, r);
+  for (int m = lane; m <= a.T; m += kWave) {
+    const float2 z = Z[gp(m)];
+    out[m] = make_float2(z.x * inv, z.y * inv);
   }
 }
 
-__global__ void rows_from_waist_dft_kernel(WaistRowsArgs a) {
-  const int N = a.fft.N, T1 = a.T + 1;
-  const long long total = (long long)a.nlead * a.nrows * N;
-  for (long long e = blockIdx.x * (long long)blockDim.x + threadIdx.x; e < total;
-       e += (long long)gridDim.x * blockDim.x) {
-    const int r = (int)(e / N), k = (int)(e % N);
-    const float2* X = a.waist_in + waist_row(a, r);
-    float acc = X[0].x;
-    for (int m = 1; m < T1; ++m) {
-      const float2 t = a.fft.tw[(int)(((long long)k * m) % N)];  // conj: e^{+2 pi i k m / N}
-      acc += 2.f * (X[m].x * t.x + X[m].y * t.y);
+__global__ void __launch_bounds__(64 * kRowWaves) rows_from_waist_gen_kernel(WaistRowsArgs a) {
+  extern __shared__ float2 lds[];
+  const int N = a.fft.N, span = gen_span(N);
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  float2* tw = lds;
+  float2* b0 = lds + N + (size_t)w * (2 * span);
+  for (int k = threadIdx.x; k < N; k += blockDim.x) tw[k] = a.fft.tw[k];
+  __syncthreads();
+  const int r = blockIdx.x * (int)(blockDim.x >> 6) + w;
+  if (r >= a.nlead * a.nrows) return;  // no block barrier below
+  const float2* X = a.waist_in + waist_row(a, r);
+  for (int k = a.T + 1 + lane; k < N - a.T; k += kWave) b0[gp(k)] = make_float2(0.f, 0.f);
+  for (int m = lane; m <= a.T; m += kWave) {
+    const float2 A = X[m];
+    if (m == 0) {
+      b0[0] = make_float2(A.x, 0.f);  // irfft reads the real part of the m = 0 bin
+    } else {
+      b0[gp(m)] = A;
+      b0[gp(N - m)] = cconj(A);
     }
-    a.rows_out[(size_t)r * N + k] = acc;
   }
+  wave_sync();
+  const float2* x = gen_fft<+1>(b0, b0 + span, N, a.fft.scalar, tw, lane);
+  float* out = a.rows_out + (size_t)r * N;
+  for (int k = lane; k < N; k += kWave) out[k] = x[gp(k)].x;
 }
 
 // reference waist -> folded analysis waist: one thread per (field, folded row
@@ -1442,27 +1494,17 @@ size_t rows_wave_lds_bytes(int N) {
   return ((size_t)N + 64 + (size_t)kRowWaves * L * kRowSpan) * sizeof(float2);
 }
 
-// Register prefetch depth per lane: PF * 64 >= N, or 0 (no prefetch) above 1536.
-int fft_pf(int N) {
-  const int need = (N + kWave - 1) / kWave;
-  const int opts[] = {2, 4, 8, 12, 16, 24};
-  for (int o : opts)
-    if (need <= o) return o;
-  return 0;
+size_t rows_gen_lds_bytes(int N, int waves) {
+  return ((size_t)N + (size_t)waves * (2 * gen_span(N))) * sizeof(float2);
+}
+// Rows per block of the generic waist row kernels.
+int rows_gen_waves(int N) {
+  int n = kRowWaves;
+  while (n > 1 && rows_gen_lds_bytes(N, n) > kWaveLdsMax) n /= 2;
+  return n;
 }
 
 }  // namespace sht
-
-#define SHT_PF_DISPATCH(KERNEL, PF, ...)                                 \
-  switch (PF) {                                                          \
-    case 2: hipLaunchKernelGGL(sht::KERNEL<2>, __VA_ARGS__); break;      \
-    case 4: hipLaunchKernelGGL(sht::KERNEL<4>, __VA_ARGS__); break;      \
-    case 8: hipLaunchKernelGGL(sht::KERNEL<8>, __VA_ARGS__); break;      \
-    case 12: hipLaunchKernelGGL(sht::KERNEL<12>, __VA_ARGS__); break;    \
-    case 16: hipLaunchKernelGGL(sht::KERNEL<16>, __VA_ARGS__); break;    \
-    case 24: hipLaunchKernelGGL(sht::KERNEL<24>, __VA_ARGS__); break;    \
-    default: hipLaunchKernelGGL(sht::KERNEL<0>, __VA_ARGS__); break;     \
-  }
 
 #define SHT_L_DISPATCH(L, LAUNCH) \
   switch (L) {                     \
@@ -1510,13 +1552,13 @@ extern "C" hipError_t sht_launch_rfft_fold(const sht::FoldArgs* a, hipStream_t s
 #undef SHT_FOLD
     return e;
   }
-  size_t lds = sht::fold_lds_bytes(a->fft.N, a->T, a->job.vector, a->rp);
-  int blocks = a->nchunks * a->job.nfields;
-  if (blocks == 0) return hipSuccess;
-  if (a->job.rowscale_hi) return hipErrorInvalidValue;  // order-dependent scales: wave path only
-  SHT_PF_DISPATCH(rfft_fold_kernel, sht::fft_pf(a->fft.N), dim3(blocks), dim3(sht::kWave * a->rp),
-                  lds, s, *a);
-  return hipGetLastError();
+  // any other N: one component per launch
+  if (a->job.rowscale_hi || a->job.vector) return hipErrorInvalidValue;
+  const int rb = sht::gen_rb(a->fft.N);
+  const int groups = a->job.nfields * (a->JHP / rb);
+  if (groups == 0) return hipSuccess;
+  return sht::launch_persistent(sht::rfft_fold_rows_kernel, groups, rb,
+                                sht::gen_lds_bytes(a->fft.N, rb), s, *a);
 }
 
 extern "C" hipError_t sht_launch_irfft_unfold(const sht::UnfoldArgs* a, hipStream_t s) {
@@ -1550,22 +1592,12 @@ extern "C" hipError_t sht_launch_irfft_unfold(const sht::UnfoldArgs* a, hipStrea
 #undef SHT_UNFOLD
     return e;
   }
-  size_t lds = sht::unfold_lds_bytes(a->fft.N, a->T, a->rp);
-  int blocks = a->nchunks * a->job.nfields;
-  if (blocks == 0) return hipSuccess;
   if (a->job.rowscale_hi) return hipErrorInvalidValue;  // order-dependent scales: wave path only
-  SHT_PF_DISPATCH(irfft_unfold_kernel, sht::fft_pf(a->fft.N), dim3(blocks),
-                  dim3(sht::kWave * a->rp), lds, s, *a);
-  return hipGetLastError();
-}
-
-template <int PF>
-static hipError_t allow_lds_one(size_t bytes) {
-  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(sht::rfft_fold_kernel<PF>),
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
-  if (e != hipSuccess) return e;
-  return hipFuncSetAttribute(reinterpret_cast<const void*>(sht::irfft_unfold_kernel<PF>),
-                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+  const int rb = sht::gen_rb(a->fft.N);
+  const int groups = a->job.nfields * ((a->JH + rb - 1) / rb);
+  if (groups == 0) return hipSuccess;
+  return sht::launch_persistent(sht::irfft_unfold_rows_kernel, groups, rb,
+                                sht::gen_lds_bytes(a->fft.N, rb), s, *a);
 }
 
 template <int L>
@@ -1605,24 +1637,21 @@ extern "C" size_t sht_fft_wave_lds_bytes(int N, int vector) {
   return sht::wave_rb(b8) == 8 ? b8 : sht::unfold_wave_lds_bytes(N, 4);
 }
 
-extern "C" hipError_t sht_fft_allow_lds(size_t bytes, size_t wave_bytes) {
+extern "C" hipError_t sht_fft_allow_lds(size_t bytes) {
   hipError_t e = hipSuccess;
-  const size_t wb = wave_bytes;
-  for (hipError_t r : {allow_lds_wave<2>(wb), allow_lds_wave<3>(wb), allow_lds_wave<4>(wb),
-                       allow_lds_wave<6>(wb), allow_lds_wave<8>(wb), allow_lds_wave<12>(wb),
-                       allow_lds_wave<16>(wb), allow_lds_wave<24>(wb)})
+  for (hipError_t r : {allow_lds_wave<2>(bytes), allow_lds_wave<3>(bytes), allow_lds_wave<4>(bytes),
+                       allow_lds_wave<6>(bytes), allow_lds_wave<8>(bytes), allow_lds_wave<12>(bytes),
+                       allow_lds_wave<16>(bytes), allow_lds_wave<24>(bytes)})
     if (r != hipSuccess) e = r;
-  for (hipError_t r : {allow_lds_one<0>(bytes), allow_lds_one<2>(bytes), allow_lds_one<4>(bytes),
-                       allow_lds_one<8>(bytes), allow_lds_one<12>(bytes), allow_lds_one<16>(bytes),
-                       allow_lds_one<24>(bytes)})
+  for (const void* k : {reinterpret_cast<const void*>(sht::rfft_fold_rows_kernel),
+                        reinterpret_cast<const void*>(sht::irfft_unfold_rows_kernel),
+                        reinterpret_cast<const void*>(sht::waist_from_rows_gen_kernel),
+                        reinterpret_cast<const void*>(sht::rows_from_waist_gen_kernel)}) {
+    hipError_t r = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
     if (r != hipSuccess) e = r;
+  }
   return e;
 }
-
-extern "C" size_t sht_fold_lds_bytes(int N, int T, int vector, int rp) {
-  return sht::fold_lds_bytes(N, T, vector, rp);
-}
-extern "C" size_t sht_unfold_lds_bytes(int N, int T, int rp) { return sht::unfold_lds_bytes(N, T, rp); }
 
 static unsigned grid_for(long long total) {
   long long b = (total + 255) / 256;
@@ -1640,8 +1669,9 @@ extern "C" hipError_t sht_launch_waist_from_rows(const sht::WaistRowsArgs* a, hi
     SHT_L_DISPATCH(L, SHT_W2R)
 #undef SHT_W2R
   } else {
-    hipLaunchKernelGGL(sht::waist_from_rows_dft_kernel, dim3(grid_for(R * (a->T + 1))), dim3(256),
-                       0, s, *a);
+    const int n = sht::rows_gen_waves(a->fft.N);
+    hipLaunchKernelGGL(sht::waist_from_rows_gen_kernel, dim3((unsigned)((R + n - 1) / n)), dim3(64 * n),
+                       sht::rows_gen_lds_bytes(a->fft.N, n), s, *a);
   }
   return hipGetLastError();
 }
@@ -1656,8 +1686,9 @@ extern "C" hipError_t sht_launch_rows_from_waist(const sht::WaistRowsArgs* a, hi
     SHT_L_DISPATCH(L, SHT_R2W)
 #undef SHT_R2W
   } else {
-    hipLaunchKernelGGL(sht::rows_from_waist_dft_kernel, dim3(grid_for(R * a->fft.N)), dim3(256),
-                       0, s, *a);
+    const int n = sht::rows_gen_waves(a->fft.N);
+    hipLaunchKernelGGL(sht::rows_from_waist_gen_kernel, dim3((unsigned)((R + n - 1) / n)), dim3(64 * n),
+                       sht::rows_gen_lds_bytes(a->fft.N, n), s, *a);
   }
   return hipGetLastError();
 }

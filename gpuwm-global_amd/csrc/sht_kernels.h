@@ -7,7 +7,6 @@
 namespace sht {
 
 constexpr int kMT = 4;           // m-tile of the waist layout W[c][m/4][p][i][m%4]
-constexpr int kFftThreads = 256;
 constexpr int kMaxStages = 16;
 
 // ---- tables (sht_tables.hip) ----
@@ -43,11 +42,15 @@ struct TableOut {
 };
 
 // ---- FFT (sht_fft.hip) ----
+struct FftPasses {
+  int n;
+  int direct;                 // radices above 4 by direct sums
+  int radix[kMaxStages];
+};
 struct FftPlan {
   int N;                      // nlon
   int wave_L;                 // N / 64 when the wave-resident path runs, else 0
-  int nstages;
-  int radix[kMaxStages];
+  FftPasses scalar, vector;   // passes of the row kernels (any other N)
   const float2* tw;           // tw[k] = exp(-2 pi i k / N), k < N
   const double2* tw64;        // the same in FP64 (the FP64 FFTs)
 };
@@ -71,18 +74,15 @@ struct FoldJob {
   double2* low;
   const double* rowscale64;   // per folded row, FP64
   const double* rowscale64_hi;  // orders m >= m0 of the fp32 waist (NULL: rowscale64)
-  int fstride;
+  int fstride;                // columns between fields (FP64 fold and row kernels)
   int m0;
   int low_stride;             // double2 per field
+  int imul;                   // row kernels: write the columns of i X
 };
 
 struct FoldArgs {
   FftPlan fft;
   int T, nlat, JH, JHP;
-  int rp;                     // folded rows (wavefronts) per block (1, 2 or 4)
-  int ngroups;                // folded-row groups covering JHP rows
-  int gpb;                    // groups per block
-  int nchunks;                // ceil(ngroups / gpb)
   FoldJob job;
 };
 
@@ -98,6 +98,7 @@ struct UnfoldJob {
   int ldw;
   int imul;                   // multiply the spectrum by 1: i, 2: i m before the FFT
   int post_exp;               // write exp() of the grid values
+  int wind;                   // a component of a wind (row kernels: the vector passes)
   // FP64 unfold (irfft_unfold_wave64_kernel): the spectrum is assembled and
   // inverted in FP64, orders m < m0 read from low + f low_stride ([m][p][i]
   // folded (E, O) in FP64) instead of the fp32 waist
@@ -112,10 +113,6 @@ struct UnfoldJob {
 struct UnfoldArgs {
   FftPlan fft;
   int T, nlat, JH, JHP;
-  int rp;
-  int ngroups;                // ceil(JH / rp)
-  int gpb;                    // groups per block
-  int nchunks;                // ceil(ngroups / gpb)
   UnfoldJob job;
 };
 
@@ -322,9 +319,7 @@ hipError_t sht_launch_legendre_tables(int T, int nlat, int JH, int JHP, const do
                                       const int* koff, const sht::TableOut* out, hipStream_t s);
 hipError_t sht_launch_rfft_fold(const sht::FoldArgs* a, hipStream_t s);
 hipError_t sht_launch_irfft_unfold(const sht::UnfoldArgs* a, hipStream_t s);
-size_t sht_fold_lds_bytes(int N, int T, int vector, int rp);
-size_t sht_unfold_lds_bytes(int N, int T, int rp);
-hipError_t sht_fft_allow_lds(size_t bytes, size_t wave_bytes);
+hipError_t sht_fft_allow_lds(size_t bytes);
 int sht_fft_wave_L(int N);                       // 0: no wave-resident path for N
 size_t sht_fft_wave_lds_bytes(int N, int vector);
 hipError_t sht_launch_legendre_gemm(const sht::GemmLaunch* launch, hipStream_t s);
