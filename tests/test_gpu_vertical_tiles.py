@@ -1,0 +1,60 @@
+"""The column operators where their tiles end: levels either side of each
+16-row tile, truncations whose orders do not fill a wavefront's 16 or a
+block's 128, against the FP64 oracle.
+
+Tolerance: three chained fp32 products of up to 65 terms, each at most
+sqrt(65) half-ulps (6e-8) of its result: 3 sqrt(65) 6e-8 = 1.5e-6, rounded up
+to 2e-6 of the largest value.
+"""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from _helpers import hip_transform
+from oracle import semi_implicit as osi
+from oracle.sht import OracleTransform, red_spectrum
+
+pytestmark = pytest.mark.gpu
+
+TOL = 2e-6
+
+
+def _close(got, want):
+    for g, w in zip(got, want):
+        g = g.detach().cpu().numpy()
+        assert np.max(np.abs(g - w)) < TOL * np.max(np.abs(w))
+        t1 = g.shape[-1]
+        assert not (g * np.triu(np.ones((t1, t1)), 1)).any()
+        assert not g[..., 0].imag.any()
+
+
+@pytest.mark.parametrize("trunc,nlev", [(3, 1), (14, 15), (15, 16), (16, 17), (21, 31), (30, 32),
+                                        (33, 47), (31, 48), (20, 63), (130, 9), (127, 5)])
+def test_levels_and_orders_at_the_edges_of_tiles(trunc, nlev):
+    from arwen_spectral import semi_implicit as si
+
+    o = OracleTransform.create(trunc, dealias_factor=1.0)
+    t = hip_transform(o, "float32")
+    f32 = lambda a: np.asarray(a, dtype=np.float32)  # noqa: E731
+    c64 = lambda a: np.asarray(a).astype(np.complex64)  # noqa: E731
+    b, c, m, modal = osi.synthetic_operator(nlev, seed=nlev)
+    k2 = f32(si.wave_operator(t))
+    # the half maps' modes come from the FP64 operator (rounded first, its null
+    # mode turns into a growing one)
+    maps = [f32(x) for x in osi.symmetric_half_maps(modal, osi.x_modes(b, c), k2, 1500.0, 0.6)]
+    b, c, m = f32(b), f32(c), f32(m)
+    d = c64(o.project(red_spectrum(trunc, (nlev,), seed=1, scale=1e-5)))
+    th = c64(o.project(red_spectrum(trunc, (nlev,), seed=2, scale=10.0)))
+    ps = c64(o.project(red_spectrum(trunc, (), seed=3, scale=1e-2)))
+    d[:, 0, 0], th[:, 0, 0], ps[0, 0] = 1e-6, 250.0, 0.3
+    inv = f32(osi.helmholtz_inverse(modal, k2, 900.0, 1.0))
+    _close(si.vertical_solve_shifted(t, d, th, ps, b, c, inv, k2, 900.0),
+           osi.solve_shifted(o, d, th, ps, b, c, inv, k2, np.float32(900.0)))
+    inv = f32(osi.helmholtz_inverse(modal, k2, 600.0, 0.6))
+    _close(si.vertical_apply(t, d, th, ps, b, c, m, inv, k2, 600.0, 0.6),
+           osi.apply(o, d, th, ps, b, c, m, inv, k2, np.float32(600.0), 0.6))
+    _close(si.vertical_linear_tendencies(t, d, th, ps, b, c, k2, 0.7),
+           osi.linear_tendencies(o, d, th, ps, b, c, k2, np.float32(0.7)))
+    _close(si.vertical_half_apply(t, d, th, ps, b, c, *maps, k2),
+           osi.half_apply(o, d, th, ps, b, c, maps, k2))
