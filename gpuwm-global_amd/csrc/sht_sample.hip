@@ -1,19 +1,30 @@
 // Spectral fields evaluated at arbitrary points (reference
 // spectral/sampling.py:382-515: sample_scalar, sample_gradient, sample_wind).
 //
-// One lane per two points, one block per (512 points, tile of FT fields, part
-// of the order range).  The lane walks its part of the triangle order by order: the normalized associated-Legendre
-// recurrence of its point in FP64 (reference legendre.py:86-146, the
-// reference's operand order in every expression but the derivative's
-// division, see rd below; this file is compiled with -ffp-contract=off and
-// the contractions below are explicit fma), and for
-// each (n, m) the tile's coefficients, which every lane of the block reads
-// at the same address, multiply-add into per-order amplitudes held in
-// registers.  Each order's amplitude is turned by the zonal phase
-// e^{i m lambda} and added into FP64 outputs.  No basis cube is stored: the
-// reference's device path materialises a (2K x points) basis per point chunk
-// for a GEMM, which on MI355X buys nothing (the FP64 and FP32 matrix peaks
-// equal the vector ones) and costs 8 bytes per basis value of HBM traffic.
+// Per order m a field's amplitude at a point is a sum over degrees of
+// coefficient times basis value, turned by e^{i m lambda} and added into the
+// output.  The amplitudes of 16 PT points and 16 CT columns (real and
+// imaginary parts of 8 fields each) are one wavefront's tiles of
+//     A (points x 4 degrees) B (4 degrees x columns)
+// on v_mfma_f64_16x16x4_f64 (v_mfma_f32_16x16x4_f32 for the float32 sampler),
+// four degrees of one order per step.  The basis is generated as it is used:
+// a lane runs the normalized associated-Legendre recurrence of its point in
+// FP64 (reference legendre.py:86-146, the reference's operand order in every
+// expression but the derivative's division, see rd below; this file is
+// compiled with -ffp-contract=off), four degrees a step, and hands them over
+// in A's layout through the wavefront's LDS.  No basis cube is stored (the
+// reference's device path materialises a (2K x points) basis per point chunk,
+// 8 bytes of HBM traffic per value).
+//
+// Bound: the FP64 matrix pipe, whose peak equals the vector peak; what the
+// former kernel (lane = two points, coefficients by scalar loads) lacked was
+// operands, since a scalar load feeds one wavefront's multiply-adds and waits
+// for all loads at once.  Here a coefficient is loaded once per lane for PT
+// MFMAs and a basis value feeds CT.  T383, 30,000 points: 40 fields 11.25 ->
+// 7.10 ms in float64 (51 TFLOP/s; 62 is what a large FP64 matrix product
+// reaches), 9.18 -> 4.74 ms in float32 (bound by the FP64 recurrence); their
+// gradients 19.9 -> 19.1 and 19.5 -> 14.5 ms (the derivative's recurrence
+// runs beside two MFMAs a value); 3 fields at 300 points 2.84 -> 0.73 ms.
 //
 // Precision: F32 = false accumulates in FP64; F32 = true rounds each basis
 // value to fp32 and accumulates an order's terms in fp32 before the FP64 sum
@@ -22,6 +33,7 @@
 
 #include <math.h>
 
+#include <algorithm>
 #include <type_traits>
 
 namespace sht {
@@ -32,8 +44,7 @@ __device__ __forceinline__ long long tri_index(int T, int n, int m) {
 }
 
 // (count, T+1, T+1) complex64 [n, m] -> (K, ldc) complex, fields fastest:
-// complex128 for the float64 sampler (the FMAs then take the coefficient
-// straight from scalar registers), complex64 for the float32 one; columns
+// complex128 for the float64 sampler, complex64 for the float32 one; columns
 // past the live fields are zero.  Winds: column 2l is psi and 2l + 1 chi of
 // level l, from vorticity / divergence by the inverse Laplacian.
 __global__ void sample_pack_kernel(SamplePackArgs a) {
@@ -66,11 +77,19 @@ __global__ void sample_pack_kernel(SamplePackArgs a) {
   }
 }
 
+typedef double d4 __attribute__((ext_vector_type(4)));
+typedef float f4 __attribute__((ext_vector_type(4)));
 template <bool F32>
 struct SampleAcc {
   using T = typename std::conditional<F32, float, double>::type;
-  using C = typename std::conditional<F32, float2, double2>::type;
+  using D = typename std::conditional<F32, f4, d4>::type;
 };
+__device__ __forceinline__ void sample_mfma(d4& acc, double a, double b) {
+  acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc, 0, 0, 0);
+}
+__device__ __forceinline__ void sample_mfma(f4& acc, float a, float b) {
+  acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, acc, 0, 0, 0);
+}
 
 // The outputs of one point from its two sums (s0: values, or zonal sums
 // d/dlambda; s1: meridional sums d/dphi).  KIND 0: the field; 1: east and
@@ -100,30 +119,39 @@ __device__ __forceinline__ void sample_store(int col, int p, int npts, int nout,
   }
 }
 
-// One block: 256 x PT points (lane l takes points l, l + 256, ...) x FT field
-// columns x one part of the order range (orders mcut[r] .. mcut[r+1]-1, cut
-// so the parts hold equal shares of the triangle).  With one part the block
-// stores the outputs; with several it stores its two raw sums per (column,
-// point) into part r of `partial` and sample_reduce_kernel adds the parts in
-// order.  The (m, n) walk is one loop over the packed index k.  The
-// coefficients arrive through scalar loads; those return out of order, so a
-// wave can wait only for all of them, and the next step's loads are the only
-// ones in flight while a step computes: each lane takes PT points so that
-// every load feeds PT x FT x 2 multiply-adds.
-constexpr int kSamplePts = 2;  // PT
-
-template <int FT, int KIND, bool F32>
-__global__ void __launch_bounds__(256) sample_kernel(
-    const typename SampleAcc<F32>::C* __restrict__ coef, const double* __restrict__ rec,
+// One wavefront: 16 PT points x CT column tiles (8 fields each) x one part of
+// the order range (orders mcut[r] .. mcut[r+1]-1, cut so the parts hold equal
+// shares of the triangle); the four wavefronts of a block take neighbouring
+// points and read the same coefficients.  With one part the outputs are
+// stored; with several the two raw sums per (column, point) go to part r of
+// `partial` and sample_reduce_kernel adds the parts in order.  An output's
+// arithmetic depends on neither PT, CT nor its neighbours.
+// MFMA operands: lane l = (g = l / 16, q = l % 16); A holds point q of the
+// tile at degree n0 + g, B degree n0 + g at column q; accumulator register i
+// is point g + 4 i (FP64) or 4 g + i (fp32) at column q.
+template <int PT, int CT, int KIND, bool F32>
+__global__ void __launch_bounds__(256, 2) sample_kernel(
+    const typename SampleAcc<F32>::T* __restrict__ coef, const double* __restrict__ rec,
     const double* __restrict__ diag, const double* __restrict__ sin_lat,
     const double* __restrict__ cos_lat, const double* __restrict__ lon, SampleCuts cuts, int T,
     int npts, int ldc, int nout, double radius, double* __restrict__ out0,
     double* __restrict__ out1, double* __restrict__ partial) {
   using Acc = typename SampleAcc<F32>::T;
-  using Cx = typename SampleAcc<F32>::C;
+  using D = typename SampleAcc<F32>::D;
   constexpr bool GRAD = KIND != 0;
-  constexpr int PT = kSamplePts;
-  const int c0 = blockIdx.y * FT;
+  constexpr int NP = 16 * PT;              // points of this wavefront
+  constexpr int NB = GRAD ? 2 : 1;         // bases: P, dP/dphi
+  // per wavefront: basis values [2 buffers][P, dP][degree][point], then
+  // cos and sin of the order's phase per point
+  __shared__ Acc sA[4][2][NB][4][NP];
+  __shared__ double sE[4][2][NP];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int g = lane >> 4, q = lane & 15;
+  const int p0 = ((int)blockIdx.x * 4 + wv) * NP;
+  if (p0 >= npts) return;  // wave-uniform; no block barrier in this kernel
+  // the last group of column tiles starts early enough to be whole: its first
+  // tiles may be another group's too, with the same bits
+  const int ct0 = min((int)blockIdx.y * CT, ldc / 8 - CT);
   const int r = blockIdx.z;
   const int m0 = cuts.m[r], m1 = cuts.m[r + 1];
   const long long K = (long long)(T + 1) * (T + 2) / 2;
@@ -132,173 +160,211 @@ __global__ void __launch_bounds__(256) sample_kernel(
   const double* rec_c = rec + 2 * K;
   const double* diag_f = diag;
   const double* diag_g = diag + (T + 1);
-  const Cx* cf = coef + c0;
   const double pi = 3.14159265358979323846;
 
-  int pt[PT];
-  double x[PT], lam[PT], root[PT], denom[PT], dg[PT], prev[PT], prev2[PT];
+  // the recurrence of point lane % NP (every 64 / NP-th lane the same one)
+  const int mine = lane % NP;
+  const int pp = min(p0 + mine, npts - 1);  // past the end: a real point
+  const double x = sin_lat[pp], lam = lon[pp];
+  const double root = sqrt(fmax(0.0, 1.0 - x * x));
   // dP = root (n x P - c P_{n-1}) / (x^2 - 1): the division by the point's
   // constant (x^2 - 1) is one multiplication by rd = root / (x^2 - 1), one
   // rounding more than the reference's form and ~10 FP64 instructions less
   // per (n, m) step
-  double rd[PT];
-#pragma unroll
-  for (int q = 0; q < PT; ++q) {
-    pt[q] = blockIdx.x * (256 * PT) + q * 256 + threadIdx.x;
-    const int pp = pt[q] < npts ? pt[q] : npts - 1;  // idle lanes evaluate a real point
-    x[q] = sin_lat[pp];
-    lam[q] = lon[pp];
-    root[q] = sqrt(fmax(0.0, 1.0 - x[q] * x[q]));
-    denom[q] = x[q] * x[q] - 1.0;
-    rd[q] = root[q] / denom[q];
-    dg[q] = 1.0 / sqrt(4.0 * pi);
-    for (int mm = 1; mm <= m0; ++mm) dg[q] = diag_f[mm] * root[q] * dg[q];  // P_{m0 m0}
-    prev[q] = prev2[q] = 0.0;
-  }
+  const double rd = GRAD ? root / (x * x - 1.0) : 0.0;
+  double dg = 1.0 / sqrt(4.0 * pi);
+  for (int mm = 1; mm <= m0; ++mm) dg = diag_f[mm] * root * dg;  // P_{m0 m0}
 
-  double o0[PT][FT], o1[PT][FT];
-  Acc ar[PT][FT], ai[PT][FT], dr[PT][FT], di[PT][FT];
+  double o[NB][PT][CT][4];
 #pragma unroll
-  for (int q = 0; q < PT; ++q)
+  for (int b = 0; b < NB; ++b)
 #pragma unroll
-    for (int f = 0; f < FT; ++f) {
-      o0[q][f] = o1[q][f] = 0.0;
-      ar[q][f] = ai[q][f] = dr[q][f] = di[q][f] = Acc(0);
-    }
+    for (int t = 0; t < PT; ++t)
+#pragma unroll
+      for (int c = 0; c < CT; ++c)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[b][t][c][i] = 0.0;
 
-  // The packed triangle is order-major, so the steps (m, n) of the part are
-  // consecutive entries k0 .. k_last: the coefficient and recurrence pointers
-  // advance by one entry per step, and each order runs as its diagonal step,
-  // its first off-diagonal step and a branch-free loop over n = m+2 .. T.
-  // Every step loads the next entry's values once it has used its own (the
-  // last step reloads its own, so no load passes k_last).
-  const long long k0 = tri_index(T, m0, m0);         // (n, m) = (m0, m0)
-  const long long k_last = tri_index(T, T, m1 - 1);  // (T, m1 - 1)
-  const Cx* cp = cf + k0 * ldc;
-  const double *pa = rec_a + k0, *pb = rec_b + k0, *pc = rec_c + k0;
-  long long left = k_last - k0;  // steps after the current one
-  Cx cur[FT];
-#pragma unroll
-  for (int f = 0; f < FT; ++f) cur[f] = cp[f];
-  double ca = pa[0], cb = pb[0], cc = pc[0];
-  // one step: P (and dP) of every point from `rule`, into the amplitudes
-  auto step = [&](auto rule) {
-#pragma unroll
-    for (int q = 0; q < PT; ++q) {
-      double P, dP = 0.0;
-      rule(q, P, dP);
-#pragma unroll
-      for (int f = 0; f < FT; ++f) {
-        if constexpr (F32) {
-          ar[q][f] = fmaf(cur[f].x, (float)P, ar[q][f]);
-          ai[q][f] = fmaf(cur[f].y, (float)P, ai[q][f]);
-          if constexpr (GRAD) {
-            dr[q][f] = fmaf(cur[f].x, (float)dP, dr[q][f]);
-            di[q][f] = fmaf(cur[f].y, (float)dP, di[q][f]);
-          }
-        } else {
-          ar[q][f] = fma(cur[f].x, P, ar[q][f]);
-          ai[q][f] = fma(cur[f].y, P, ai[q][f]);
-          if constexpr (GRAD) {
-            dr[q][f] = fma(cur[f].x, dP, dr[q][f]);
-            di[q][f] = fma(cur[f].y, dP, di[q][f]);
-          }
-        }
-      }
-      prev2[q] = prev[q];
-      prev[q] = P;
-    }
-    // the next entry's values go into the same registers once this step has
-    // used them: scalar loads return out of order, so a wave waits for all of
-    // its outstanding ones at once and a second register set would buy no
-    // overlap, only scalar registers (and their spills)
-    const long long adv = left > 0 ? 1 : 0;
-    cp += adv * ldc;
-    pa += adv;
-    pb += adv;
-    pc += adv;
-    --left;
-#pragma unroll
-    for (int f = 0; f < FT; ++f) cur[f] = cp[f];
-    ca = pa[0];
-    cb = pb[0];
-    cc = pc[0];
-  };
+  const size_t row = 2 * (size_t)ldc;  // values of one packed (n, m)
   for (int m = m0; m < m1; ++m) {
-    // n = m
-    step([&](int q, double& P, double& dP) {
-      P = dg[q];
-      if constexpr (GRAD) dP = (m >= 1) ? rd[q] * ((double)m * x[q] * dg[q]) : 0.0;
-    });
-    if (m < T) {
-      // n = m + 1
-      const double g = diag_g[m];
-      const int n = m + 1;
-      step([&](int q, double& P, double& dP) {
-        P = g * x[q] * dg[q];
-        if constexpr (GRAD) dP = rd[q] * ((double)n * x[q] * P - cc * prev[q]);
-      });
-      for (int n2 = m + 2; n2 <= T; ++n2) {
-        step([&](int q, double& P, double& dP) {
-          P = ca * (x[q] * prev[q] - cb * prev2[q]);
-          if constexpr (GRAD) dP = rd[q] * ((double)n2 * x[q] * P - cc * prev[q]);
-        });
+    const long long k0 = tri_index(T, m, m);
+    const int len = T + 1 - m;  // degrees
+    const Acc* cp = coef + ((size_t)k0 + g) * row + 16 * ct0 + q;  // degree m + g
+    D acc[NB][PT][CT];
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int t = 0; t < PT; ++t)
+#pragma unroll
+        for (int c = 0; c < CT; ++c) acc[b][t][c] = D{0, 0, 0, 0};
+    // degrees m + j + g of the step at j; past T the order's last row, taken
+    // as 0 by `tail` steps
+    auto load_b = [&](Acc(&v)[CT], int j) {
+      const Acc* at = cp + (long long)(min(j + g, len - 1) - g) * (long long)row;
+#pragma unroll
+      for (int c = 0; c < CT; ++c) v[c] = at[16 * c];
+    };
+    double prev = 0.0, prev2 = 0.0;  // P of the two degrees before
+    // basis values of the step at j into buffer `buf`; FIRST: j = 0, whose
+    // degrees m and m + 1 have their own rules; TAIL: degrees past T are 0
+    auto basis = [&](auto FIRST, auto TAIL, int j, int buf) {
+      constexpr bool first = decltype(FIRST)::value, tail = decltype(TAIL)::value;
+      double P[4], dP[4];
+      double ra[4], rb[4], rc[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const long long k = k0 + (tail ? min(j + u, len - 1) : j + u);
+        ra[u] = rec_a[k];
+        rb[u] = rec_b[k];
+        rc[u] = GRAD ? rec_c[k] : 0.0;
       }
-    }
-    // the order is complete: turn its amplitudes by e^{i m lambda}
-    const double mult = m == 0 ? 1.0 : 2.0;
 #pragma unroll
-    for (int q = 0; q < PT; ++q) {
-      double sm, cm;
-      sincos((double)m * lam[q], &sm, &cm);
-#pragma unroll
-      for (int f = 0; f < FT; ++f) {
-        const double re = (double)ar[q][f], im = (double)ai[q][f];
-        if constexpr (KIND == 0) {
-          o0[q][f] += mult * (re * cm - im * sm);
-        } else {
-          // Re(i m A e^{i m lambda}) and Re(dA e^{i m lambda})
-          o0[q][f] += mult * (-(double)m * (re * sm + im * cm));
-          o1[q][f] += mult * ((double)dr[q][f] * cm - (double)di[q][f] * sm);
+      for (int u = 0; u < 4; ++u) {
+        double v;
+        if (first && u == 0) v = dg;
+        else if (first && u == 1) v = diag_g[m] * x * dg;
+        else v = ra[u] * (x * prev - rb[u] * prev2);
+        double d = 0.0;
+        if constexpr (GRAD) {
+          const double nn = (double)(m + j + u);
+          if (first && u == 0) d = m >= 1 ? rd * (nn * x * dg) : 0.0;
+          else d = rd * (nn * x * v - rc[u] * prev);
         }
-        ar[q][f] = ai[q][f] = dr[q][f] = di[q][f] = Acc(0);
+        prev2 = prev;
+        prev = v;
+        P[u] = tail && j + u >= len ? 0.0 : v;
+        dP[u] = tail && j + u >= len ? 0.0 : d;
+      }
+      // the lanes that share a point write its four degrees between them
+      constexpr int SHARE = 64 / NP, EACH = 4 / SHARE;
+      const int part = lane / NP;
+#pragma unroll
+      for (int e = 0; e < EACH; ++e) {
+        double v = P[e], d = dP[e];
+#pragma unroll
+        for (int h = 1; h < SHARE; ++h) {
+          v = part == h ? P[h * EACH + e] : v;
+          d = part == h ? dP[h * EACH + e] : d;
+        }
+        sA[wv][buf][0][part * EACH + e][mine] = (Acc)v;
+        if constexpr (GRAD) sA[wv][buf][NB - 1][part * EACH + e][mine] = (Acc)d;
+      }
+    };
+    auto lds_sync = [] {  // this wavefront's LDS accesses, in order
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    // one step: the A fragments of `buf`, its coefficients v; the next step's
+    // basis values and the coefficients two steps ahead are started before
+    // the MFMAs.  TAIL: this step or the next may pass T.
+    auto step = [&](Acc(&v)[CT], int j, int buf, auto TAIL) {
+      Acc a[NB][PT], b[CT];
+#pragma unroll
+      for (int s = 0; s < NB; ++s)
+#pragma unroll
+        for (int t = 0; t < PT; ++t) a[s][t] = sA[wv][buf][s][g][16 * t + q];
+#pragma unroll
+      for (int c = 0; c < CT; ++c) {
+        b[c] = v[c];
+        if (decltype(TAIL)::value) b[c] = j + g < len ? b[c] : Acc(0);
+      }
+      load_b(v, j + 8);
+      basis(std::false_type{}, TAIL, j + 4, buf ^ 1);
+      lds_sync();
+#pragma unroll
+      for (int s = 0; s < NB; ++s)
+#pragma unroll
+        for (int t = 0; t < PT; ++t)
+#pragma unroll
+          for (int c = 0; c < CT; ++c) sample_mfma(acc[s][t][c], a[s][t], b[c]);
+    };
+    Acc v0[CT], v1[CT];
+    load_b(v0, 0);
+    load_b(v1, 4);
+    basis(std::true_type{}, std::true_type{}, 0, 0);
+    lds_sync();
+    int j = 0;
+    for (; j + 12 <= len; j += 8) {  // both steps and the basis values after them whole
+      step(v0, j, 0, std::false_type{});
+      step(v1, j + 4, 1, std::false_type{});
+    }
+    for (int buf = 0; j < len; j += 4, buf ^= 1) {  // at most three steps
+      step(v0, j, buf, std::true_type{});
+#pragma unroll
+      for (int c = 0; c < CT; ++c) {
+        const Acc y = v0[c];
+        v0[c] = v1[c];
+        v1[c] = y;
       }
     }
-    if (m + 1 <= T) {
-      const double fm = diag_f[m + 1];
-#pragma unroll
-      for (int q = 0; q < PT; ++q) dg[q] = fm * root[q] * dg[q];
+    // the order is complete: turn its amplitudes by e^{i m lambda}.  The real
+    // column of a field takes cos (for d/dlambda: -m sin), the imaginary one
+    // -sin (-m cos); the two are added at the end.
+    const double mult = m == 0 ? 1.0 : 2.0;
+    {
+      double sm, cm;
+      sincos((double)m * lam, &sm, &cm);
+      sE[wv][0][mine] = mult * cm;
+      sE[wv][1][mine] = mult * sm;
     }
-  }
+    lds_sync();
+    const bool im = q & 1;
 #pragma unroll
-  for (int q = 0; q < PT; ++q) {
-    const int p = pt[q];
-    if (p >= npts) continue;
-    if (gridDim.z > 1) {
-      // raw sums of this part: partial[r][c][p], then [R + r] for the second sum
-      const size_t plane = (size_t)ldc * npts;
+    for (int t = 0; t < PT; ++t)
 #pragma unroll
-      for (int f = 0; f < FT; ++f) {
-        partial[(size_t)r * plane + (size_t)(c0 + f) * npts + p] = o0[q][f];
-        if constexpr (GRAD)
-          partial[(size_t)(gridDim.z + r) * plane + (size_t)(c0 + f) * npts + p] = o1[q][f];
+      for (int i = 0; i < 4; ++i) {
+        const int at = 16 * t + (F32 ? 4 * g + i : g + 4 * i);
+        const double cm = sE[wv][0][at], sm = sE[wv][1][at];
+        const double w = im ? -sm : cm;
+        if constexpr (KIND == 0) {
+#pragma unroll
+          for (int c = 0; c < CT; ++c) o[0][t][c][i] = fma((double)acc[0][t][c][i], w, o[0][t][c][i]);
+        } else {
+          const double wz = -(double)m * (im ? cm : sm);
+#pragma unroll
+          for (int c = 0; c < CT; ++c) {
+            o[0][t][c][i] = fma((double)acc[0][t][c][i], wz, o[0][t][c][i]);
+            o[NB - 1][t][c][i] = fma((double)acc[NB - 1][t][c][i], w, o[NB - 1][t][c][i]);
+          }
+        }
       }
-      continue;
-    }
-    const double coslat = KIND == 0 ? 0.0 : cos_lat[p];
-    if constexpr (KIND == 2) {
-      static_assert(FT % 2 == 0, "wind tiles hold whole (psi, chi) pairs");
-#pragma unroll
-      for (int f = 0; f < FT; f += 2)
-        sample_store<KIND>(c0 + f, p, npts, nout, o0[q][f], o1[q][f], o0[q][f + 1],
-                           o1[q][f + 1], radius, coslat, out0, out1);
-    } else {
-#pragma unroll
-      for (int f = 0; f < FT; ++f)
-        sample_store<KIND>(c0 + f, p, npts, nout, o0[q][f], o1[q][f], 0.0, 0.0, radius, coslat,
-                           out0, out1);
-    }
+    lds_sync();  // the phases are read before the next order's land
+    if (m + 1 <= T) dg = diag_f[m + 1] * root * dg;
   }
+
+  // real and imaginary shares meet; lane pair (2 f, 2 f + 1) of a tile is field f
+  const size_t plane = (size_t)ldc * npts;
+#pragma unroll
+  for (int t = 0; t < PT; ++t)
+#pragma unroll
+    for (int c = 0; c < CT; ++c)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        double s0 = o[0][t][c][i], s1 = GRAD ? o[NB - 1][t][c][i] : 0.0;
+        s0 += __shfl_xor(s0, 1);
+        if constexpr (GRAD) s1 += __shfl_xor(s1, 1);
+        const int p = p0 + 16 * t + (F32 ? 4 * g + i : g + 4 * i);
+        const int col = 8 * (ct0 + c) + (q >> 1);
+        const bool ok = p < npts && !(q & 1);
+        if (gridDim.z > 1) {
+          // raw sums of this part: partial[r][col][p], then [R + r] for the second
+          if (ok) {
+            partial[(size_t)r * plane + (size_t)col * npts + p] = s0;
+            if constexpr (GRAD)
+              partial[(size_t)(gridDim.z + r) * plane + (size_t)col * npts + p] = s1;
+          }
+          continue;
+        }
+        double s0b = 0.0, s1b = 0.0;
+        if constexpr (KIND == 2) {  // the level's chi, two lanes on
+          s0b = __shfl_xor(s0, 2);
+          s1b = __shfl_xor(s1, 2);
+        }
+        if (ok && !(KIND == 2 && (q & 2)))
+          sample_store<KIND>(col, p, npts, nout, s0, s1, s0b, s1b, radius,
+                             KIND == 0 ? 0.0 : cos_lat[p], out0, out1);
+      }
 }
 
 // Adds the R parts' sums of each (column, point) in part order and stores
@@ -342,42 +408,64 @@ extern "C" hipError_t sht_launch_sample_pack(const sht::SamplePackArgs* a, hipSt
   return hipGetLastError();
 }
 
-// Field tile per precision and kind: fp64 accumulators take twice the
-// registers of fp32 ones, gradients twice those of values.
-// Fields per block: eight in every mode (the FP64 gradient and wind kernels
-// hold 255 VGPRs at eight, two waves per SIMD, and are still 7% faster than
-// at four fields with three)
-int sht_sample_field_tile(int kind, int f32) {
-  (void)kind;
-  (void)f32;
-  return 8;
+namespace {
+
+template <int PT, int CT, int KIND, bool F32>
+hipError_t launch_sample_tile(const sht::SampleArgs& a, hipStream_t s) {
+  const int tiles = a.ldc / 8;
+  const dim3 g((unsigned)((a.npts + 64 * PT - 1) / (64 * PT)), (unsigned)((tiles + CT - 1) / CT),
+               (unsigned)a.cuts.parts);
+  hipLaunchKernelGGL((sht::sample_kernel<PT, CT, KIND, F32>), g, dim3(256), 0, s,
+                     static_cast<const typename sht::SampleAcc<F32>::T*>(a.coef), a.rec, a.diag,
+                     a.sin_lat, a.cos_lat, a.lon, a.cuts, a.T, a.npts, a.ldc, a.nout, a.radius,
+                     a.out0, a.out1, a.partial);
+  return hipGetLastError();
 }
+
+// The tile of a wavefront.  Two point tiles and as many column tiles as the
+// registers of two wavefronts per SIMD hold (five for values, two for the two
+// bases of gradients and winds) feed the most MFMAs per basis value and
+// coefficient; fewer points or columns take smaller tiles, so that the launch
+// still has a wavefront for each of the chip's 1024 SIMDs.
+template <int KIND, bool F32>
+hipError_t launch_sample_kind(const sht::SampleArgs& a, hipStream_t s) {
+  const long long most = KIND == 0 ? 5 : 2, tiles = a.ldc / 8;
+  const long long groups = (tiles + most - 1) / most;
+  const int ct = (int)((tiles + groups - 1) / groups);
+  const long long waves2 = (a.npts + 31) / 32 * groups * a.cuts.parts;
+  const long long waves1 = (a.npts + 15) / 16 * groups * a.cuts.parts;
+  if (waves2 >= 2048 || (waves2 >= 1024 && ct >= 2)) {
+    switch (ct) {
+      case 1: return launch_sample_tile<2, 1, KIND, F32>(a, s);
+      case 2: return launch_sample_tile<2, 2, KIND, F32>(a, s);
+      default:
+        if constexpr (KIND == 0) {
+          if (ct == 3) return launch_sample_tile<2, 3, KIND, F32>(a, s);
+          if (ct == 4) return launch_sample_tile<2, 4, KIND, F32>(a, s);
+          return launch_sample_tile<2, 5, KIND, F32>(a, s);
+        }
+    }
+  }
+  if (waves1 >= 1024 && ct >= 2) {
+    if constexpr (KIND == 0)
+      if (ct > 2) return launch_sample_tile<1, 5, KIND, F32>(a, s);
+    return launch_sample_tile<1, 2, KIND, F32>(a, s);
+  }
+  return launch_sample_tile<1, 1, KIND, F32>(a, s);
+}
+
+}  // namespace
 
 extern "C" hipError_t sht_launch_sample(const sht::SampleArgs* a, hipStream_t s) {
   if (a->npts <= 0 || a->ldc <= 0) return hipSuccess;
-  const int ft = sht_sample_field_tile(a->kind, a->f32);
   const int R = a->cuts.parts;
-  if (a->ldc % ft || R < 1 || R > sht::kSampleMaxParts || (R > 1 && !a->partial))
+  if (a->ldc % 8 || R < 1 || R > sht::kSampleMaxParts || (R > 1 && !a->partial))
     return hipErrorInvalidValue;
-  constexpr int kPointsPerBlock = 256 * sht::kSamplePts;
-  const dim3 g((unsigned)((a->npts + kPointsPerBlock - 1) / kPointsPerBlock),
-               (unsigned)(a->ldc / ft), (unsigned)R),
-      b(256);
-#define SHT_SAMPLE(FT, KIND, F32)                                                             \
-  hipLaunchKernelGGL((sht::sample_kernel<FT, KIND, F32>), g, b, 0, s,                          \
-                     static_cast<const typename sht::SampleAcc<F32>::C*>(a->coef), a->rec,   \
-                     a->diag, a->sin_lat, a->cos_lat, a->lon, a->cuts, a->T, a->npts, a->ldc, \
-                     a->nout, a->radius, a->out0, a->out1, a->partial)
-  if (a->f32) {
-    if (a->kind == 0) SHT_SAMPLE(8, 0, true);
-    else if (a->kind == 1) SHT_SAMPLE(8, 1, true);
-    else SHT_SAMPLE(8, 2, true);
-  } else {
-    if (a->kind == 0) SHT_SAMPLE(8, 0, false);
-    else if (a->kind == 1) SHT_SAMPLE(8, 1, false);
-    else SHT_SAMPLE(8, 2, false);
-  }
-#undef SHT_SAMPLE
+  hipError_t le = hipErrorInvalidValue;
+  if (a->kind == 0) le = a->f32 ? launch_sample_kind<0, true>(*a, s) : launch_sample_kind<0, false>(*a, s);
+  else if (a->kind == 1) le = a->f32 ? launch_sample_kind<1, true>(*a, s) : launch_sample_kind<1, false>(*a, s);
+  else le = a->f32 ? launch_sample_kind<2, true>(*a, s) : launch_sample_kind<2, false>(*a, s);
+  if (le != hipSuccess) return le;
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || R == 1) return e;
   const int stride = a->kind == 2 ? 2 : 1;

@@ -1,0 +1,82 @@
+"""The point sampler where its tiles end: points and fields either side of a
+tile, orders of every remainder of four degrees, one part and several, against
+the FP64 oracle; and a point's bits must not depend on the tile it fell in.
+
+Tolerance: FP64 sums of at most T^2/2 products of a three-term recurrence,
+1e-12 of the largest value; the float32 sampler sums one order's T+1 fp32
+terms, (T+1) 6e-8 at most, 2e-6 with T <= 33.
+"""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from _helpers import hip_transform
+from oracle import sampling as osamp
+from oracle.sht import OracleTransform, red_spectrum
+
+pytestmark = pytest.mark.gpu
+
+TOL = {"float64": 1e-12, "float32": 2e-6}
+
+
+def _points(n):
+    rng = np.random.default_rng(n)
+    return rng.uniform(-89.0, 89.0, n), rng.uniform(0.0, 360.0, n)
+
+
+def _fields(T, count, seed):
+    return red_spectrum(T, (count,), seed=seed).astype(np.complex64)
+
+
+@pytest.mark.parametrize("T,count,points", [(1, 1, 1), (2, 3, 15), (3, 8, 16), (6, 9, 17),
+                                            (21, 5, 33), (31, 16, 65), (32, 17, 130), (33, 41, 97)])
+@pytest.mark.parametrize("precision", list(TOL))
+def test_tiles_match_the_oracle(T, count, points, precision):
+    from arwen_spectral import sampling
+
+    o = OracleTransform.create(T)
+    t = hip_transform(o, "float32")
+    lat, lon = _points(points)
+    c, d = _fields(T, count, 1), _fields(T, count, 2)
+    c128, d128 = c.astype(np.complex128), d.astype(np.complex128)
+
+    def close(got, want):
+        assert np.max(np.abs(got - want)) < TOL[precision] * np.max(np.abs(want))
+
+    close(sampling.sample_scalar(t, c, lat, lon, precision=precision),
+          osamp.sample_scalar(o, c128, lat, lon))
+    for got, want in zip(sampling.sample_gradient(t, c, lat, lon, precision=precision),
+                         osamp.sample_gradient(o, c128, lat, lon)):
+        close(got, want)
+    # psi and chi are formed in fp32 from vorticity and divergence (one
+    # rounding of each coefficient) before the FP64 sums
+    for got, want in zip(sampling.sample_wind(t, c, d, lat, lon, precision=precision),
+                         osamp.sample_wind(o, c128, d128, lat, lon)):
+        assert np.max(np.abs(got - want)) < 2e-6 * np.max(np.abs(want))
+
+
+@pytest.mark.parametrize("kind", ["scalar", "gradient", "wind"])
+@pytest.mark.parametrize("precision", list(TOL))
+def test_a_points_bits_do_not_depend_on_its_tile(kind, precision):
+    from arwen_spectral import sampling
+
+    o = OracleTransform.create(63, dealias_factor=1.0)
+    t = hip_transform(o, "float32")
+    lat, lon = _points(9000)
+    c = _fields(63, 40, 3)
+    fn = {"scalar": sampling.sample_scalar, "gradient": sampling.sample_gradient,
+          "wind": sampling.sample_wind}[kind]
+
+    def call(fields, s):
+        args = (fields, fields[::-1].copy()) if kind == "wind" else (fields,)
+        out = fn(t, *args, lat[s], lon[s], precision=precision)
+        return out if isinstance(out, tuple) else (out,)
+
+    whole = call(c, slice(None))
+    for s in (slice(0, 1), slice(5, 40), slice(100, 1700)):
+        for w, got in zip(whole, call(c, s)):
+            assert np.array_equal(w[:, s], got)
+    if kind != "wind":  # fewer fields: other column tiles
+        for w, got in zip(whole, call(c[3:20].copy(), slice(None))):
+            assert np.array_equal(w[3:20], got)
