@@ -465,6 +465,9 @@ struct arwen_sht_batch {
   std::vector<sht::WaistFoldArgs> waist_folds;      // analysis from a reference waist
   std::vector<sht::LowSynArgs> low_syns;            // vector jobs' FP64 low orders
   std::vector<sht::LowAnaArgs> low_anas;
+  bool single = false;  // one operation of a plan's cache: may take the few-column kernels
+  std::vector<std::pair<sht::SmallSynArgs, int>> small_syns;  // and the jobs of each
+  std::vector<sht::SmallAnaArgs> small_anas;
   std::vector<HostGroup> groups[2];  // GEMM work groups per direction (0 SYN, 1 ANA)
   GemmLists lists[2];
   arwen_sht_gemm_config config{{32, 32}, {0, 0}, 1};
@@ -709,6 +712,28 @@ void add_ana_group(std::vector<HostGroup>& b, const arwen_sht_plan* P, int mb, i
   b.push_back(g);
 }
 
+// Whether a single operation takes the few-column kernels (small_*_kernel):
+// the scalar operations, while their time stays below the grouped path's.
+// That grows with the fields and, through the gathers and the k chain of one
+// wavefront, with the square (synthesis) or the cube (analysis, whose results
+// leave in 8-byte pieces) of K = ceil((T+1)/64) k-chunks.  GPU time of a call
+// either side of the lines, grouped -> few-column, us (float32; bf16x6 alike):
+//   synthesis, fields K^2 <= 72:   T127 16 fields 17.1 -> 13.1, T255 4 21.8 ->
+//     17.7, T383 2 31.8 -> 28.9
+//   two contractions, <= 36:       T255 2 fields 38.0 -> 36.6, 4 39.1 -> 39.6;
+//     T383 1 58.5 -> 54.7
+//   analysis, fields K^3 <= 100:   T95 16 fields 14.5 -> 12.8, 32 15.8 -> 16.6;
+//     T191 2 15.7 -> 13.8, 4 16.2 -> 17.1; T255 1 18.3 -> 17.2, 2 18.6 -> 20.2
+bool small_job(const arwen_sht_batch* B, const arwen_sht_job& J) {
+  if (!B->single || J.op == ARWEN_SHT_OP_UV_FROM_VORDIV || J.op == ARWEN_SHT_OP_VORDIV_FROM_UV ||
+      J.op == ARWEN_SHT_OP_VORDIV_FROM_WAIST || J.op == ARWEN_SHT_OP_DIVERGENCE_FROM_WAIST)
+    return false;
+  const long long K = (J.plan->T + 64) / 64, n = J.count;
+  if (!is_synthesis(J.op)) return n * K * K * K <= 100;
+  const bool two = J.op == ARWEN_SHT_OP_GRADIENT || J.op == ARWEN_SHT_OP_SYNTHESIS_GRADIENT;
+  return n * K * K <= (two ? 36 : 72);
+}
+
 // One job's share of a batch.  prepare: allocate its workspaces, add its
 // grouped-GEMM work groups and its algorithmic work (once, at batch
 // creation); always: append its launch arguments, which carry the caller's
@@ -737,7 +762,8 @@ void setup_job(arwen_sht_batch* B, JobState* js, bool prepare) {
     // ---- pack ----
     const int ncol = vec ? 4 : 2;
     js->ncols = ncol * n;
-    if (prepare) js->packed_a.alloc((size_t)js->ncols * P->ldp * 4);
+    const bool small = small_job(B, J);
+    if (prepare && !small) js->packed_a.alloc((size_t)js->ncols * P->ldp * 4);
     if (prepare) js->waist_a.alloc((size_t)js->ncols * P->ldw * 4);
     const bool grad = J.op == ARWEN_SHT_OP_GRADIENT;
     if ((grad || sgrad) && prepare) js->waist_b.alloc((size_t)js->ncols * P->ldw * 4);
@@ -766,7 +792,31 @@ void setup_job(arwen_sht_batch* B, JobState* js, bool prepare) {
     pa.job.off00 = static_cast<const float2*>(J.coeff_offset);
     pa.job.m0 = low ? P->m0 : 0;
     pa.job.mdp = recp ? sht::kMT : 0;
-    B->packs.push_back(pa);
+    if (!small) {
+      B->packs.push_back(pa);
+    } else {
+      // table kind and output of each contraction (dP/dphi flips the parity)
+      const bool merid = J.op == ARWEN_SHT_OP_MERIDIONAL_DERIVATIVE ||
+                         J.op == ARWEN_SHT_OP_MERIDIONAL_TO_WAIST;
+      const int kinds[2] = {merid ? kD : grad ? kPm : kP, kD};
+      const int njobs = grad || sgrad ? 2 : 1;
+      sht::SmallSynArgs sa{};
+      sa.in = pa.job.in0;
+      sa.off00 = pa.job.off00;
+      sa.koff = pa.koff;
+      for (int k = 0; k < njobs; ++k) {
+        sa.table[k] = P->table(kinds[k], true, &sa.piece);
+        sa.waist[k] = (k == 0 ? js->waist_a : js->waist_b).as<float>();
+        sa.pflip[k] = kinds[k] == kD ? 1 : 0;
+      }
+      sa.T = T;
+      sa.JHP = P->JHP;
+      sa.ldw = P->ldw;
+      sa.nfields = n;
+      sa.mode = pa.job.mode;
+      sa.radius = pa.job.radius;
+      B->small_syns.emplace_back(sa, njobs);
+    }
     // ---- FP64 low orders of u, v (orders m < m0) ----
     if (low) {
       if (prepare) js->low.alloc((size_t)n * 2 * P->m0 * 2 * P->JHP * sizeof(double2));
@@ -785,7 +835,7 @@ void setup_job(arwen_sht_batch* B, JobState* js, bool prepare) {
     }
     // ---- grouped GEMM: one group per (m-tile, output parity) ----
     const DataRef pk{js->packed_a.as<char>()};
-    for (int mb = low ? P->m0 / sht::kMT : 0; prepare && mb < P->MB; ++mb)
+    for (int mb = low ? P->m0 / sht::kMT : 0; prepare && !small && mb < P->MB; ++mb)
       for (int q = 0; q < 2; ++q) {
         if (low || (recp && mb >= 1)) {
           // recurrence form: a cos(phi) [u, v] = P [U, V] (pack_vector_rec_kernel)
@@ -901,7 +951,8 @@ void setup_job(arwen_sht_batch* B, JobState* js, bool prepare) {
     js->ncols = ncol * n;
     if (prepare) js->waist_a.alloc((size_t)js->ncols * P->ldw * 4);
     if (prepare && divw) js->waist_b.alloc((size_t)js->ncols * P->ldw * 4);
-    if (prepare) js->packed_out.alloc((size_t)js->ncols * P->ldp * 4);
+    const bool small = small_job(B, J);
+    if (prepare && !small) js->packed_out.alloc((size_t)js->ncols * P->ldp * 4);
     if (from_waist(J.op)) {
       // a reference waist (*lead, nlat, T+1), already divided by nlon
       sht::WaistFoldArgs wf{};
@@ -995,7 +1046,7 @@ void setup_job(arwen_sht_batch* B, JobState* js, bool prepare) {
       if (prepare) B->fft_bytes += (vec ? 2.0 : 1.0) * n * fftb;
     }
     const DataRef wst{js->waist_a.as<char>()};
-    for (int mb = low ? P->m0 / sht::kMT : 0; prepare && mb < P->MB; ++mb)
+    for (int mb = low ? P->m0 / sht::kMT : 0; prepare && !small && mb < P->MB; ++mb)
       for (int q = 0; q < 2; ++q) {
         if (low || (recp && mb >= 1)) {
           // recurrence form: [iB, iA] = P^T [iV, iU] / cos(phi); unpack_vector_rec_kernel
@@ -1021,6 +1072,20 @@ void setup_job(arwen_sht_batch* B, JobState* js, bool prepare) {
       B->legendre_flops += 2.0 * n * pcf + 2.0 * n * pcf_t0;
     } else if (prepare) {
       B->legendre_flops += (vec ? 4.0 : divw ? 2.0 : 1.0) * n * pcf;
+    }
+    if (small) {
+      sht::SmallAnaArgs sa{};
+      sa.waist = js->waist_a.as<float>();
+      sa.table = P->table(kP, false, &sa.piece);
+      sa.koff = P->d_koff.as<int>();
+      sa.out = static_cast<float2*>(J.out0);
+      sa.off00 = static_cast<const float2*>(J.coeff_offset);
+      sa.T = T;
+      sa.JHP = P->JHP;
+      sa.ldw = P->ldw;
+      sa.nfields = n;
+      B->small_anas.push_back(sa);
+      return;
     }
     sht::UnpackArgs ua{};
     ua.koff = P->d_koff.as<int>();
@@ -1051,6 +1116,8 @@ void bind_jobs(arwen_sht_batch* B) {
   B->waist_folds.clear();
   B->low_syns.clear();
   B->low_anas.clear();
+  B->small_syns.clear();
+  B->small_anas.clear();
   for (auto& js : B->jobs) setup_job(B, js.get(), false);
 }
 
@@ -1156,6 +1223,9 @@ void run_batch(arwen_sht_batch* B, hipStream_t s, hipEvent_t* ev = nullptr) {
   for (auto& a : B->packs) hip_check(sht_launch_pack(&a, s), "pack launch");
   mark(1);
   hip_check(launch_gemm(B, 0, s), "synthesis GEMM launch");
+  for (auto& a : B->small_syns)
+    hip_check(sht_launch_small_synthesis(&a.first, B->precision, a.second, s),
+              "few-column synthesis launch");
   mark(2);
   for (auto& a : B->low_syns) hip_check(sht_launch_low_synthesis(&a, s), "low-order synthesis launch");
   mark(3);
@@ -1166,6 +1236,8 @@ void run_batch(arwen_sht_batch* B, hipStream_t s, hipEvent_t* ev = nullptr) {
   for (auto& a : B->waist_folds) hip_check(sht_launch_waist_fold(&a, s), "waist fold launch");
   mark(5);
   hip_check(launch_gemm(B, 1, s), "analysis GEMM launch");
+  for (auto& a : B->small_anas)
+    hip_check(sht_launch_small_analysis(&a, B->precision, s), "few-column analysis launch");
   mark(6);
   for (auto& a : B->low_anas) hip_check(sht_launch_low_analysis(&a, s), "low-order analysis launch");
   mark(7);
@@ -1234,6 +1306,7 @@ int single_job(arwen_sht_plan* P, const arwen_sht_job& job, void* stream) {
     J.plan = P;
     if (!B) {
       auto nb = std::make_unique<arwen_sht_batch>();
+      nb->single = true;
       plan_batch_on(nb.get(), &J, 1, static_cast<hipStream_t>(stream));
       B = nb.release();
       P->cache.push_front({key, B});

@@ -513,6 +513,217 @@ __global__ void __launch_bounds__(256, BN == 32 ? 3 : 2) legendre_gemm_kernel(Ge
   }
 }
 
+// ---------------------------------------------------------------------------
+// Few columns: contraction straight from and to the boundary layout
+// ---------------------------------------------------------------------------
+// A single operation on a few fields is bound by latency: of its launches
+// (pack, grouped GEMM, FFTs) the GEMM walks up to 24 dependent steps in its
+// longest panels (four orders after each other) behind a chain of list and
+// descriptor loads, and pack and unpack are a launch each.  Here a wavefront
+// takes one order alone (a block the four orders of an m-tile, so that the
+// waist is written in 16-byte pieces), addresses follow from the indices, and
+// the data operand is gathered from, and the result scattered to, the
+// (n, m) arrays, so pack and unpack disappear.  Every output runs the same
+// MFMAs in the same order as the grouped GEMM's (two accumulators in the
+// split modes), so the bits are the same.
+// No LDS in the loop: lane (li, kg) gathers its own B fragment, 8 values of
+// column li, once for all of the wavefront's RT row tiles; the next k-chunk's
+// gathers and table fragments are in flight behind the current one's MFMAs.
+// Measured (GPU time of a whole call): one field's synthesis at T63 13.3 ->
+// 6.9 us, T127 15.6 -> 8.4, T255 21.0 -> 13.4; its analysis 11.4 -> 7.2,
+// 13.6 -> 8.8, 18.3 -> 17.2.
+
+// B fragment of 32 k for this lane from its values x[j], in the layout of
+// mfma_step (fp32: x[4 h + s] at k = 16 h + 4 kg + s; bf16: x[j] at
+// k = 8 kg + j).
+template <int MODE>
+__device__ __forceinline__ void small_fragment(const float (&x)[8], u32x4 (&b)[3]) {
+  if constexpr (MODE == kFP32) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      b[h] = u32x4{__float_as_uint(x[4 * h]), __float_as_uint(x[4 * h + 1]),
+                   __float_as_uint(x[4 * h + 2]), __float_as_uint(x[4 * h + 3])};
+  } else {
+    constexpr int NP = MODE == kBF16X6 ? 3 : 2;
+    u32x2 lo[3], hi[3];
+    const float a[4] = {x[0], x[1], x[2], x[3]}, c[4] = {x[4], x[5], x[6], x[7]};
+    split4(a, NP, lo);
+    split4(c, NP, hi);
+#pragma unroll
+    for (int pc = 0; pc < NP; ++pc) b[pc] = u32x4{lo[pc][0], lo[pc][1], hi[pc][0], hi[pc][1]};
+  }
+}
+// k within its 32-chunk of value j of lane group kg
+template <int MODE>
+__device__ __forceinline__ int small_k(int j, int kg) {
+  return MODE == kFP32 ? 16 * (j >> 2) + 4 * kg + (j & 3) : 8 * kg + j;
+}
+// A fragments of one 16-row tile and k-chunk: `tile` = row 0 of the tile in
+// the tiled table (bytes), rows of 32 k.
+template <int MODE>
+__device__ __forceinline__ void small_table(const char* tile, long long piece_bytes, int li, int kg,
+                                            u32x4 (&a)[3]) {
+  if constexpr (MODE == kFP32) {
+    a[0] = *reinterpret_cast<const u32x4*>(tile + li * 128 + kg * 16);
+    a[1] = *reinterpret_cast<const u32x4*>(tile + li * 128 + (kg + 4) * 16);
+  } else {
+#pragma unroll
+    for (int pc = 0; pc < (MODE == kBF16X6 ? 3 : 2); ++pc)
+      a[pc] = *reinterpret_cast<const u32x4*>(tile + pc * piece_bytes + li * 64 + kg * 16);
+  }
+}
+
+// The k loop of both directions: nch chunks; load(k) gives this lane's stored
+// data value at k, shape(k, v) the operand value from it (apart, so that a
+// chunk's loads are all in flight before the first is used), table(ch, rt)
+// the first row of a tile.
+template <int MODE, int RT, class Load, class Shape, class Table>
+__device__ __forceinline__ void small_contract(f32x4 (&acc)[RT], int nch, int kg, int li,
+                                               long long piece_bytes, Load&& load, Shape&& shape,
+                                               Table&& table) {
+  f32x4 acc2[RT];
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) acc[rt] = acc2[rt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float x[8];
+  u32x4 a[RT][3];
+  auto fetch = [&](int ch) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) x[j] = load(32 * ch + small_k<MODE>(j, kg));
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) small_table<MODE>(table(ch, rt), piece_bytes, li, kg, a[rt]);
+  };
+  if (nch > 0) fetch(0);
+  for (int ch = 0; ch < nch; ++ch) {
+    u32x4 b[3], c[RT][3];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) x[j] = shape(32 * ch + small_k<MODE>(j, kg), x[j]);
+    small_fragment<MODE>(x, b);
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+      for (int pc = 0; pc < 3; ++pc) c[rt][pc] = a[rt][pc];
+    if (ch + 1 < nch) fetch(ch + 1);
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+      if constexpr (MODE == kFP32) mfma_step<MODE>(acc[rt], acc[rt], c[rt], b);
+      else mfma_step<MODE>(acc[rt], acc2[rt], c[rt], b);
+    }
+  }
+  if constexpr (MODE != kFP32)
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) acc[rt] = acc[rt] + acc2[rt];
+}
+
+// Synthesis: grid (m-tile, output parity, row group) x column group (8
+// fields) x job.
+template <int MODE, int RT>
+__global__ void __launch_bounds__(256) small_synthesis_kernel(SmallSynArgs a) {
+  constexpr int ESZ = MODE == kFP32 ? 4 : 2;
+  __shared__ float sOut[16 * 17 * 4];  // [column][row, padded][order]
+  const int lane = threadIdx.x & 63, z = threadIdx.x >> 6;
+  const int li = lane & 15, kg = lane >> 4;
+  const int rg = (int)blockIdx.x % a.rgroups, q = (int)blockIdx.x / a.rgroups % 2;
+  const int mb = (int)blockIdx.x / a.rgroups / 2;
+  const int job = blockIdx.z, T1 = a.T + 1;
+  const int m = mb * kMT + z, p = q ^ a.pflip[job];
+  const int kc = m <= a.T ? (a.T - m - p) / 2 + (a.T >= m + p ? 1 : 0) : 0;  // degrees m + p + 2 k
+  const int f = (int)blockIdx.y * 8 + (li >> 1), part = li & 1;
+  const bool live = f < a.nfields;
+  const float* in = reinterpret_cast<const float*>(a.in + (size_t)min(f, a.nfields - 1) * T1 * T1);
+  const int comp = a.mode == kIM ? part ^ 1 : part;
+  const double a2 = (double)a.radius * (double)a.radius;
+  auto load = [&](int k) {
+    return in[2 * ((size_t)min(m + p + 2 * k, a.T) * T1 + m) + comp];
+  };
+  const float im = a.mode == kIM ? (part ? (float)m : -(float)m) : 1.f;  // x * 1 = x exactly
+  const bool inv = a.mode == kInvLap;
+  const float2 off = a.off00 && m == 0 ? a.off00[min(f, a.nfields - 1)] : make_float2(0.f, 0.f);
+  const float add = part ? off.y : off.x;
+  auto shape = [&](int k, float v) {
+    const int n = m + p + 2 * k;
+    v *= im;
+    if (inv) {  // the spectral inverse Laplacian's own arithmetic
+      const float eig = (float)(-((double)n * ((double)n + 1.0)) / a2);
+      v = n >= 1 && !(m == 0 && part) ? v / eig : 0.f;
+    }
+    if (a.off00 && n == 0) v += add;
+    return live && k < kc ? v : 0.f;
+  };
+  const char* tab = static_cast<const char*>(a.table[job]) +
+                    (size_t)a.koff[2 * min(m, a.T) + p] * a.JHP * ESZ;
+  const int r0 = rg * RT * 16;
+  f32x4 acc[RT];
+  small_contract<MODE, RT>(acc, (kc + 31) / 32, kg, li, a.piece * ESZ, load, shape, [&](int ch, int rt) {
+    return tab + ((size_t)ch * a.JHP + min(r0 + 16 * rt, a.JHP - 16)) * 32 * ESZ;
+  });
+  const int col = threadIdx.x >> 4, row = threadIdx.x & 15, c = (int)blockIdx.y * 16 + col;
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) sOut[(li * 17 + 4 * kg + r) * 4 + z] = acc[rt][r];
+    __syncthreads();
+    if (c < 2 * a.nfields && r0 + 16 * rt < a.JHP)
+      *reinterpret_cast<f32x4*>(a.waist[job] + (size_t)c * a.ldw +
+                                ((size_t)(mb * 2 + q) * a.JHP + r0 + 16 * rt + row) * kMT) =
+          *reinterpret_cast<const f32x4*>(&sOut[(col * 17 + row) * 4]);
+    __syncthreads();
+  }
+}
+
+// Analysis: grid (m-tile, parity, row group of degrees) x column group.  The
+// block of row group 0 also writes the zeros above the triangle of its orders
+// and parity.
+template <int MODE, int RT>
+__global__ void __launch_bounds__(256) small_analysis_kernel(SmallAnaArgs a) {
+  constexpr int ESZ = MODE == kFP32 ? 4 : 2;
+  const int lane = threadIdx.x & 63, z = threadIdx.x >> 6;
+  const int li = lane & 15, kg = lane >> 4;
+  const int rg = (int)blockIdx.x % a.rgroups, q = (int)blockIdx.x / a.rgroups % 2;
+  const int mb = (int)blockIdx.x / a.rgroups / 2;
+  const int T1 = a.T + 1;
+  const int m = mb * kMT + z;
+  const size_t plane = (size_t)T1 * T1;
+  const int f = (int)blockIdx.y * 8 + (li >> 1), part = li & 1;
+  if (rg == 0) {  // degrees n < 4 mb + zz of the orders 4 mb + zz, (n - m) mod 2 = q
+    const int nmax = min(mb * kMT + kMT - 1, T1);
+    for (int e = threadIdx.x; e < nmax * 32; e += 256) {
+      const int zz = e & 3, ff = (int)blockIdx.y * 8 + ((e >> 2) & 7), n = e >> 5;
+      const int mm = mb * kMT + zz;
+      if (n < mm && mm <= a.T && ((mm - n) & 1) == q && ff < a.nfields)
+        a.out[(size_t)ff * plane + (size_t)n * T1 + mm] = make_float2(0.f, 0.f);
+    }
+  }
+  const int kq = m <= a.T ? (a.T - m - q) / 2 + (a.T >= m + q ? 1 : 0) : 0;  // rows m + q + 2 r
+  const int r0 = rg * RT * 16;
+  if (r0 >= kq) return;  // wave-uniform, and no barrier below
+  const int KP = a.koff[2 * m + q + 1] - a.koff[2 * m + q];
+  const char* tab = static_cast<const char*>(a.table) + (size_t)a.koff[2 * m + q] * a.JHP * ESZ;
+  const float* W = a.waist + (size_t)min(2 * f + part, 2 * a.nfields - 1) * a.ldw +
+                   (size_t)(mb * 2 + q) * a.JHP * kMT + z;
+  f32x4 acc[RT];
+  small_contract<MODE, RT>(
+      acc, a.JHP / 32, kg, li, a.piece * ESZ, [&](int k) { return W[(size_t)k * kMT]; },
+      [](int, float v) { return v; },
+      [&](int ch, int rt) {
+        return tab + ((size_t)ch * KP + min(r0 + 16 * rt, KP - 16)) * 32 * ESZ;
+      });
+  if (f >= a.nfields) return;
+  float* out = reinterpret_cast<float*>(a.out + (size_t)f * plane) + part;
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = r0 + 16 * rt + 4 * kg + r, n = m + q + 2 * row;
+      if (row >= kq) continue;
+      float v = m == 0 && part ? 0.f : acc[rt][r];
+      if (a.off00 && n == 0) {  // m = 0 as well
+        const float2 d = a.off00[f];
+        v += part ? d.y : d.x;
+      }
+      out[2 * ((size_t)n * T1 + m)] = v;
+    }
+}
+
 }  // namespace sht
 
 namespace {
@@ -559,4 +770,63 @@ extern "C" hipError_t sht_launch_legendre_gemm(const sht::GemmLaunch* L, hipStre
   const dim3 g(L->grid);
   return L->dir == 0 ? launch_dir<0>(L->mode, w, L->bn, L->acc2, g, s)
                      : launch_dir<1>(L->mode, w, L->bn, L->acc2, g, s);
+}
+
+namespace {
+
+// Row tiles per wavefront: as many as still leave the chip two blocks per CU
+// (more tiles per gathered data fragment), at most 4.
+int small_row_tiles(int blocks_of_one, int tiles) {
+  int rt = 4;
+  while (rt > 1 && (rt > tiles || blocks_of_one / rt < 512)) rt /= 2;
+  return rt;
+}
+
+template <int MODE>
+void launch_small_syn(const sht::SmallSynArgs& a, int rt, dim3 g, hipStream_t s) {
+  if (rt == 4) hipLaunchKernelGGL((sht::small_synthesis_kernel<MODE, 4>), g, dim3(256), 0, s, a);
+  else if (rt == 2) hipLaunchKernelGGL((sht::small_synthesis_kernel<MODE, 2>), g, dim3(256), 0, s, a);
+  else hipLaunchKernelGGL((sht::small_synthesis_kernel<MODE, 1>), g, dim3(256), 0, s, a);
+}
+template <int MODE>
+void launch_small_ana(const sht::SmallAnaArgs& a, int rt, dim3 g, hipStream_t s) {
+  if (rt == 4) hipLaunchKernelGGL((sht::small_analysis_kernel<MODE, 4>), g, dim3(256), 0, s, a);
+  else if (rt == 2) hipLaunchKernelGGL((sht::small_analysis_kernel<MODE, 2>), g, dim3(256), 0, s, a);
+  else hipLaunchKernelGGL((sht::small_analysis_kernel<MODE, 1>), g, dim3(256), 0, s, a);
+}
+
+}  // namespace
+
+extern "C" hipError_t sht_launch_small_synthesis(const sht::SmallSynArgs* a, int mode, int njobs,
+                                                 hipStream_t s) {
+  if (a->nfields <= 0) return hipSuccess;
+  const int MB = (a->T + sht::kMT) / sht::kMT, tiles = a->JHP / 16, cg = (a->nfields + 7) / 8;
+  const int rt = small_row_tiles(MB * 2 * tiles * cg * njobs, tiles);
+  sht::SmallSynArgs b = *a;
+  b.rgroups = (tiles + rt - 1) / rt;
+  const dim3 g((unsigned)(MB * 2 * b.rgroups), (unsigned)cg, (unsigned)njobs);
+  switch (mode) {
+    case sht::kFP32: launch_small_syn<sht::kFP32>(b, rt, g, s); break;
+    case sht::kBF16X3: launch_small_syn<sht::kBF16X3>(b, rt, g, s); break;
+    case sht::kBF16X6: launch_small_syn<sht::kBF16X6>(b, rt, g, s); break;
+    default: return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
+}
+
+extern "C" hipError_t sht_launch_small_analysis(const sht::SmallAnaArgs* a, int mode,
+                                                hipStream_t s) {
+  if (a->nfields <= 0) return hipSuccess;
+  const int MB = (a->T + sht::kMT) / sht::kMT, tiles = (a->T / 2 + 16) / 16, cg = (a->nfields + 7) / 8;
+  const int rt = small_row_tiles(MB * tiles * cg, tiles);  // half of the blocks lie past the triangle
+  sht::SmallAnaArgs b = *a;
+  b.rgroups = (tiles + rt - 1) / rt;
+  const dim3 g((unsigned)(MB * 2 * b.rgroups), (unsigned)cg);
+  switch (mode) {
+    case sht::kFP32: launch_small_ana<sht::kFP32>(b, rt, g, s); break;
+    case sht::kBF16X3: launch_small_ana<sht::kBF16X3>(b, rt, g, s); break;
+    case sht::kBF16X6: launch_small_ana<sht::kBF16X6>(b, rt, g, s); break;
+    default: return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
 }

@@ -288,6 +288,32 @@ struct PackArgs {
   PackJob job;
 };
 
+// Contractions of a few columns straight from / to the boundary layout
+// (sht_gemm.hip, small_*_kernel).
+struct SmallSynArgs {
+  const float2* in;           // (nfields, T+1, T+1)
+  const float2* off00;        // kPlain: per field, added to its (0, 0) coefficient (or NULL)
+  const int* koff;
+  const void* table[2];       // per job (grid z): synthesis-layout table,
+  float* waist[2];            // output waist,
+  int pflip[2];               // data parity = output parity ^ pflip
+  long long piece;            // table piece stride, elements
+  int T, JHP, ldw, nfields;
+  int mode;                   // kPlain, kIM or kInvLap
+  int rgroups;                // row groups per (m-tile, parity), set by the launcher
+  float radius;
+};
+struct SmallAnaArgs {
+  const float* waist;
+  const void* table;          // analysis layout
+  const int* koff;
+  float2* out;                // (nfields, T+1, T+1)
+  const float2* off00;        // per field, added to its (0, 0) output (or NULL)
+  long long piece;
+  int T, JHP, ldw, nfields;
+  int rgroups;
+};
+
 struct UnpackJob {
   const float* in;
   float2* out0;               // [f][n][m] (vorticity for vector jobs)
@@ -323,6 +349,9 @@ hipError_t sht_fft_allow_lds(size_t bytes);
 int sht_fft_wave_L(int N);                       // 0: no wave-resident path for N
 size_t sht_fft_wave_lds_bytes(int N, int vector);
 hipError_t sht_launch_legendre_gemm(const sht::GemmLaunch* launch, hipStream_t s);
+hipError_t sht_launch_small_synthesis(const sht::SmallSynArgs* a, int mode, int njobs,
+                                      hipStream_t s);
+hipError_t sht_launch_small_analysis(const sht::SmallAnaArgs* a, int mode, hipStream_t s);
 hipError_t sht_launch_waist_from_rows(const sht::WaistRowsArgs* a, hipStream_t s);
 hipError_t sht_launch_rows_from_waist(const sht::WaistRowsArgs* a, hipStream_t s);
 hipError_t sht_launch_waist_fold(const sht::WaistFoldArgs* a, hipStream_t s);

@@ -1,0 +1,57 @@
+"""Single operations on a few fields (contracted straight from and to the
+boundary layout) against the same operation as a batch job (the grouped GEMM):
+equal bits, either side of the field counts where the path changes, at the
+edges of its tiles: orders that do not fill an m-tile, one and several
+k-chunks, an odd latitude count, 8 and 9 fields (column groups).  The grouped
+path itself is held to the FP64 oracle elsewhere.
+"""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _red(torch, T, count, seed):
+    g = torch.Generator(device="cuda")
+    g.manual_seed(seed)
+    x = torch.view_as_complex(torch.randn(count, T + 1, T + 1, 2, device="cuda", generator=g))
+    return x.contiguous()  # above the triangle and Im(m = 0) as they come
+
+
+@pytest.mark.parametrize("precision", ["float32", "bf16x6", "bf16x3"])
+@pytest.mark.parametrize("T,nlat,nlon,counts", [
+    (1, 2, 4, (1,)), (4, 7, 16, (1, 9)), (21, 33, 66, (8, 72, 73)), (63, 64, 128, (1, 9, 36, 37)),
+    (64, 65, 192, (2, 9, 13)), (127, 128, 256, (1, 12, 18, 19)), (130, 140, 320, (3, 4, 8, 9)),
+    (255, 256, 512, (1, 2, 4, 5)), (383, 384, 768, (1, 2, 3))])
+def test_few_fields_have_the_grouped_bits(T, nlat, nlon, counts, precision):
+    import torch
+
+    from arwen_spectral import SphericalHarmonicTransform, TransformBatch
+
+    t = SphericalHarmonicTransform.create(T, nlat=nlat, nlon=nlon, dealias_factor=1.0,
+                                          precision=precision)
+    for n in counts:
+        c = _red(torch, T, n, T + n)
+        f = torch.randn(n, nlat, nlon, device="cuda")
+        goff = torch.linspace(-1.0, 2.0, n, device="cuda")
+        coff = torch.complex(goff, torch.zeros_like(goff)) + 0.5
+        grids = [torch.empty(n, nlat, nlon, device="cuda") for _ in range(9)]
+        specs = [torch.empty_like(c) for _ in range(2)]
+        TransformBatch([
+            ("inverse", t, c, grids[0]), ("inverse", t, c, grids[1], {"coeff_offset": coff}),
+            ("zonal", t, c, grids[2]), ("meridional", t, c, grids[3]),
+            ("gradient", t, c, (grids[4], grids[5])),
+            ("inverse_gradient", t, c, tuple(grids[6:9])),
+            ("forward", t, f, specs[0]),
+            ("forward", t, f, specs[1], {"grid_offset": goff, "coeff_offset": coff})]).run()
+        got = [t.inverse(c), t.inverse_about(c, coff), t.inverse_zonal_derivative(c),
+               t.inverse_meridional_derivative(c), *t.gradient(c), *t.inverse_with_gradient(c),
+               t.forward(f), t.forward_about(f, goff, coff)]
+        for k, (a, b) in enumerate(zip(got, grids + specs)):
+            assert torch.equal(a, b), f"T{T} {n} fields, result {k}"
+        # the waist's head and tail take the same contraction
+        w = t.contract_to_waist(c)
+        assert np.isfinite(w.values.abs().sum().item())
+        assert (t.waist_to_grid(w) - got[0]).abs().max() <= 2e-6 * got[0].abs().max()
