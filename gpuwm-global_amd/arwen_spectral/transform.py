@@ -208,17 +208,17 @@ class SphericalHarmonicTransform:
 
     @staticmethod
     def _count(t) -> int:
-        return int(np.prod(t.shape[:-2], dtype=np.int64)) if t.dim() > 2 else 1
+        return math.prod(t.shape[:-2])  # 1 for a single plane
 
     def _empty_grid(self, lead):
         torch = self.backend.xp
         return torch.empty((*lead, *self.grid.shape), dtype=self.backend.float_dtype,
-                           device=self.backend.device())
+                           device=torch.cuda.current_device())
 
     def _empty_spectral(self, lead):
         torch = self.backend.xp
         return torch.empty((*lead, *self.spectral_shape), dtype=self.backend.complex_dtype,
-                           device=self.backend.device())
+                           device=torch.cuda.current_device())
 
     # ---- transforms -----------------------------------------------------
     def forward(self, field):
@@ -350,7 +350,7 @@ class SphericalHarmonicTransform:
                            dtype=self.backend.complex_dtype, device=self.backend.device())
 
     def _waist_from_rows(self, rows, values, row0: int, nrows: int) -> None:
-        nlead = int(np.prod(rows.shape[:-2], dtype=np.int64))
+        nlead = math.prod(rows.shape[:-2])
         _native.check(self._lib.arwen_sht_waist_from_rows(
             self._plan, _vp(rows), _vp(values), nlead, int(nrows), int(row0),
             self.backend.stream()))
@@ -420,7 +420,7 @@ class SphericalHarmonicTransform:
         torch = self.backend.xp
         out = torch.empty((*waist.lead, r1 - r0, self.grid.nlon),
                           dtype=self.backend.float_dtype, device=self.backend.device())
-        nlead = int(np.prod(waist.lead, dtype=np.int64))
+        nlead = math.prod(waist.lead)
         _native.check(self._lib.arwen_sht_rows_from_waist(
             self._plan, _vp(values), _vp(out), nlead, r1 - r0, r0, self.backend.stream()))
         return out
