@@ -502,6 +502,40 @@ bool from_waist(int op) {
 
 constexpr int kXcds = 8;  // MI355X: 8 XCDs x 32 CUs
 
+// Column tile of a new batch's direction: 64 columns where the launch is bound
+// by table reads and has enough of the larger tiles, else 32.  A tile reads
+// its table fragments through L1 once for its columns, so 64 halve that
+// traffic; they cost residency (two blocks per CU, not three) and padding.
+// Measured (us, 32 against 64 columns, synthesis / analysis):
+//   bf16x6  T383 160 columns 76.2/80.6 : 69.4/76.2, 256 columns 122/121 : 96/101
+//           T255 128 columns 25.2/28.6 : 21.7/25.9, 160 columns 31.0/35.0 : 30.7/35.0
+//           T383 80 columns (128 padded) 48.3/51.1 : 48.3/54.8
+//           T127 320 columns 18.2/17.5 : 20.1/19.5
+//   fp32    T383 256 columns 118/126 : 109/121, 128 columns 63.6/71.5 : 61.4/75.7,
+//           160 columns 77.7/84.8 : 81.5/94.8
+// so: tables from half of the eight 4 MB L2s up; in the split modes at most a
+// quarter of padding and as many tiles as run together (512), in FP32, whose
+// MFMA time weighs more, hardly any padding and four times as many tiles.
+int default_cols(const std::vector<HostGroup>& groups, int precision) {
+  const bool split = precision != ARWEN_SHT_FP32;
+  long long tiles = 0, used = 0, wide = 0, table = 0;
+  const int pieces = split ? (precision == ARWEN_SHT_BF16X6 ? 3 : 2) : 1;
+  for (const HostGroup& g : groups) {
+    int rows = 0;
+    for (int z = 0; z < g.mcount; ++z) rows = std::max(rows, g.R[z]);
+    const long long panels = (rows + sht::kGemmBM - 1) / sht::kGemmBM, nt = (g.N + 63) / 64;
+    tiles += panels * nt;
+    used += panels * g.N;
+    wide += panels * nt * 64;
+    for (int sg = 0; sg < g.nseg; ++sg)
+      for (int z = 0; z < g.mcount; ++z)
+        table += (long long)g.K[sg][z] * g.Arows[sg][z] * (long long)g.esz * pieces;
+  }
+  const bool fits = split ? 4 * wide <= 5 * used && tiles >= 512
+                          : 10 * wide <= 11 * used && tiles >= 2048;
+  return fits && table >= (16ll << 20) ? 64 : 32;
+}
+
 // Cuts the work groups of one direction into panels (group x 64-row tile),
 // their k-step lists and (panel, column tile) work items, in XCD-aware order.
 // Workgroups are dispatched round-robin over the 8 XCDs and the kernels walk
@@ -1162,7 +1196,10 @@ void plan_batch(arwen_sht_batch* B, const arwen_sht_job* jobs, int njobs) {
     setup_job(B, js.get(), true);
     B->jobs.push_back(std::move(js));
   }
-  for (int d = 0; d < 2; ++d) build_lists(d, B->groups[d], B->config.cols[d], B->lists[d]);
+  for (int d = 0; d < 2; ++d) {
+    B->config.cols[d] = default_cols(B->groups[d], B->precision);
+    build_lists(d, B->groups[d], B->config.cols[d], B->lists[d]);
+  }
   if (!g_setup_stream) hip_check(hipDeviceSynchronize(), "batch setup");
 }
 
@@ -1974,7 +2011,9 @@ int arwen_sht_batch_autotune(arwen_sht_batch* B, void* stream, int reps,
       // split accumulators, is a candidate only where they are off.
       const bool wide = B->precision == ARWEN_SHT_FP32 || !B->config.split_acc;
       const std::vector<int> cols = wide ? std::vector<int>{32, 64, 96} : std::vector<int>{32, 64};
-      const int grids[4] = {256 * 4, 256 * 8, 256 * 16, 256 * 32};
+      // from one generation of 64- or 96-column blocks (96-column analysis at
+      // T383, 160 columns: 69.8 us there, 78.4 with 256 x 8) to one tile a block
+      const int grids[4] = {256 * 2, 256 * 4, 256 * 8, 256 * 32};
       for (int d = 0; d < 2; ++d) {
         if (B->lists[d].ntiles == 0) continue;
         float best_ms = 0.f;
