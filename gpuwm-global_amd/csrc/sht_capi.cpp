@@ -756,14 +756,16 @@ void add_ana_group(std::vector<HostGroup>& b, const arwen_sht_plan* P, int mb, i
 //     17.7, T383 2 31.8 -> 28.9
 //   two contractions, <= 36:       T255 2 fields 38.0 -> 36.6, 4 39.1 -> 39.6;
 //     T383 1 58.5 -> 54.7
-//   analysis, fields K^3 <= 100:   T95 16 fields 14.5 -> 12.8, 32 15.8 -> 16.6;
-//     T191 2 15.7 -> 13.8, 4 16.2 -> 17.1; T255 1 18.3 -> 17.2, 2 18.6 -> 20.2
+//   analysis, fields K^3 <= 100, and 256 up to 16 fields (bf16x6): T127 16
+//     fields 17.3 -> 14.3; T191 8 17.0 -> 16.1, 16 19.7 -> 23.8; T255 4
+//     19.1 -> 18.1, 8 20.8 -> 21.0; T383 1 29.6 -> 27.7, 4 31.3 -> 33.6;
+//     T511 1 50.3 -> 56.2
 bool small_job(const arwen_sht_batch* B, const arwen_sht_job& J) {
   if (!B->single || J.op == ARWEN_SHT_OP_UV_FROM_VORDIV || J.op == ARWEN_SHT_OP_VORDIV_FROM_UV ||
       J.op == ARWEN_SHT_OP_VORDIV_FROM_WAIST || J.op == ARWEN_SHT_OP_DIVERGENCE_FROM_WAIST)
     return false;
   const long long K = (J.plan->T + 64) / 64, n = J.count;
-  if (!is_synthesis(J.op)) return n * K * K * K <= 100;
+  if (!is_synthesis(J.op)) return n * K * K * K <= (n <= 16 ? 256 : 100);
   const bool two = J.op == ARWEN_SHT_OP_GRADIENT || J.op == ARWEN_SHT_OP_SYNTHESIS_GRADIENT;
   return n * K * K <= (two ? 36 : 72);
 }

@@ -61,6 +61,7 @@
 // Lane l of a
 // 16x16 MFMA: (l & 15) is the row/column and (l >> 4) selects the k chunk;
 // A and B use the same k mapping.
+#include <algorithm>
 #include <type_traits>
 
 #include "sht_kernels.h"
@@ -774,7 +775,7 @@ extern "C" hipError_t sht_launch_legendre_gemm(const sht::GemmLaunch* L, hipStre
 
 namespace {
 
-// Row tiles per wavefront: as many as still leave the chip two blocks per CU
+// Synthesis row tiles per wavefront: as many as still leave the chip two blocks per CU
 // (more tiles per gathered data fragment), at most 4.
 int small_row_tiles(int blocks_of_one, int tiles) {
   int rt = 4;
@@ -791,8 +792,7 @@ void launch_small_syn(const sht::SmallSynArgs& a, int rt, dim3 g, hipStream_t s)
 template <int MODE>
 void launch_small_ana(const sht::SmallAnaArgs& a, int rt, dim3 g, hipStream_t s) {
   if (rt == 4) hipLaunchKernelGGL((sht::small_analysis_kernel<MODE, 4>), g, dim3(256), 0, s, a);
-  else if (rt == 2) hipLaunchKernelGGL((sht::small_analysis_kernel<MODE, 2>), g, dim3(256), 0, s, a);
-  else hipLaunchKernelGGL((sht::small_analysis_kernel<MODE, 1>), g, dim3(256), 0, s, a);
+  else hipLaunchKernelGGL((sht::small_analysis_kernel<MODE, 2>), g, dim3(256), 0, s, a);
 }
 
 }  // namespace
@@ -818,7 +818,12 @@ extern "C" hipError_t sht_launch_small_analysis(const sht::SmallAnaArgs* a, int 
                                                 hipStream_t s) {
   if (a->nfields <= 0) return hipSuccess;
   const int MB = (a->T + sht::kMT) / sht::kMT, tiles = (a->T / 2 + 16) / 16, cg = (a->nfields + 7) / 8;
-  const int rt = small_row_tiles(MB * tiles * cg, tiles);  // half of the blocks lie past the triangle
+  // Row tiles per wavefront: four share one gathered data fragment where the
+  // rows are many or the fields spread the gathers over more lines, else two
+  // (more wavefronts).  Two against four, us a call (bf16x6): T127 8 fields
+  // 13.2 : 14.2, T191 1 field 12.2 : 13.0, 4 15.4 : 14.5, T255 1 15.4 : 15.8,
+  // 4 19.8 : 18.1, T383 1 29.9 : 27.7.
+  const int rt = tiles >= 6 && std::min(a->nfields, 8) * tiles * tiles >= 128 ? 4 : 2;
   sht::SmallAnaArgs b = *a;
   b.rgroups = (tiles + rt - 1) / rt;
   const dim3 g((unsigned)(MB * 2 * b.rgroups), (unsigned)cg);

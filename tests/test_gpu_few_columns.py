@@ -55,3 +55,23 @@ def test_few_fields_have_the_grouped_bits(T, nlat, nlon, counts, precision):
         w = t.contract_to_waist(c)
         assert np.isfinite(w.values.abs().sum().item())
         assert (t.waist_to_grid(w) - got[0]).abs().max() <= 2e-6 * got[0].abs().max()
+
+
+@pytest.mark.parametrize("precision", ["float32", "bf16x6", "bf16x3"])
+@pytest.mark.parametrize("T,nlat,nlon,counts", [
+    (30, 31, 64, (1, 16)), (127, 128, 256, (16, 17)), (160, 170, 486, (6, 9)),
+    (191, 192, 384, (1, 3, 4, 9, 10)), (255, 257, 514, (3,))])
+def test_few_field_analysis_row_tiles(T, nlat, nlon, counts, precision):
+    """Two and four row tiles per wavefront, the last block partly past the
+    degrees (tiles not a multiple of four), both sides of the field counts."""
+    import torch
+
+    from arwen_spectral import SphericalHarmonicTransform, TransformBatch
+
+    t = SphericalHarmonicTransform.create(T, nlat=nlat, nlon=nlon, dealias_factor=1.0,
+                                          precision=precision)
+    for n in counts:
+        f = torch.randn(n, nlat, nlon, device="cuda")
+        out = torch.full((n, T + 1, T + 1), 7.0, device="cuda", dtype=torch.complex64)
+        TransformBatch([("forward", t, f, out)]).run()
+        assert torch.equal(t.forward(f), out), f"T{T} {n} fields"
