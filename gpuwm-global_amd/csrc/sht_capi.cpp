@@ -15,6 +15,7 @@
 #include <list>
 #include <memory>
 #include <mutex>
+#include <queue>
 #include <string>
 #include <tuple>
 #include <vector>
@@ -435,11 +436,13 @@ struct HostGroup {
   size_t esz = 4;                   // table element bytes (4 fp32, 2 bf16 pieces); data are fp32
 };
 
-// Device work lists of one GEMM direction, built for one column tile.
+// Device work lists of one GEMM direction, built for one column tile and grid.
 struct GemmLists {
-  DevBuf panels, steps, tiles;
-  int ntiles = 0;
+  DevBuf panels, steps, items;
+  int nitems = 0, nsteps = 0;
   int bn = 0;
+  int slots = 0;  // the grid asked for
+  int grid = 0;   // workgroups launched (at most `slots`)
 };
 
 struct JobState {
@@ -507,16 +510,17 @@ constexpr int kXcds = 8;  // MI355X: 8 XCDs x 32 CUs
 // its table fragments through L1 once for its columns, so 64 halve that
 // traffic; they cost residency (two blocks per CU, not three) and padding.
 // Measured (us, 32 against 64 columns, synthesis / analysis):
-//   bf16x6  T383 160 columns 76.2/80.6 : 69.4/76.2, 256 columns 122/121 : 96/101
-//           T255 128 columns 25.2/28.6 : 21.7/25.9, 160 columns 31.0/35.0 : 30.7/35.0
-//           T383 80 columns (128 padded) 48.3/51.1 : 48.3/54.8
-//           T127 320 columns 18.2/17.5 : 20.1/19.5
-//   fp32    T383 256 columns 118/126 : 109/121, 128 columns 63.6/71.5 : 61.4/75.7,
-//           160 columns 77.7/84.8 : 81.5/94.8
+//   bf16x6  T383 160 columns 77.1/80.0 : 66.6/72.0, 256 columns 121/123 : 95/98
+//           T255 128 columns 24.7/27.6 : 22.0/25.5, 160 columns 32.1/32.5 : 30.0/34.1
+//           T383 80 columns (128 padded) 49.8/52.2 : 45.5/55.6
+//           T127 256 columns 17.0/17.5 : 16.6/19.5
+//   fp32    T383 256 columns 122/125 : 106/115, 128 columns 64.4/70.5 : 58.2/72.5,
+//           160 columns 78.9/78.9 : 77.3/81.7; T255 256 columns 49.5/54.4 : 43.0/54.1
 // so: tables from half of the eight 4 MB L2s up; in the split modes at most a
-// quarter of padding and as many tiles as run together (512), in FP32, whose
-// MFMA time weighs more, hardly any padding and four times as many tiles.
-int default_cols(const std::vector<HostGroup>& groups, int precision) {
+// quarter of padding and as many tiles as run together (512), or in synthesis
+// more padding and twice the tiles; in FP32, whose MFMA time weighs more,
+// hardly any padding and two (synthesis) or four times as many tiles.
+int default_cols(int dir, const std::vector<HostGroup>& groups, int precision) {
   const bool split = precision != ARWEN_SHT_FP32;
   long long tiles = 0, used = 0, wide = 0, table = 0;
   const int pieces = split ? (precision == ARWEN_SHT_BF16X6 ? 3 : 2) : 1;
@@ -531,36 +535,53 @@ int default_cols(const std::vector<HostGroup>& groups, int precision) {
       for (int z = 0; z < g.mcount; ++z)
         table += (long long)g.K[sg][z] * g.Arows[sg][z] * (long long)g.esz * pieces;
   }
-  const bool fits = split ? 4 * wide <= 5 * used && tiles >= 512
-                          : 10 * wide <= 11 * used && tiles >= 2048;
+  const bool fits = split ? (4 * wide <= 5 * used && tiles >= 512) ||
+                                (dir == 0 && 5 * wide <= 8 * used && tiles >= 1024)
+                          : 10 * wide <= 11 * used && tiles >= (dir == 0 ? 1024 : 2048);
   return fits && table >= (16ll << 20) ? 64 : 32;
 }
 
+// Persistent grid of direction d; 0 in the config = the workgroups that are
+// resident together (256 CUs).
+int gemm_slots(const arwen_sht_batch* B, const arwen_sht_gemm_config& c, int d) {
+  return c.grid[d] > 0 ? c.grid[d]
+                       : 256 * sht::gemm_blocks_per_cu(B->precision == ARWEN_SHT_FP32, c.cols[d]);
+}
+
 // Cuts the work groups of one direction into panels (group x 64-row tile),
-// their k-step lists and (panel, column tile) work items, in XCD-aware order.
-// Workgroups are dispatched round-robin over the 8 XCDs and the kernels walk
-// the list with a grid stride that is a multiple of 8, so list position t
-// always runs on XCD t % 8.  Every work item of one group (same orders, same
-// tables, same data columns) goes to one XCD, where its tiles run side by
-// side and share that XCD's L2; groups are balanced over the XCDs longest
-// first.  Short lists are padded with idle items (-1).
-void build_lists(int dir, const std::vector<HostGroup>& groups, int bn, GemmLists& out) {
+// their k-step lists and (panel, column tile) work items, and deals the items
+// to `slots` persistent workgroups.
+// Workgroups are dispatched round-robin over the 8 XCDs, and the grid is a
+// multiple of 8, so workgroup b runs on XCD b % 8.  Every work item of one
+// group (same orders, same tables, same data columns) goes to one XCD, where
+// its tiles run side by side and share that XCD's L2; groups are balanced
+// over the XCDs longest first, and an XCD's items go, in that order, each to
+// its workgroup with the least work so far.  A workgroup walks its own queue,
+// so it knows its next item early enough to load it ahead.
+// The time of an item: its steps, and kItemSteps more for its stores and its
+// change-over (measured at T383 with 32-column tiles: 0.8 us a step, 1.6 us
+// of stores).
+constexpr int kItemSteps = 2;
+
+void build_lists(int dir, const std::vector<HostGroup>& groups, int bn, int slots,
+                 GemmLists& out) {
   const int TR = sht::kGemmBM;
   std::vector<sht::GemmPanel> panels;
   std::vector<sht::GemmStep> steps;
   std::vector<long long> gwork(groups.size(), 0);
-  std::vector<std::vector<int2>> per_group(groups.size());
+  std::vector<std::vector<sht::GemmItem>> per_group(groups.size());
   for (size_t gid = 0; gid < groups.size(); ++gid) {
     const HostGroup& g = groups[gid];
     int Rmax = 0;
     for (int z = 0; z < g.mcount; ++z) Rmax = std::max(Rmax, g.R[z]);
     for (int r0 = 0; r0 < Rmax; r0 += TR) {
       sht::GemmPanel pn{};
-      pn.step0 = (int)steps.size();
-      pn.N = g.N;
-      pn.bcs = g.bcs;
+      sht::GemmItem it{};
+      it.step0 = (int)steps.size();
+      it.N = g.N;
+      it.bcs = g.bcs;
+      it.piece_bytes = g.piece_bytes;
       pn.ccs = g.ccs;
-      pn.piece_bytes = g.piece_bytes;
       for (int z = 0; z < sht::kMT; ++z) {
         pn.rows[z] = z < g.mcount ? std::max(0, std::min(TR, g.R[z] - r0)) : 0;
         if (dir == 0)
@@ -603,28 +624,27 @@ void build_lists(int dir, const std::vector<HostGroup>& groups, int bn, GemmList
           }
         }
       }
-      pn.nsteps = (int)steps.size() - pn.step0;
+      it.nsteps = (int)steps.size() - it.step0;
       bool any = false;
-      for (int e = pn.step0; e < (int)steps.size(); ++e) any = any || steps[e].a_bytes > 0;
+      for (int e = it.step0; e < (int)steps.size(); ++e) any = any || steps[e].a_bytes > 0;
       if (!any) {  // nothing reaches this row tile
-        steps.resize(pn.step0);
+        steps.resize(it.step0);
         continue;
       }
-      if (pn.nsteps + 2 > sht::kGemmMaxSteps)
+      if (it.nsteps + sht::kGemmNulls > sht::kGemmMaxSteps)
         fail(ARWEN_SHT_EINVAL, "truncation too large for the GEMM step list (" +
-                                   std::to_string(pn.nsteps) + " steps in one panel, at most " +
-                                   std::to_string(sht::kGemmMaxSteps - 2) + ")");
-      // two null steps: the kernel's loads run ahead of the list's end
+                                   std::to_string(it.nsteps) + " steps in one panel, at most " +
+                                   std::to_string(sht::kGemmMaxSteps - sht::kMT) + ")");
+      // null steps: the kernel's loads run ahead of the list's end
       sht::GemmStep null{};
-      null.a = steps[pn.step0].a;
-      null.b = steps[pn.step0].b ? steps[pn.step0].b : steps[pn.step0].a;
-      steps.push_back(null);
-      steps.push_back(null);
-      const int pid = (int)panels.size();
+      null.a = steps[it.step0].a;
+      null.b = steps[it.step0].b ? steps[it.step0].b : steps[it.step0].a;
+      for (int e = 0; e < sht::kGemmNulls; ++e) steps.push_back(null);
       panels.push_back(pn);
-      for (int c0 = 0; c0 < g.N; c0 += bn) {
-        gwork[gid] += (long long)pn.nsteps * std::min(bn, g.N - c0);
-        per_group[gid].push_back(int2{pid, c0});
+      it.panel = (int)panels.size();
+      for (it.c0 = 0; it.c0 < g.N; it.c0 += bn) {
+        gwork[gid] += it.nsteps + kItemSteps;
+        per_group[gid].push_back(it);
       }
     }
   }
@@ -633,24 +653,42 @@ void build_lists(int dir, const std::vector<HostGroup>& groups, int bn, GemmList
   for (size_t g = 0; g < order.size(); ++g) order[g] = (int)g;
   std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return gwork[a] > gwork[b]; });
   std::vector<long long> load(nx, 0);
-  std::vector<std::vector<int2>> lists(nx);
+  std::vector<std::vector<sht::GemmItem>> lists(nx);
   for (int g : order) {
     if (per_group[g].empty()) continue;
     const int x = (int)(std::min_element(load.begin(), load.end()) - load.begin());
     load[x] += gwork[g];
-    for (auto& tt : per_group[g]) lists[x].push_back(tt);
+    lists[x].insert(lists[x].end(), per_group[g].begin(), per_group[g].end());
   }
   size_t longest = 0;
   for (auto& l : lists) longest = std::max(longest, l.size());
-  std::vector<int2> t;
-  t.reserve(longest * nx);
-  for (size_t j = 0; j < longest; ++j)
-    for (int x = 0; x < nx; ++x) t.push_back(j < lists[x].size() ? lists[x][j] : int2{-1, 0});
+  // workgroups per XCD; a launch takes at least one each
+  const int per_xcd = (int)std::max<size_t>(1, std::min<size_t>(slots / nx, longest));
+  std::vector<std::vector<sht::GemmItem>> queues((size_t)per_xcd * nx);
+  for (int x = 0; x < nx; ++x) {
+    using Slot = std::pair<long long, int>;  // work so far, workgroup of the XCD
+    std::priority_queue<Slot, std::vector<Slot>, std::greater<Slot>> free;
+    for (int b = 0; b < per_xcd; ++b) free.push({0, b});
+    for (const sht::GemmItem& it : lists[x]) {
+      const Slot sl = free.top();
+      free.pop();
+      queues[(size_t)sl.second * nx + x].push_back(it);
+      free.push({sl.first + it.nsteps + kItemSteps, sl.second});
+    }
+  }
+  longest = 0;
+  for (auto& q : queues) longest = std::max(longest, q.size());
+  std::vector<sht::GemmItem> t(longest * queues.size());  // zero = none
+  for (size_t b = 0; b < queues.size(); ++b)
+    for (size_t k = 0; k < queues[b].size(); ++k) t[k * queues.size() + b] = queues[b][k];
   upload(out.panels, panels);
   upload(out.steps, steps);
-  upload(out.tiles, t);
-  out.ntiles = (int)t.size();
+  upload(out.items, t);
+  out.nitems = (int)t.size();
+  out.nsteps = (int)steps.size();
   out.bn = bn;
+  out.slots = slots;
+  out.grid = (int)queues.size();
 }
 
 const char* table_block(const arwen_sht_plan* P, int kind, bool syn, int m, int p,
@@ -1199,8 +1237,8 @@ void plan_batch(arwen_sht_batch* B, const arwen_sht_job* jobs, int njobs) {
     B->jobs.push_back(std::move(js));
   }
   for (int d = 0; d < 2; ++d) {
-    B->config.cols[d] = default_cols(B->groups[d], B->precision);
-    build_lists(d, B->groups[d], B->config.cols[d], B->lists[d]);
+    B->config.cols[d] = default_cols(d, B->groups[d], B->precision);
+    build_lists(d, B->groups[d], B->config.cols[d], gemm_slots(B, B->config, d), B->lists[d]);
   }
   if (!g_setup_stream) hip_check(hipDeviceSynchronize(), "batch setup");
 }
@@ -1221,15 +1259,6 @@ void plan_batch_on(arwen_sht_batch* B, const arwen_sht_job* jobs, int njobs, hip
   plan_batch(B, jobs, njobs);
 }
 
-// Persistent grid of direction d: a multiple of the XCD count (see
-// build_lists); 0 in the config = 8 workgroups per CU.
-int gemm_grid(const arwen_sht_batch* B, int d) {
-  int g = B->config.grid[d] > 0 ? B->config.grid[d] : 256 * 8;
-  g = std::min(g, std::max(B->lists[d].ntiles, 1));
-  if (g >= kXcds) g -= g % kXcds;
-  return std::max(g, 1);
-}
-
 hipError_t launch_gemm(const arwen_sht_batch* B, int d, hipStream_t s) {
   const GemmLists& L = B->lists[d];
   sht::GemmLaunch g{};
@@ -1239,9 +1268,10 @@ hipError_t launch_gemm(const arwen_sht_batch* B, int d, hipStream_t s) {
   g.acc2 = B->config.split_acc;
   g.panels = L.panels.as<sht::GemmPanel>();
   g.steps = L.steps.as<sht::GemmStep>();
-  g.tiles = L.tiles.as<int2>();
-  g.ntiles = L.ntiles;
-  g.grid = gemm_grid(B, d);
+  g.items = L.items.as<sht::GemmItem>();
+  g.nitems = L.nitems;
+  g.nsteps = L.nsteps;
+  g.grid = L.grid;
   return sht_launch_legendre_gemm(&g, s);
 }
 
@@ -1310,7 +1340,8 @@ void apply_config(arwen_sht_batch* B, const arwen_sht_gemm_config& c) {
   hip_check(hipDeviceSynchronize(), "config change");
   drop_graph(B);
   for (int d = 0; d < 2; ++d)
-    if (B->lists[d].bn != c.cols[d]) build_lists(d, B->groups[d], c.cols[d], B->lists[d]);
+    if (B->lists[d].bn != c.cols[d] || B->lists[d].slots != gemm_slots(B, c, d))
+      build_lists(d, B->groups[d], c.cols[d], gemm_slots(B, c, d), B->lists[d]);
   B->config = c;
   hip_check(hipDeviceSynchronize(), "config upload");
 }
@@ -2013,11 +2044,10 @@ int arwen_sht_batch_autotune(arwen_sht_batch* B, void* stream, int reps,
       // split accumulators, is a candidate only where they are off.
       const bool wide = B->precision == ARWEN_SHT_FP32 || !B->config.split_acc;
       const std::vector<int> cols = wide ? std::vector<int>{32, 64, 96} : std::vector<int>{32, 64};
-      // from one generation of 64- or 96-column blocks (96-column analysis at
-      // T383, 160 columns: 69.8 us there, 78.4 with 256 x 8) to one tile a block
-      const int grids[4] = {256 * 2, 256 * 4, 256 * 8, 256 * 32};
+      // one generation of resident blocks, or more that the hardware deals
+      const int grids[2] = {0, 256 * 8};
       for (int d = 0; d < 2; ++d) {
-        if (B->lists[d].ntiles == 0) continue;
+        if (B->lists[d].nitems == 0) continue;
         float best_ms = 0.f;
         for (int bn : cols) {
           for (int gr : grids) {

@@ -32,8 +32,17 @@
 // one barrier ends the step; ANA needs barriers only where its resident B
 // tile changes.  The panel's step descriptors sit in LDS for the whole tile,
 // so no memory load other than the tiles is waited on inside the loop.
-// Reads past the panel's list return its last null step (extent 0), so every
-// load is issued unconditionally.
+//
+// A workgroup's items follow each other without a gap: the host deals each
+// workgroup its queue, an item's LDS list ends with the next item's first
+// three steps (null steps, extent 0, where there is none), so the last trip's
+// loads are the next item's, and they are in flight while the outputs are
+// stored.  What bounds the launch is what it moves: the tables and data once
+// from memory, and 12 KB of table per 64-column step through L1; without
+// MFMAs it takes the same time.  T383 bf16x6, 160 columns, 64-column tiles:
+// 69.4 / 77.5 us (synthesis / analysis) with a prologue of 4-5 us per tile
+// (panel, list, first tiles, each waited on) and list order, 66.6 / 72.0 us
+// here; 96-column analysis 78.4 -> 69.5 us.
 //
 // LDS B tiles are unpadded rows of 32 k, one row per column (128 bytes fp32,
 // 64 bytes per bf16 piece), whose 16-byte chunks are XOR-swizzled by row, so
@@ -105,8 +114,25 @@ struct GemmDesc {
 struct GemmWork {
   const GemmPanel* panels;
   const GemmStep* steps;
-  const int2* tiles;  // {panel, c0}; panel < 0 = idle padding
-  int ntiles;
+  const GemmItem* items;
+  int nitems, nsteps;  // entries of items and steps
+};
+
+// A work item as every lane loads it (16-byte vectors); uniform fields.
+struct GemmItemRaw {
+  u32x4 lo, hi;
+  __device__ __forceinline__ GemmItem scalar() const {
+    auto rfl = [](unsigned v) { return (unsigned)__builtin_amdgcn_readfirstlane((int)v); };
+    GemmItem t;
+    t.panel = (int)rfl(lo[0]);
+    t.c0 = (int)rfl(lo[1]);
+    t.step0 = (int)rfl(lo[2]);
+    t.nsteps = (int)rfl(lo[3]);
+    t.N = (int)rfl(hi[0]);
+    t.bcs = (int)rfl(hi[1]);
+    t.piece_bytes = (long long)(((unsigned long long)rfl(hi[3]) << 32) | rfl(hi[2]));
+    return t;
+  }
 };
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(unsigned long long addr,
@@ -198,153 +224,252 @@ __device__ __forceinline__ void mfma_step(f32x4& acc, f32x4& acc2, const u32x4 (
 #undef SHT_MFMA_BF
 }
 
-// 32-column tiles fit three workgroups per CU (<= 168 VGPRs), 64- and
-// 96-column ones two (the 96-column analysis tile's LDS, B tile plus step
+// 32-column tiles fit three workgroups per CU (<= 168 VGPRs; fp32 four, <= 128),
+// 64- and 96-column ones two (the 96-column analysis tile's LDS, B tile plus step
 // list, is exactly half of the CU's 160 KB in bf16x6).
 template <int MODE, int DIR, int BN, bool ACC2>
-__global__ void __launch_bounds__(256, BN == 32 ? 3 : 2) legendre_gemm_kernel(GemmWork w) {
+__global__ void __launch_bounds__(256, gemm_blocks_per_cu(MODE == kFP32, BN)) legendre_gemm_kernel(GemmWork w) {
   using C = GemmCfg<MODE, DIR, BN>;
   constexpr bool F32 = C::F32;
   constexpr int NP = C::NP, ROWB = C::ROWB, NB = C::NB;
   __shared__ __attribute__((aligned(16))) unsigned char sB[C::B_BUFS][NP * C::B_TILE];
-  __shared__ u32x4 sDesc[2 * kGemmMaxSteps];  // the current panel's step list
+  // the current panel's step list, the next item's first steps (kGemmNulls)
+  // and the item after that one
+  __shared__ u32x4 sDesc[2 * kGemmMaxSteps];
 
   const SHT_CONST GemmPanel* panels = (const SHT_CONST GemmPanel*)w.panels;
-  const SHT_CONST int2* tiles = (const SHT_CONST int2*)w.tiles;
 
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
   const int li = lane & 15, kg = lane >> 4;
   const int arow = 16 * wave + li;  // the row of this lane's A fragment
 
-  for (int t = blockIdx.x; t < w.ntiles; t += gridDim.x) {
-    const int2 tile = tiles[t];
-    if (tile.x < 0) continue;
-    const GemmPanel P = panels[tile.x];
-    const int c0 = tile.y;
-    const int ncol = min(BN, P.N - c0);
-    const unsigned long long coloff = (unsigned long long)c0 * P.bcs * 4;  // fp32 data
-    const int step0 = P.step0, nsteps = P.nsteps;
+  // this workgroup's items: list positions blockIdx.x + k gridDim.x (none past
+  // the list)
+  int pos = blockIdx.x;
+  auto load_item = [&](int at) {
+    GemmItem it = ((const SHT_CONST GemmItem*)w.items)[min(at, w.nitems - 1)];
+    if (at >= w.nitems) it.panel = 0;
+    return it;
+  };
+  GemmItem cur = load_item(pos), nxt = load_item(pos + (int)gridDim.x),
+           nn = load_item(pos + 2 * (int)gridDim.x);
+  if (cur.panel == 0) return;  // block-uniform
+  GemmPanel P = panels[cur.panel - 1];
 
-    // ---- register stages and their loads: step j's tiles sit in stage
-    // j % 4 (its order within the trip), so loads run three steps ahead.
-    // ANA loads B once per trip (one stage). ----
-    constexpr int kStages = kMT;
-    constexpr int kBStages = DIR == 0 ? kStages : 1;
-    u32x4 ra[kStages][C::A_REGS], rb[kBStages][C::B_REGS];
-    // The panel's step list (with its two null steps) is copied to LDS once
-    // per tile; a step's descriptor is then an LDS broadcast read, off the
-    // memory queue that the tile loads wait in.
-    {
-      const __amdgpu_buffer_rsrc_t srs = make_rsrc(
-          reinterpret_cast<unsigned long long>(w.steps) + (unsigned long long)step0 * 32,
-          (unsigned)(nsteps + 2) * 32u);
-      for (int e = tid; e < 2 * (nsteps + 2); e += 256) sDesc[e] = load16(srs, (unsigned)e * 16u);
-      __syncthreads();
+  // An item's LDS list: entries 2 j, 2 j + 1 = step j; from j = nsteps the
+  // first kGemmNulls steps of the item `after` it (its own null steps where
+  // there is none), then the item at list position `at3` (zeros = none past
+  // the list).  At most 512 16-byte entries.  load_list takes a thread's first
+  // entry and the item's two, without branches; put_list writes them, and
+  // loads and writes the second entry of a list of more than 256.
+  const __amdgpu_buffer_rsrc_t srs =
+      make_rsrc(reinterpret_cast<unsigned long long>(w.steps), (unsigned)w.nsteps * 32u);
+  const __amdgpu_buffer_rsrc_t irs =
+      make_rsrc(reinterpret_cast<unsigned long long>(w.items), (unsigned)w.nitems * 32u);
+  constexpr unsigned kNoRead = ~15u;  // past every extent: 0, and no memory access
+  auto list_entry = [&](int q, const GemmItem& it, const GemmItem& after) {
+    const int n2 = 2 * it.nsteps;
+    const int own = 2 * it.step0, tail = (after.panel ? 2 * after.step0 : own + n2) - n2;
+    const unsigned off = (unsigned)(q + (q < n2 ? own : tail)) * 16u;
+    return load16(srs, q < n2 + 2 * kGemmNulls ? off : kNoRead);
+  };
+  auto load_list = [&](u32x4(&e)[2], const GemmItem& it, const GemmItem& after, int at3) {
+    int tl = threadIdx.x;
+    asm volatile("" : "+v"(tl));  // formed per item, not held across the loop
+    e[0] = list_entry(tl, it, after);
+    e[1] = load16(irs, tl < 2 ? (unsigned)at3 * 32u + (unsigned)tl * 16u : kNoRead);
+  };
+  auto put_list = [&](const u32x4(&e)[2], const GemmItem& it, const GemmItem& after) {
+    int tl = threadIdx.x;
+    asm volatile("" : "+v"(tl));
+    const int n = 2 * (it.nsteps + kGemmNulls);
+    if (tl < n) sDesc[tl] = e[0];
+    if (tl < 2) sDesc[n + tl] = e[1];
+    if (n > 256 && tl + 256 < n) sDesc[tl + 256] = list_entry(tl + 256, it, after);
+  };
+
+  // ---- register stages and their loads: step j's tiles sit in stage j % 4
+  // (its order within the trip), so loads run three steps ahead.  ANA loads B
+  // once per trip (one stage). ----
+  constexpr int kStages = kMT;
+  constexpr int kBStages = DIR == 0 ? kStages : 1;
+  u32x4 ra[kStages][C::A_REGS], rb[kBStages][C::B_REGS];
+  int nsteps = cur.nsteps;
+  auto fetch_desc = [&](int j) {
+    const int e = 2 * min(j, nsteps + kGemmNulls - 1);
+    return GemmDesc{sDesc[e], sDesc[e + 1]};
+  };
+  // what a step's loads need of its item
+  struct Cols {
+    long long piece_bytes;
+    unsigned long long coloff;
+    int ncol, bcs;
+  };
+  auto cols_of = [](const GemmItem& it) {
+    return Cols{it.piece_bytes, (unsigned long long)it.c0 * it.bcs * 4,  // fp32 data
+                min(BN, it.N - it.c0), it.bcs};
+  };
+  Cols in = cols_of(cur);  // of the item whose steps are being loaded
+  // WITH_B: the step may carry a B tile (SYN: every step; ANA: the first
+  // step of each k-chunk, position 0 of a trip of kMT steps)
+  auto issue = [&](u32x4(&A)[C::A_REGS], u32x4(&B)[C::B_REGS], const GemmStep& s,
+                   auto WITH_B) {
+    // A: this lane's fragment of each piece, 16 bytes (bf16: k chunk kg of
+    // row arow; fp32: chunks kg and kg + 4); rows past a_bytes read 0
+#pragma unroll
+    for (int pc = 0; pc < NP; ++pc) {
+      const __amdgpu_buffer_rsrc_t r =
+          make_rsrc(s.a + (unsigned long long)(pc * in.piece_bytes), s.a_bytes);
+      if constexpr (F32) {
+        A[0] = load16(r, (unsigned)(arow * ROWB + kg * 16));
+        A[1] = load16(r, (unsigned)(arow * ROWB + (kg + 4) * 16));
+      } else {
+        A[pc] = load16(r, (unsigned)(arow * ROWB + kg * 16));
+      }
     }
-    auto fetch_desc = [&](int j) {
-      const int e = 2 * min(j, nsteps + 1);
-      return GemmDesc{sDesc[e], sDesc[e + 1]};
-    };
-    // WITH_B: the step may carry a B tile (SYN: every step; ANA: the first
-    // step of each k-chunk, position 0 of a trip of kMT steps)
-    auto issue = [&](u32x4(&A)[C::A_REGS], u32x4(&B)[C::B_REGS], const GemmStep& s,
-                     auto WITH_B) {
-      // A: this lane's fragment of each piece, 16 bytes (bf16: k chunk kg of
-      // row arow; fp32: chunks kg and kg + 4); rows past a_bytes read 0
+    const int rev = (s.cmap & 1) ? 3 : 0;
+    if constexpr (DIR == 0) {
+      // packed fp32 columns, k contiguous: a thread takes 4 k of one column
+      int ext = (in.ncol - 1) * in.bcs + s.b_klen;
+      asm volatile("" : "+s"(ext));  // a select, not a branch across the step's loads
+      const unsigned bytes = s.b_klen > 0 ? (unsigned)ext * 4u : 0u;
+      const __amdgpu_buffer_rsrc_t r = make_rsrc(s.b + in.coloff, bytes);
 #pragma unroll
-      for (int pc = 0; pc < NP; ++pc) {
-        const __amdgpu_buffer_rsrc_t r =
-            make_rsrc(s.a + (unsigned long long)(pc * P.piece_bytes), s.a_bytes);
+      for (int u = 0; u < C::B_REGS; ++u) {
+        const int q = tid + 256 * u;
+        const int col = q >> 3;
+        B[u] = load16(r, (unsigned)((col ^ rev) * in.bcs * 4 + (q & 7) * 16));
+      }
+    } else if constexpr (decltype(WITH_B)::value) {
+      // k-chunk of the fp32 waist: per column 32 latitudes x 4 orders; a
+      // thread takes 4 latitudes (a quad, 64 bytes) of one column
+      int ext = (in.ncol - 1) * in.bcs + s.b_klen * kMT;
+      asm volatile("" : "+s"(ext));
+      const unsigned bytes = s.b_klen > 0 ? (unsigned)ext * 4u : 0u;
+      const __amdgpu_buffer_rsrc_t r = make_rsrc(s.b + in.coloff, bytes);
+#pragma unroll
+      for (int u = 0; u < BN / 32; ++u) {
+        const int q = tid + 256 * u;
+        const int col = q >> 3, quad = q & 7;
+        const unsigned off = (unsigned)((col ^ rev) * in.bcs * 4 + quad * 64);
+#pragma unroll
+        for (int h = 0; h < 4; ++h) B[u * 4 + h] = load16(r, off + 16u * h);
+      }
+    }
+  };
+  // B stage -> LDS (split into pieces in the bf16 modes); `cmap` bits 1..4
+  // negate columns 0..3 of each group of four
+  auto put_b = [&](const u32x4(&B)[C::B_REGS], int buf, int cmap) {
+    auto flip_of = [&](int col) { return ((cmap >> (1 + (col & 3))) & 1) ? 0x80000000u : 0u; };
+    if constexpr (DIR == 0) {
+#pragma unroll
+      for (int u = 0; u < C::B_REGS; ++u) {
+        const int q = tid + 256 * u;
+        const int col = q >> 3, ch = q & 7;  // 4 k starting at 4 ch
+        const u32x4 v = B[u] ^ flip_of(col);
+        unsigned char* row = &sB[buf][col * ROWB];
         if constexpr (F32) {
-          A[0] = load16(r, (unsigned)(arow * ROWB + kg * 16));
-          A[1] = load16(r, (unsigned)(arow * ROWB + (kg + 4) * 16));
+          *reinterpret_cast<u32x4*>(row + swz<true>(col, ch) * 16) = v;
         } else {
-          A[pc] = load16(r, (unsigned)(arow * ROWB + kg * 16));
+          const float x[4] = {__uint_as_float(v[0]), __uint_as_float(v[1]),
+                              __uint_as_float(v[2]), __uint_as_float(v[3])};
+          u32x2 pcs[3];
+          split4(x, NP, pcs);
+#pragma unroll
+          for (int pc = 0; pc < NP; ++pc)
+            *reinterpret_cast<u32x2*>(row + pc * C::B_TILE + swz<false>(col, ch >> 1) * 16 +
+                                      (ch & 1) * 8) = pcs[pc];
         }
       }
-      const int rev = (s.cmap & 1) ? 3 : 0;
-      if constexpr (DIR == 0) {
-        // packed fp32 columns, k contiguous: a thread takes 4 k of one column
-        const unsigned bytes =
-            s.b_klen > 0 ? (unsigned)(((ncol - 1) * P.bcs + s.b_klen) * 4) : 0u;
-        const __amdgpu_buffer_rsrc_t r = make_rsrc(s.b + coloff, bytes);
+    } else {
+      (void)buf;
 #pragma unroll
-        for (int u = 0; u < C::B_REGS; ++u) {
-          const int q = tid + 256 * u;
-          const int col = q >> 3;
-          B[u] = load16(r, (unsigned)((col ^ rev) * P.bcs * 4 + (q & 7) * 16));
-        }
-      } else if constexpr (decltype(WITH_B)::value) {
-        // k-chunk of the fp32 waist: per column 32 latitudes x 4 orders; a
-        // thread takes 4 latitudes (a quad, 64 bytes) of one column
-        const unsigned bytes =
-            s.b_klen > 0 ? (unsigned)(((ncol - 1) * P.bcs + s.b_klen * kMT) * 4) : 0u;
-        const __amdgpu_buffer_rsrc_t r = make_rsrc(s.b + coloff, bytes);
+      for (int u = 0; u < BN / 32; ++u) {
+        const int q = tid + 256 * u;
+        const int col = q >> 3, quad = q & 7;
+        const unsigned flip = flip_of(col);
+        const u32x4* v = &B[u * 4];  // v[h] = latitude 4 quad + h, four orders
 #pragma unroll
-        for (int u = 0; u < BN / 32; ++u) {
-          const int q = tid + 256 * u;
-          const int col = q >> 3, quad = q & 7;
-          const unsigned off = (unsigned)((col ^ rev) * P.bcs * 4 + quad * 64);
-#pragma unroll
-          for (int h = 0; h < 4; ++h) B[u * 4 + h] = load16(r, off + 16u * h);
-        }
-      }
-    };
-    // B stage -> LDS (split into pieces in the bf16 modes); `cmap` bits 1..4
-    // negate columns 0..3 of each group of four
-    auto put_b = [&](const u32x4(&B)[C::B_REGS], int buf, int cmap) {
-      auto flip_of = [&](int col) { return ((cmap >> (1 + (col & 3))) & 1) ? 0x80000000u : 0u; };
-      if constexpr (DIR == 0) {
-#pragma unroll
-        for (int u = 0; u < C::B_REGS; ++u) {
-          const int q = tid + 256 * u;
-          const int col = q >> 3, ch = q & 7;  // 4 k starting at 4 ch
-          const u32x4 v = B[u] ^ flip_of(col);
-          unsigned char* row = &sB[buf][col * ROWB];
+        for (int z = 0; z < kMT; ++z) {
+          unsigned char* row = &sB[0][(z * BN + col) * ROWB];
+          const u32x4 wv = u32x4{v[0][z], v[1][z], v[2][z], v[3][z]} ^ flip;
           if constexpr (F32) {
-            *reinterpret_cast<u32x4*>(row + swz<true>(col, ch) * 16) = v;
+            *reinterpret_cast<u32x4*>(row + swz<true>(col, quad) * 16) = wv;
           } else {
-            const float x[4] = {__uint_as_float(v[0]), __uint_as_float(v[1]),
-                                __uint_as_float(v[2]), __uint_as_float(v[3])};
+            const float x[4] = {__uint_as_float(wv[0]), __uint_as_float(wv[1]),
+                                __uint_as_float(wv[2]), __uint_as_float(wv[3])};
             u32x2 pcs[3];
             split4(x, NP, pcs);
 #pragma unroll
             for (int pc = 0; pc < NP; ++pc)
-              *reinterpret_cast<u32x2*>(row + pc * C::B_TILE + swz<false>(col, ch >> 1) * 16 +
-                                        (ch & 1) * 8) = pcs[pc];
-          }
-        }
-      } else {
-        (void)buf;
-#pragma unroll
-        for (int u = 0; u < BN / 32; ++u) {
-          const int q = tid + 256 * u;
-          const int col = q >> 3, quad = q & 7;
-          const unsigned flip = flip_of(col);
-          const u32x4* v = &B[u * 4];  // v[h] = latitude 4 quad + h, four orders
-#pragma unroll
-          for (int z = 0; z < kMT; ++z) {
-            unsigned char* row = &sB[0][(z * BN + col) * ROWB];
-            const u32x4 wv = u32x4{v[0][z], v[1][z], v[2][z], v[3][z]} ^ flip;
-            if constexpr (F32) {
-              *reinterpret_cast<u32x4*>(row + swz<true>(col, quad) * 16) = wv;
-            } else {
-              const float x[4] = {__uint_as_float(wv[0]), __uint_as_float(wv[1]),
-                                  __uint_as_float(wv[2]), __uint_as_float(wv[3])};
-              u32x2 pcs[3];
-              split4(x, NP, pcs);
-#pragma unroll
-              for (int pc = 0; pc < NP; ++pc)
-                *reinterpret_cast<u32x2*>(row + pc * C::B_TILE + swz<false>(col, quad >> 1) * 16 +
-                                          (quad & 1) * 8) = pcs[pc];
-            }
+              *reinterpret_cast<u32x2*>(row + pc * C::B_TILE + swz<false>(col, quad >> 1) * 16 +
+                                        (quad & 1) * 8) = pcs[pc];
           }
         }
       }
-    };
+    }
+  };
 
-    f32x4 acc[kMT][NB], acc2[kMT][NB];
+  f32x4 acc[kMT][NB], acc2[kMT][NB];
+
+  // B fragments of a step's column block nb from LDS buffer `buf`
+  auto fragment = [&](int buf, auto ZC, int nb, u32x4(&bf)[3]) {
+    const int bbuf = DIR == 0 ? buf : 0;
+    constexpr int bz = DIR == 0 ? 0 : decltype(ZC)::value;
+    const int col = nb * 16 + li;
+    const unsigned char* base = &sB[bbuf][(bz * BN + col) * ROWB];
+    if constexpr (F32) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        bf[h] = *reinterpret_cast<const u32x4*>(base + swz<true>(col, kg + 4 * h) * 16);
+    } else {
+#pragma unroll
+      for (int pc = 0; pc < NP; ++pc)
+        bf[pc] = *reinterpret_cast<const u32x4*>(base + pc * C::B_TILE + swz<false>(col, kg) * 16);
+    }
+  };
+  // one step into the accumulators of order Z: A fragments from register
+  // stage Z, B fragments from LDS buffer `buf` (kEarly: block 0's already in bf)
+  constexpr bool kEarly = DIR == 0 || F32;
+  auto compute = [&](int buf, auto ZC, u32x4(&bf)[3]) {
+    constexpr int Z = decltype(ZC)::value;
+    u32x4 af[3];
+#pragma unroll
+    for (int r = 0; r < C::A_REGS; ++r) af[r] = ra[Z][r];
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+      if (nb > 0 || !kEarly) fragment(buf, ZC, nb, bf);
+      if constexpr (ACC2) mfma_step<MODE>(acc[Z][nb], acc2[Z][nb], af, bf);
+      else mfma_step<MODE>(acc[Z][nb], acc[Z][nb], af, bf);
+    }
+  };
+
+  // ---- the first item's prologue: steps 0, 1 and 2 in flight, step 0's B
+  // in LDS buffer 0 ----
+  // q1, q2, q3: steps j+1, j+2, j+3 (scalar) at the start of step j; dn:
+  // the raw descriptor of step j+4, fetched one step ahead.
+  GemmStep q1, q2, q3;
+  GemmDesc dn;
+  u32x4 list[2];
+  load_list(list, cur, nxt, pos + 3 * (int)gridDim.x);
+  put_list(list, cur, nxt);
+  __syncthreads();
+  {
+    const GemmStep s0 = fetch_desc(0).scalar();
+    q1 = fetch_desc(1).scalar();
+    q2 = fetch_desc(2).scalar();
+    issue(ra[0], rb[0], s0, std::true_type{});
+    issue(ra[1], rb[DIR == 0 ? 1 : 0], q1, std::integral_constant<bool, DIR == 0>{});
+    issue(ra[2], rb[DIR == 0 ? 2 : 0], q2, std::integral_constant<bool, DIR == 0>{});
+    q3 = fetch_desc(3).scalar();
+    dn = fetch_desc(4);
+    put_b(rb[0], 0, s0.cmap);
+  }
+  __syncthreads();
+
+  for (;;) {
+    const int c0 = cur.c0, ncol = in.ncol;
 #pragma unroll
     for (int a = 0; a < kMT; ++a)
 #pragma unroll
@@ -353,90 +478,73 @@ __global__ void __launch_bounds__(256, BN == 32 ? 3 : 2) legendre_gemm_kernel(Ge
         acc2[a][n] = f32x4{0.f, 0.f, 0.f, 0.f};
       }
 
-    // one step into the accumulators of order Z: A fragments from register
-    // stage Z, B fragments from LDS buffer `buf`
-    auto compute = [&](int buf, auto ZC) {
-      constexpr int Z = decltype(ZC)::value;
-      const int bbuf = DIR == 0 ? buf : 0;
-      constexpr int bz = DIR == 0 ? 0 : Z;
-      u32x4 af[3];
-#pragma unroll
-      for (int r = 0; r < C::A_REGS; ++r) af[r] = ra[Z][r];
-#pragma unroll
-      for (int nb = 0; nb < NB; ++nb) {
-        const int col = nb * 16 + li;
-        const unsigned char* base = &sB[bbuf][(bz * BN + col) * ROWB];
-        u32x4 bf[3];
-        if constexpr (F32) {
-#pragma unroll
-          for (int h = 0; h < 2; ++h)
-            bf[h] = *reinterpret_cast<const u32x4*>(base + swz<true>(col, kg + 4 * h) * 16);
-        } else {
-#pragma unroll
-          for (int pc = 0; pc < NP; ++pc)
-            bf[pc] =
-                *reinterpret_cast<const u32x4*>(base + pc * C::B_TILE + swz<false>(col, kg) * 16);
-        }
-        if constexpr (ACC2) mfma_step<MODE>(acc[Z][nb], acc2[Z][nb], af, bf);
-        else mfma_step<MODE>(acc[Z][nb], acc[Z][nb], af, bf);
-      }
-    };
-
-    // ---- prologue: steps 0, 1 and 2 in flight, step 0's B in LDS buffer 0 ----
-    // q1, q2, q3: steps j+1, j+2, j+3 (scalar) at the start of step j; dn:
-    // the raw descriptor of step j+4, fetched one step ahead.
-    GemmStep q1, q2, q3;
-    GemmDesc dn;
-    {
-      const GemmStep s0 = fetch_desc(0).scalar();
-      q1 = fetch_desc(1).scalar();
-      q2 = fetch_desc(2).scalar();
-      issue(ra[0], rb[0], s0, std::true_type{});
-      issue(ra[1], rb[DIR == 0 ? 1 : 0], q1, std::integral_constant<bool, DIR == 0>{});
-      issue(ra[2], rb[DIR == 0 ? 2 : 0], q2, std::integral_constant<bool, DIR == 0>{});
-      q3 = fetch_desc(3).scalar();
-      dn = fetch_desc(4);
-      put_b(rb[0], 0, s0.cmap);
-    }
-    __syncthreads();
-
     // ---- main loop: trips of kMT steps, one per order Z of the panel (the
     // host pads every k-chunk to kMT steps), so each step's accumulators,
     // register stage and LDS buffer are fixed at compile time ----
-    auto body = [&](auto ZC, int j) {
+    // The last trip loads the next item's first three steps (the list goes on
+    // with them), so an item begins with its tiles in flight.
+    int next_cmap = 0;  // of the next item's step 0 (ANA)
+    auto body = [&](auto ZC, int j, bool last) {
       constexpr int Z = decltype(ZC)::value;
       constexpr int s = Z & 1;               // LDS buffer of step j's B (SYN)
       constexpr int R3 = (Z + 3) % kStages;  // register stage (= trip position) of step j+3
       constexpr int R1 = (Z + 1) % kStages;  // register stage of step j+1
+      // the first fragments' LDS reads go ahead of the loads' issue (the split
+      // analysis, whose registers are full, leaves the order to the compiler)
+      u32x4 bf[3];
+      if constexpr (kEarly) {
+        fragment(s, ZC, 0, bf);
+        __builtin_amdgcn_sched_barrier(0);
+      }
       issue(ra[R3], rb[DIR == 0 ? R3 : 0], q3, std::integral_constant<bool, DIR == 0 || R3 == 0>{});
       const GemmStep q4 = dn.scalar();
       dn = fetch_desc(j + 5);
-      compute(s, ZC);
+      compute(s, ZC, bf);
       if constexpr (DIR == 0) {
         // step j+1's B goes to the other buffer; the barrier orders it before
         // step j+1 reads it and after every read of this buffer two steps ago
-        if (j + 1 < nsteps) put_b(rb[R1], s ^ 1, q1.cmap);
+        // (after the MFMAs: among them, its wait for the loads would stall them)
+        __builtin_amdgcn_sched_barrier(0);
+        put_b(rb[R1], s ^ 1, q1.cmap);
         __syncthreads();
       } else if constexpr (R1 == 0) {
         // ANA: the resident B tile changes with the next trip
-        __syncthreads();  // every wavefront is done with it
-        if (j + 1 < nsteps) put_b(rb[0], 0, q1.cmap);
-        __syncthreads();
+        next_cmap = q1.cmap;
+        if (!last) {
+          __syncthreads();  // every wavefront is done with it
+          put_b(rb[0], 0, q1.cmap);
+          __syncthreads();
+        }
       }
       q1 = q2;
       q2 = q3;
       q3 = q4;
     };
     static_assert(kMT == 4, "trip of four steps");
+    GemmItem n3{};
     for (int j = 0; j < nsteps; j += kMT) {
-      body(std::integral_constant<int, 0>{}, j);
-      body(std::integral_constant<int, 1>{}, j + 1);
-      body(std::integral_constant<int, 2>{}, j + 2);
-      body(std::integral_constant<int, 3>{}, j + 3);
+      const bool last = j + kMT >= nsteps;
+      body(std::integral_constant<int, 0>{}, j, last);
+      if (last && nxt.panel) {
+        in = cols_of(nxt);
+        // the item after the next two, which this list ends with: read here,
+        // where barriers still lie between it and any wavefront's put_list
+        // (SYN: the ends of the next three steps; ANA: the epilogue's)
+        const int e = 2 * (nsteps + kGemmNulls);
+        n3 = GemmItemRaw{sDesc[e], sDesc[e + 1]}.scalar();
+      }
+      body(std::integral_constant<int, 1>{}, j + 1, last);
+      body(std::integral_constant<int, 2>{}, j + 2, last);
+      body(std::integral_constant<int, 3>{}, j + 3, last);
     }
+    if (nxt.panel) load_list(list, nxt, nn, pos + 4 * (int)gridDim.x);
 
     // ---- epilogue: this lane holds rows 16 wave + 4 kg + q (q < 4) of
-    // column 16 nb + li ----
+    // column 16 nb + li.  The thread index is made opaque, so that nothing
+    // derived from it here is formed before the loop and held across it. ----
+    int te = threadIdx.x;
+    asm volatile("" : "+v"(te));
+    const int elane = te & 63, ewave = te >> 6, eli = te & 15, ekg = elane >> 4;
     auto wave_lds_sync = [] {  // this wavefront's LDS accesses, in order
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
@@ -444,7 +552,7 @@ __global__ void __launch_bounds__(256, BN == 32 ? 3 : 2) legendre_gemm_kernel(Ge
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     };
     if constexpr (DIR == 0) {
-      // A lane's four rows x four orders are 64 contiguous bytes of the
+      // A elane's four rows x four orders are 64 contiguous bytes of the
       // waist, and the four lanes of a column 256.  Each column block passes
       // through the wavefront's own LDS area, transposed, so that a store
       // instruction writes four whole 256-byte column runs rather than 16-byte
@@ -453,7 +561,7 @@ __global__ void __launch_bounds__(256, BN == 32 ? 3 : 2) legendre_gemm_kernel(Ge
       // to 17 against bank conflicts); declared here, so the analysis
       // instantiations keep their LDS budget
       __shared__ f32x4 sOut[4 * 16 * 17];
-      f32x4* mine = sOut + wave * 16 * 17;
+      f32x4* mine = sOut + ewave * 16 * 17;
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb) {
 #pragma unroll
@@ -465,13 +573,13 @@ __global__ void __launch_bounds__(256, BN == 32 ? 3 : 2) legendre_gemm_kernel(Ge
             if constexpr (!F32 && ACC2) v = v + acc2[zz][nb];
             o[zz] = v[q];
           }
-          mine[li * 17 + 4 * kg + q] = o;
+          mine[eli * 17 + 4 * ekg + q] = o;
         }
         wave_lds_sync();
-        const int r = lane & 15, row = 16 * wave + r;
+        const int r = elane & 15, row = 16 * ewave + r;
 #pragma unroll
-        for (int tt = 0; tt < 4; ++tt) {  // columns 4 tt + lane / 16 of the block, row r
-          const int cl = 4 * tt + (lane >> 4), col = nb * 16 + cl;
+        for (int tt = 0; tt < 4; ++tt) {  // columns 4 tt + elane / 16 of the block, row r
+          const int cl = 4 * tt + (elane >> 4), col = nb * 16 + cl;
           const f32x4 o = mine[cl * 17 + r];
           if (col < ncol && row < P.rows[0])
             *reinterpret_cast<SHT_GLOBAL f32x4*>(reinterpret_cast<SHT_GLOBAL float*>(P.c[0]) +
@@ -496,13 +604,13 @@ __global__ void __launch_bounds__(256, BN == 32 ? 3 : 2) legendre_gemm_kernel(Ge
         for (int nb = 0; nb < NB; ++nb) {
           f32x4 v = acc[zz][nb];
           if constexpr (!F32 && ACC2) v = v + acc2[zz][nb];
-          *reinterpret_cast<f32x4*>(stage + (nb * 16 + li) * CS + 16 * wave + 4 * kg) = v;
+          *reinterpret_cast<f32x4*>(stage + (nb * 16 + eli) * CS + 16 * ewave + 4 * ekg) = v;
         }
         __syncthreads();
-        const int r4 = 4 * (lane & 15);
+        const int r4 = 4 * (elane & 15);
 #pragma unroll
-        for (int tt = 0; tt < BN / 16; ++tt) {  // columns 4 (wave + 4 tt) + lane / 16
-          const int col = 4 * (wave + 4 * tt) + (lane >> 4);
+        for (int tt = 0; tt < BN / 16; ++tt) {  // columns 4 (ewave + 4 tt) + elane / 16
+          const int col = 4 * (ewave + 4 * tt) + (elane >> 4);
           const f32x4 o = *reinterpret_cast<const f32x4*>(stage + col * CS + r4);
           if (col < ncol && r4 < P.rows[zz])
             *reinterpret_cast<SHT_GLOBAL f32x4*>(reinterpret_cast<SHT_GLOBAL float*>(P.c[zz]) +
@@ -510,7 +618,25 @@ __global__ void __launch_bounds__(256, BN == 32 ? 3 : 2) legendre_gemm_kernel(Ge
         }
       }
     }
-    __syncthreads();  // sB and sDesc are reused by the next tile
+    if (nxt.panel == 0) break;  // block-uniform
+    cur = nxt;
+    P = panels[cur.panel - 1];
+    nxt = nn;
+    nn = n3;
+    pos += gridDim.x;
+    nsteps = cur.nsteps;
+    if constexpr (DIR == 1) {
+      __syncthreads();  // the staged outputs are read: sB is free
+      put_b(rb[0], 0, next_cmap);
+    }
+    // every wavefront has passed its last reads of the old list: they precede
+    // the barrier that ends the loop (SYN) or those of the epilogue (ANA)
+    put_list(list, cur, nxt);
+    __syncthreads();
+    q1 = fetch_desc(1).scalar();
+    q2 = fetch_desc(2).scalar();
+    q3 = fetch_desc(3).scalar();
+    dn = fetch_desc(4);
   }
 }
 
@@ -764,10 +890,10 @@ hipError_t launch_dir(int mode, const sht::GemmWork& w, int bn, int acc2, dim3 g
 }  // namespace
 
 extern "C" hipError_t sht_launch_legendre_gemm(const sht::GemmLaunch* L, hipStream_t s) {
-  if (L->ntiles <= 0) return hipSuccess;
+  if (L->nitems <= 0) return hipSuccess;
   if (L->bn != 32 && L->bn != 64 && L->bn != 96) return hipErrorInvalidValue;
   if (L->bn == 96 && L->acc2 && L->mode != sht::kFP32) return hipErrorInvalidValue;
-  const sht::GemmWork w{L->panels, L->steps, L->tiles, L->ntiles};
+  const sht::GemmWork w{L->panels, L->steps, L->items, L->nitems, L->nsteps};
   const dim3 g(L->grid);
   return L->dir == 0 ? launch_dir<0>(L->mode, w, L->bn, L->acc2, g, s)
                      : launch_dir<1>(L->mode, w, L->bn, L->acc2, g, s);

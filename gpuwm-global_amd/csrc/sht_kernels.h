@@ -215,21 +215,34 @@ struct GemmStep {
 };
 
 constexpr int kGemmBM = 64;      // GEMM block tile rows
-constexpr int kGemmMaxSteps = 256;  // steps per panel incl. the two null steps (LDS-resident):
-                                     // two segments of JHP/32 chunks x 4 orders, JHP <= 992;
-                                     // 8 KB, which with the 72 KB B tile of the 96-column
-                                     // bf16x6 analysis leaves room for two blocks per CU
+constexpr int kGemmNulls = 3;     // null steps after a panel's list
+constexpr int kGemmMaxSteps = 256;  // steps per panel incl. the null steps (LDS-resident, with
+                                     // one work item in the 32 bytes left: a list is a multiple
+                                     // of four steps): two segments of JHP/32 chunks x 4
+                                     // orders, JHP <= 992; 8 KB, which with the 72 KB B tile of
+                                     // the 96-column bf16x6 analysis leaves room for two blocks
+                                     // per CU
+// Workgroups per CU the kernels are compiled for: the default persistent grid.
+constexpr int gemm_blocks_per_cu(bool f32, int bn) { return bn == 32 ? (f32 ? 4 : 3) : 2; }
 
 struct GemmPanel {
   unsigned long long c[kMT];  // SYN: c[0] = waist block + r0 rows; ANA: packed block of order z + r0
-  long long piece_bytes;      // bf16 piece stride of the tables (data B are fp32)
-  int step0, nsteps;          // steps[step0 .. step0+nsteps), followed by two null steps
-  int N;                      // data columns
-  int bcs;                    // B column stride, floats
   int ccs;                    // C column stride, floats
   int rows[kMT];              // rows of C written per order (<= tile rows)
-  int pad;
+  int pad[3];
 };
+
+// A work item: one panel and BN of its columns, with what the loads of its
+// steps need.
+struct GemmItem {
+  int panel;              // 1 + index of the panel; 0 = none
+  int c0;                 // first column
+  int step0, nsteps;      // steps[step0 .. step0+nsteps), followed by kGemmNulls null steps
+  int N;                  // data columns
+  int bcs;                // B column stride, floats
+  long long piece_bytes;  // bf16 piece stride of the tables (data B are fp32)
+};
+static_assert(sizeof(GemmItem) == 32 && sizeof(GemmPanel) == 64, "as the kernel loads them");
 static_assert(sizeof(GemmStep) == 32, "GemmStep is one 8-dword scalar load");
 
 // One grouped-GEMM launch: precision mode, direction (0 SYN, 1 ANA), column
@@ -238,8 +251,8 @@ struct GemmLaunch {
   int mode, dir, bn, acc2;
   const GemmPanel* panels;
   const GemmStep* steps;
-  const int2* tiles;
-  int ntiles, grid;
+  const GemmItem* items;  // workgroup b's k-th item at [k * grid + b]
+  int nitems, nsteps, grid;  // entries of items and steps; workgroups
 };
 
 // ---- the vector operators' FP64 low orders (sht_lowm.hip) ----

@@ -348,8 +348,9 @@ int arwen_sht_batch_launch(arwen_sht_batch* batch, void* stream);
 int arwen_sht_batch_profile(arwen_sht_batch* batch, void* stream, int reps, double* ms);
 /* Grouped-GEMM schedule of a batch, per direction (0 synthesis, 1 analysis):
  * column tile (32, 64 or 96 data columns per workgroup; 96 only with
- * split_acc = 0 in the split precisions) and persistent grid (workgroups,
- * 0 = 8 per CU); for the split precisions, whether the small products keep
+ * split_acc = 0 in the split precisions; a new batch takes 32 or 64 by its
+ * sizes) and persistent grid (workgroups, a multiple of 8; 0 = as many as run
+ * together); for the split precisions, whether the small products keep
  * their own accumulators (1, default) or share the main one (0).  Changing
  * it rebuilds the work lists and drops the captured graph.  No reference
  * counterpart (the reference has no kernel schedule). */
