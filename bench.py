@@ -559,7 +559,7 @@ def sampler_bench(args, torch):
                    "fields": F, "points": N},
         "float32": res["float32"], "gradient": res["gradient"], "wind": res["wind"],
         "roofline": {"bound": "valu_fp64",
-                     "kernel": "sample_pack + sample_kernel<8, 0, false> + sample_reduce",
+                     "kernel": "sample_pack + sample_kernel + sample_reduce",
                      "achieved": achieved, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": achieved / FP64_PEAK_TFLOPS, "traffic": None,
                      "algorithmic_flop_per_call": flops},
@@ -664,7 +664,7 @@ def vertical_bench(args, torch):
         "vs_baseline": None, "dtype": "f32",
         "data": "synthetic: seeded red-spectrum fields, synthetic well-posed vertical operator",
         "config": {"workload": f"solve_shifted T{T}, {L} levels", "T": T, "levels": L},
-        "roofline": {"bound": "hbm", "kernel": "vertical_rows_kernel", "achieved": achieved,
+        "roofline": {"bound": "hbm", "kernel": "vertical_kernel", "achieved": achieved,
                      "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS,
                      "traffic": None, "algorithmic_bytes": alg},
         "other_operations": others,
