@@ -1641,7 +1641,9 @@ int arwen_sht_spectral_op(arwen_sht_plan* P, int op, const void* in, void* out, 
 }
 
 namespace {
-constexpr int kSampleColPad = 8;  // sampler field columns are padded to the widest field tile
+// Sampler field columns are padded to one 8-field MFMA column tile; a
+// wavefront takes several, never more than there are (sht_sample_tile).
+constexpr int kSampleColPad = 8;
 
 int sample_columns(int count, int kind) {
   const long long cols = (kind == 2 ? 2LL : 1LL) * count;

@@ -371,6 +371,8 @@ hipError_t sht_launch_waist_fold(const sht::WaistFoldArgs* a, hipStream_t s);
 hipError_t sht_launch_waist_unfold(const sht::WaistUnfoldArgs* a, hipStream_t s);
 hipError_t sht_launch_sample_pack(const sht::SamplePackArgs* a, hipStream_t s);
 hipError_t sht_launch_sample(const sht::SampleArgs* a, hipStream_t s);
+// point tiles (16 points) and column tiles (8 fields) of a wavefront of that launch
+void sht_sample_tile(int kind, int ldc, int npts, int parts, int* pt, int* ct);
 hipError_t sht_launch_vertical_solve(const sht::VerticalArgs* a, hipStream_t s);
 hipError_t sht_launch_pack(const sht::PackArgs* a, hipStream_t s);
 hipError_t sht_launch_low_synthesis(const sht::LowSynArgs* a, hipStream_t s);

@@ -413,6 +413,7 @@ namespace {
 template <int PT, int CT, int KIND, bool F32>
 hipError_t launch_sample_tile(const sht::SampleArgs& a, hipStream_t s) {
   const int tiles = a.ldc / 8;
+  if (tiles < CT) return hipErrorInvalidValue;  // the first column would be negative
   const dim3 g((unsigned)((a.npts + 64 * PT - 1) / (64 * PT)), (unsigned)((tiles + CT - 1) / CT),
                (unsigned)a.cuts.parts);
   hipLaunchKernelGGL((sht::sample_kernel<PT, CT, KIND, F32>), g, dim3(256), 0, s,
@@ -426,35 +427,51 @@ hipError_t launch_sample_tile(const sht::SampleArgs& a, hipStream_t s) {
 // registers of two wavefronts per SIMD hold (five for values, two for the two
 // bases of gradients and winds) feed the most MFMAs per basis value and
 // coefficient; fewer points or columns take smaller tiles, so that the launch
-// still has a wavefront for each of the chip's 1024 SIMDs.
-template <int KIND, bool F32>
-hipError_t launch_sample_kind(const sht::SampleArgs& a, hipStream_t s) {
-  const long long most = KIND == 0 ? 5 : 2, tiles = a.ldc / 8;
+// still has a wavefront for each of the chip's 1024 SIMDs.  ct is the even
+// share of the column tiles between the groups, so it is never above their
+// number: a group wider than all of them would begin at a negative column.
+struct SampleTile {
+  int pt, ct;
+};
+SampleTile sample_tile(int kind, int ldc, int npts, int parts) {
+  const long long most = kind == 0 ? 5 : 2, tiles = ldc / 8;
   const long long groups = (tiles + most - 1) / most;
   const int ct = (int)((tiles + groups - 1) / groups);
-  const long long waves2 = (a.npts + 31) / 32 * groups * a.cuts.parts;
-  const long long waves1 = (a.npts + 15) / 16 * groups * a.cuts.parts;
-  if (waves2 >= 2048 || (waves2 >= 1024 && ct >= 2)) {
-    switch (ct) {
-      case 1: return launch_sample_tile<2, 1, KIND, F32>(a, s);
-      case 2: return launch_sample_tile<2, 2, KIND, F32>(a, s);
-      default:
-        if constexpr (KIND == 0) {
-          if (ct == 3) return launch_sample_tile<2, 3, KIND, F32>(a, s);
-          if (ct == 4) return launch_sample_tile<2, 4, KIND, F32>(a, s);
-          return launch_sample_tile<2, 5, KIND, F32>(a, s);
-        }
-    }
+  const long long waves2 = ((long long)npts + 31) / 32 * groups * parts;
+  const long long waves1 = ((long long)npts + 15) / 16 * groups * parts;
+  if (waves2 >= 2048 || (waves2 >= 1024 && ct >= 2)) return {2, ct};
+  if (waves1 >= 1024 && ct >= 2) return {1, ct};
+  return {1, 1};
+}
+
+template <int KIND, bool F32>
+hipError_t launch_sample_kind(const sht::SampleArgs& a, hipStream_t s) {
+  const SampleTile t = sample_tile(KIND, a.ldc, a.npts, a.cuts.parts);
+#define SHT_TILE(PT, CT) \
+  if (t.pt == PT && t.ct == CT) return launch_sample_tile<PT, CT, KIND, F32>(a, s)
+  SHT_TILE(1, 1);
+  SHT_TILE(1, 2);
+  SHT_TILE(2, 1);
+  SHT_TILE(2, 2);
+  if constexpr (KIND == 0) {
+    SHT_TILE(1, 3);
+    SHT_TILE(1, 4);
+    SHT_TILE(1, 5);
+    SHT_TILE(2, 3);
+    SHT_TILE(2, 4);
+    SHT_TILE(2, 5);
   }
-  if (waves1 >= 1024 && ct >= 2) {
-    if constexpr (KIND == 0)
-      if (ct > 2) return launch_sample_tile<1, 5, KIND, F32>(a, s);
-    return launch_sample_tile<1, 2, KIND, F32>(a, s);
-  }
-  return launch_sample_tile<1, 1, KIND, F32>(a, s);
+#undef SHT_TILE
+  return hipErrorInvalidValue;
 }
 
 }  // namespace
+
+extern "C" void sht_sample_tile(int kind, int ldc, int npts, int parts, int* pt, int* ct) {
+  const SampleTile t = sample_tile(kind, ldc, npts, parts);
+  *pt = t.pt;
+  *ct = t.ct;
+}
 
 extern "C" hipError_t sht_launch_sample(const sht::SampleArgs* a, hipStream_t s) {
   if (a->npts <= 0 || a->ldc <= 0) return hipSuccess;

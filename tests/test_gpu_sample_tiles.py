@@ -80,3 +80,51 @@ def test_a_points_bits_do_not_depend_on_its_tile(kind, precision):
     if kind != "wind":  # fewer fields: other column tiles
         for w, got in zip(whole, call(c[3:20].copy(), slice(None))):
             assert np.array_equal(w[3:20], got)
+
+
+@pytest.mark.parametrize("T,points", [(127, 2033), (127, 3000), (127, 4064), (63, 4081), (63, 8160),
+                                      (21, 16369), (21, 32736)])
+@pytest.mark.parametrize("precision", list(TOL))
+def test_two_to_five_column_tiles_of_one_point_tile(T, points, precision):
+    """The ranges of points where a wavefront holds one point tile and several
+    column tiles, with several parts and with one (T21): the oracle's values
+    at some points, every output the bits of an 8-field call's, and nothing
+    written beside the outputs and the workspace.
+
+    Tolerance: float64 as above (T^2 / 2 roundings of 1.1e-16 are 9e-13 at
+    T127); float32 (T + 1) 6e-8."""
+    import ctypes
+
+    import torch
+
+    from arwen_spectral import _native
+
+    o = OracleTransform.create(T, dealias_factor=1.0)
+    t = hip_transform(o, "float32")
+    lib, dev = _native.load(), t.backend.device()
+    lat, lon = _points(points)
+    la, lo = np.deg2rad(lat), np.deg2rad(lon)
+    pts = [torch.from_numpy(x).to(dev) for x in (np.sin(la), np.cos(la), lo)]
+    fields = torch.from_numpy(_fields(T, 33, 5)).to(dev)
+    pad, code = 4096, 0 if precision == "float64" else 1
+    vp = lambda x: ctypes.c_void_p(x.data_ptr())  # noqa: E731
+
+    def call(c):
+        n = c.shape[0]
+        nbytes = int(lib.arwen_sht_sample_workspace_bytes(t.plan_handle, n, 0, points))
+        out = torch.full((n * points + 2 * pad,), 7.5, dtype=torch.float64, device=dev)
+        work = torch.full((nbytes + 16 * pad,), 0x5A, dtype=torch.uint8, device=dev)
+        _native.check(lib.arwen_sht_sample(
+            t.plan_handle, vp(c), None, n, *map(vp, pts), points, 0, code, vp(work[8 * pad:]),
+            nbytes, vp(out[pad:]), None, t.backend.stream()))
+        assert (out[:pad] == 7.5).all() and (out[-pad:] == 7.5).all()
+        assert (work[:8 * pad] == 0x5A).all() and (work[-8 * pad:] == 0x5A).all()
+        return out[pad:-pad].reshape(n, points)
+
+    tiles = torch.cat([call(fields[k:k + 8]) for k in range(0, 33, 8)])
+    some = np.linspace(0, points - 1, 64).astype(int)
+    want = osamp.sample_scalar(o, fields.cpu().numpy().astype(np.complex128), lat[some], lon[some])
+    tol = TOL[precision] if precision == "float64" else (T + 1) * 6e-8
+    assert np.max(np.abs(tiles[:, some].cpu().numpy() - want)) < tol * np.max(np.abs(want))
+    for count in (17, 24, 25, 32, 33):
+        assert torch.equal(call(fields[:count]), tiles[:count]), count

@@ -99,3 +99,26 @@ def test_sampler_argument_rules_without_a_device():
     for args in ((1, 8), (4, 3), (True, 8), (4.5, 8)):
         with pytest.raises(ValueError):
             sampling.regular_latlon_coordinates(*args)
+
+
+@pytest.mark.parametrize("kind", [0, 1, 2], ids=["scalar", "gradient", "wind"])
+def test_a_wavefronts_columns_never_exceed_the_launchs(kind):
+    """Fields 1..128, points 1..70000 (the choice depends on blocks of 16 and
+    32 of them) and 1..8 parts: column tiles within those there are, within the
+    kernels built, and no column of the last group before the first."""
+    import ctypes
+
+    from arwen_spectral import _native
+
+    choose = _native.load().sht_sample_tile
+    pt, ct = ctypes.c_int(), ctypes.c_int()
+    p, c = ctypes.byref(pt), ctypes.byref(ct)
+    seen = set()
+    for tiles in range(1, 17):
+        for parts in range(1, 9):
+            for npts in range(1, 70001, 16):
+                choose(kind, 8 * tiles, npts, parts, p, c)
+                seen.add((tiles, pt.value, ct.value))
+    assert all(c <= t for t, _, c in seen), sorted(x for x in seen if x[2] > x[0])
+    assert {p for _, p, _ in seen} == {1, 2}
+    assert {c for _, _, c in seen} == set(range(1, 6 if kind == 0 else 3))
