@@ -275,8 +275,12 @@ __global__ void __launch_bounds__(512, NT <= 3 ? 4 : 2) vertical_kernel(Vertical
   } else {
     store_levels(a.d_out,
                  pinned(mul_add(3, col_scale(k2, bx), tl, L, mul(2, D, tl, L)), D));
-    const Cols<NT> cd = mul(1, D, NT, L);
-    store_x(pinned(mul_add(5, cd, NT, L1, mul(4, x, NT, L1)), x));
+    // P_x x and Q_x (C D) apart, added once.  Carried on in P_x x's
+    // accumulators, each of the small product's terms is rounded at its size:
+    // 1.6 times the error of theta and ln ps.  The divergence's two products
+    // are of a size, and one accumulation is as exact as two.
+    const Cols<NT> qx = mul(5, mul(1, D, NT, L), NT, L1);
+    store_x(pinned(col_axpy(mul(4, x, NT, L1), 1.f, qx), x));
   }
 }
 

@@ -58,3 +58,42 @@ def test_levels_and_orders_at_the_edges_of_tiles(trunc, nlev):
            osi.linear_tendencies(o, d, th, ps, b, c, k2, np.float32(0.7)))
     _close(si.vertical_half_apply(t, d, th, ps, b, c, *maps, k2),
            osi.half_apply(o, d, th, ps, b, c, maps, k2))
+
+
+@pytest.mark.parametrize("trunc,nlev", [(33, 17), (38, 6), (60, 40), (30, 64)])
+def test_half_map_error_is_that_of_two_sums(trunc, nlev):
+    """x' = P_x x + Q_x (C D) with the two products summed apart and added
+    once, in fp32 on the host: the device's rms error against FP64 is no more
+    than that of the same sums.  Both are rms over thousands of rounded values
+    of one distribution, so they agree to a few per cent; one accumulation
+    through both products is at least sqrt(2) off.  Line: 1.2."""
+    from arwen_spectral import semi_implicit as si
+
+    o = OracleTransform.create(trunc, dealias_factor=1.0)
+    t = hip_transform(o, "float32")
+    f32 = lambda a: np.asarray(a, dtype=np.float32)  # noqa: E731
+    b, c, _, modal = osi.synthetic_operator(nlev, seed=nlev)
+    k2 = f32(si.wave_operator(t))
+    maps = [f32(x) for x in osi.symmetric_half_maps(modal, osi.x_modes(b, c), k2, 1500.0, 0.6)]
+    b, c = f32(b), f32(c)
+    d, th, ps = (o.project(red_spectrum(trunc, lead, seed=s, scale=a)).astype(np.complex64)
+                 for lead, s, a in (((nlev,), 1, 1e-5), ((nlev,), 2, 10.0), ((), 3, 1e-2)))
+
+    def dot(a, x):  # (n, i, j) by (j, n, m), a term at a time
+        acc = np.zeros((a.shape[1], *x.shape[1:]), dtype=np.complex64)
+        for j in range(a.shape[2]):
+            term = a[:, :, j].T[:, :, None].astype(np.float64) * x[j].astype(np.complex128)
+            acc = (acc + term).astype(np.complex64)  # one rounding of each part: an fma
+        return acc
+
+    every = np.broadcast_to(c, (trunc + 1, *c.shape))
+    x = np.concatenate([th, ps[None]])
+    host = dot(maps[2], x) + dot(maps[3], dot(every, d))
+    want = osi.half_apply(o, d, th, ps, b, c, maps, k2)
+    got = si.vertical_half_apply(t, d, th, ps, b, c, *maps, k2)
+    rms = lambda e: float(np.sqrt(np.mean(np.abs(e) ** 2)))  # noqa: E731
+    keep = np.tril(np.ones((trunc + 1, trunc + 1)))
+    keep[0, 0] = 0  # passed through
+    for g, h, w in zip(got[1:], (host[:-1], host[-1]), want[1:]):
+        g = g.detach().cpu().numpy().astype(np.complex128)
+        assert rms((g - w) * keep) < 1.2 * rms((h - w) * keep)
