@@ -114,6 +114,21 @@ __device__ __forceinline__ Cols<NT> col_scale(float s, const Cols<NT>& x) {
   return o;
 }
 
+// x with the places of levels `len` and up zero.  The matrices' padding is
+// zero, but times an infinite value of the operand it leaves NaN in a
+// product's padding, which the next product would spread over the column
+// unless `len` fills its steps of four.
+template <int NT>
+__device__ __forceinline__ Cols<NT> col_trim(Cols<NT> x, int len, int g) {
+  if (len % 4 == 0) return x;  // uniform
+#pragma unroll
+  for (int r = 0; r < 4; ++r)  // only the last tile has any
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+      x.v[NT - 1][c][r] = 16 * (NT - 1) + 4 * r + g < len ? x.v[NT - 1][c][r] : 0.f;
+  return x;
+}
+
 // The level at row or column place p of a staged matrix: place 16 t + 4 g + r
 // holds level 16 t + 4 r + g.
 __device__ __forceinline__ int level_at(int p) {
@@ -268,18 +283,19 @@ __global__ void __launch_bounds__(512, NT <= 3 ? 4 : 2) vertical_kernel(Vertical
   } else if constexpr (MODE == 0) {
     Cols<NT> f = col_axpy(D, k2 * a.s_bx, bx);
     if (with_m) f = col_axpy(f, k2 * a.s_md, mul(3, D, tl, L));
-    const Cols<NT> d = mul(2, f, tl, L);
+    const Cols<NT> d = col_trim(mul(2, col_trim(f, L, g), tl, L), L, g);
     store_levels(a.d_out, pinned(d, D));
     const Cols<NT> u = col_axpy(col_scale(a.s_cd, D), a.s_cn, d);
     store_x(pinned(col_axpy(x, a.s_c, mul(1, u, NT, L)), x));
   } else {
     store_levels(a.d_out,
-                 pinned(mul_add(3, col_scale(k2, bx), tl, L, mul(2, D, tl, L)), D));
+                 pinned(mul_add(3, col_trim(col_scale(k2, bx), L, g), tl, L,
+                                     mul(2, D, tl, L)), D));
     // P_x x and Q_x (C D) apart, added once.  Carried on in P_x x's
     // accumulators, each of the small product's terms is rounded at its size:
     // 1.6 times the error of theta and ln ps.  The divergence's two products
     // are of a size, and one accumulation is as exact as two.
-    const Cols<NT> qx = mul(5, mul(1, D, NT, L), NT, L1);
+    const Cols<NT> qx = mul(5, col_trim(mul(1, D, NT, L), L1, g), NT, L1);
     store_x(pinned(col_axpy(mul(4, x, NT, L1), 1.f, qx), x));
   }
 }

@@ -97,3 +97,44 @@ def test_half_map_error_is_that_of_two_sums(trunc, nlev):
     for g, h, w in zip(got[1:], (host[:-1], host[-1]), want[1:]):
         g = g.detach().cpu().numpy().astype(np.complex128)
         assert rms((g - w) * keep) < 1.2 * rms((h - w) * keep)
+
+
+@pytest.mark.parametrize("nlev", [1, 4, 5, 15, 16, 18, 33])
+def test_an_infinite_value_stays_infinite(nlev):
+    """Matrices of one sign: +inf in one level of one column makes +inf of every
+    output it reaches, not NaN, and touches no other column.  (The solve weighs
+    the old divergence with 0 in x': 0 inf is NaN there.)"""
+    from arwen_spectral import semi_implicit as si
+
+    trunc, at = 6, (3, 1)
+    o = OracleTransform.create(trunc, dealias_factor=1.0)
+    t = hip_transform(o, "float32")
+    rng = np.random.default_rng(nlev)
+    pos = lambda *shape: rng.uniform(0.5, 1.0, shape).astype(np.float32)  # noqa: E731
+    k2, n1 = pos(trunc + 1), trunc + 1
+    b, c, m, inv = pos(nlev, nlev + 1), pos(nlev + 1, nlev), -pos(nlev, nlev), pos(n1, nlev, nlev)
+    maps = [pos(n1, nlev, nlev), pos(n1, nlev, nlev), pos(n1, nlev + 1, nlev + 1),
+            pos(n1, nlev + 1, nlev + 1)]
+    d, th, ps = (o.project(red_spectrum(trunc, lead, seed=s)).astype(np.complex64)
+                 for lead, s in (((nlev,), 1), ((nlev,), 2), ((), 3)))
+    calls = {
+        "solve": lambda d, th: si.vertical_solve_shifted(t, d, th, ps, b, c, inv, k2, 2.0),
+        "apply": lambda d, th: si.vertical_apply(t, d, th, ps, b, c, m, inv, k2, 2.0, 0.6),
+        "tendencies": lambda d, th: si.vertical_linear_tendencies(t, d, th, ps, b, c, k2, 0.7),
+        "half": lambda d, th: si.vertical_half_apply(t, d, th, ps, b, c, *maps, k2)}
+    for name, call in calls.items():
+        plain = [x.cpu().numpy() for x in call(d, th)]
+        for which in (0, 1):
+            args = [d.copy(), th.copy()]
+            args[which].real[0, at[0], at[1]] = np.inf
+            for k, (got, was) in enumerate(zip((x.cpu().numpy() for x in call(*args)), plain)):
+                # tendencies: divergence from x alone, x from divergence alone
+                reached = name != "tendencies" or (k == 0) == (which == 1)
+                column = got.real[..., at[0], at[1]]
+                if name == "solve" and which == 0 and k:
+                    assert np.isnan(column).all()
+                else:
+                    assert np.isposinf(column).all() if reached else np.isfinite(column).all(), \
+                        (name, which, k)
+                got.real[..., at[0], at[1]] = was.real[..., at[0], at[1]]
+                assert np.array_equal(got, was), (name, k)
