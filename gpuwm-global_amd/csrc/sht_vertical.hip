@@ -313,8 +313,10 @@ hipError_t launch_vertical(const sht::VerticalArgs& a, hipStream_t s) {
   // matrices, or as many as the degree has orders for.  At T383: four take
   // 52 (solve) and 90 us (half map) at 40 levels and 70 and 175 us at 64,
   // eight 52 and 82, 64 and 108; five or six spread unevenly over a CU's four
-  // SIMDs (62-73 us).
-  const int waves = std::min(8, (T1 + 15) / 16);
+  // SIMDs (62-73 us).  From 32 levels on, also eight where a degree has fewer
+  // orders (T <= 63): the others only stage, most of the time of such a launch
+  // (half map, T31: 40 levels 24.3 -> 19.0 us a call, 64 levels 53.9 -> 32.5).
+  const int waves = T1 <= 64 && NT >= 3 ? 8 : std::min(8, (T1 + 15) / 16);
   const int per = (T1 + 16 * waves - 1) / (16 * waves);
   const void* k = reinterpret_cast<const void*>(sht::vertical_kernel<NT, MODE>);
   hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
