@@ -140,9 +140,12 @@ constexpr int vertical_slot() { return 16 * NT * vertical_ld(NT); }  // floats o
 
 // NT = ceil((L + 1) / 16) tiles.  A block is one degree and 16 orders per
 // wavefront; the orders of one degree (which share its matrices) are
-// neighbours in launch order.
+// neighbours in launch order.  Two blocks per CU (128 VGPRs) where the mode
+// fits them: the tendencies also at four tiles, at the price of 8 spilled
+// registers (50 levels, 139 against 128 VGPRs: T255 35.2 -> 31.0 us, T383
+// 59.4 -> 52.0).
 template <int NT, int MODE>
-__global__ void __launch_bounds__(512, NT <= 3 ? 4 : 2) vertical_kernel(VerticalArgs a) {
+__global__ void __launch_bounds__(512, NT <= 3 || (NT == 4 && MODE == 1) ? 4 : 2) vertical_kernel(VerticalArgs a) {
   constexpr int LD = vertical_ld(NT), SLOT = vertical_slot<NT>();
   extern __shared__ float smem[];
   const int L = a.nlev, L1 = a.nlev + 1, T1 = a.T + 1;
