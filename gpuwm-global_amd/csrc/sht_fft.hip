@@ -1277,12 +1277,25 @@ int wave_rb(size_t lds8) { return lds8 <= kWaveLdsMax ? 8 : 4; }
 size_t gen_lds_bytes(int N, int rb) {
   return ((size_t)N + (size_t)rb * (2 * gen_span(N) + kSpanPad)) * sizeof(float2);
 }
-// Rows per block: the most, up to 8, that fit (a single row needs 131 KB at
-// N = 5120, the longest a plan accepts).
+// Rows per block: the most, up to 8, that fit, or half as many where more than
+// 1.25 times the wavefronts then run on a CU (LDS in granules of 1280 bytes;
+// the kernels' 104 VGPRs let 16 run): occupancy is worth more than whole lines
+// of the waist from there on.  Wind of 32 levels, us and (wavefronts), at 8 : 4
+// : 2 rows: N = 576 126.9 (8) : 116.0 (12) : 124.2 (12); 640 163.3 (8) : 147.9
+// (12) : 183.4 (10); 704 194.0 (8) : 207.0 (8) : 208.5 (10); 1152 at 4 : 2 : 1
+// 412.1 (4) : 371.1 (6) : 425.4 (5).
+// (A single row needs 131 KB at N = 5120, the longest a plan accepts.)
 int gen_rb(int N) {
-  int rb = 8;
-  while (rb > 1 && gen_lds_bytes(N, rb) > kWaveLdsMax) rb /= 2;
-  return rb;
+  int best = 1, most = 0;
+  for (int rb = 8; rb >= 1; rb /= 2) {
+    const size_t lds = (gen_lds_bytes(N, rb) + 1279) / 1280 * 1280;
+    const int waves = std::min(16, rb * (int)(kWaveLdsMax / lds));
+    if (4 * waves > 5 * most) {
+      most = waves;
+      best = rb;
+    }
+  }
+  return best;
 }
 
 // ---- the reference's Fourier waist (*lead, nlat, T+1) complex ----

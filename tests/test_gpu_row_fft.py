@@ -74,3 +74,27 @@ def test_vector_components_fold_one_at_a_time(nlon):
     for got, want in zip(v.vordiv_from_wind(u32, v32),
                          o.vordiv_from_wind(u32.astype(np.float64), v32.astype(np.float64))):
         assert rel_err(got, want) < tol
+
+
+@pytest.mark.parametrize("nlon", [558, 560, 698, 700, 1120, 1130, 1272, 1274])
+def test_lengths_either_side_of_a_change_of_rows_per_block(nlon):
+    """Eight rows a block up to 558 points, four from 560, eight from 700, two from
+    1130 and four from 1274; rows of several blocks and a remainder.
+    Tolerances as above."""
+    from arwen_spectral import VorticityDivergenceOperator
+
+    o = OracleTransform.create(18, nlat=19, nlon=nlon, dealias_factor=1.0)
+    t = hip_transform(o, "float32")
+    tol = _tol(nlon)
+    c, z, d = (red_spectrum(18, (3,), seed=s) for s in (nlon, nlon + 1, nlon + 2))
+    g32 = o.inverse(c).astype(np.float32)
+    assert rel_err(t.inverse(c), o.inverse(c)) < tol
+    assert rel_err(t.forward(g32), o.forward(g32.astype(np.float64))) < tol
+    v = VorticityDivergenceOperator(t)
+    want = o.wind_from_vordiv(z, d)
+    for got, w in zip(v.wind_from_vordiv(z, d), want):
+        assert rel_err(got, w) < tol
+    u32, v32 = (w.astype(np.float32) for w in want)
+    for got, w in zip(v.vordiv_from_wind(u32, v32),
+                      o.vordiv_from_wind(u32.astype(np.float64), v32.astype(np.float64))):
+        assert rel_err(got, w) < tol * 18 / 4
