@@ -543,9 +543,8 @@ int default_cols(int dir, const std::vector<HostGroup>& groups, int precision) {
 
 // Persistent grid of direction d; 0 in the config = the workgroups that are
 // resident together (256 CUs).
-int gemm_slots(const arwen_sht_batch* B, const arwen_sht_gemm_config& c, int d) {
-  return c.grid[d] > 0 ? c.grid[d]
-                       : 256 * sht::gemm_blocks_per_cu(B->precision == ARWEN_SHT_FP32, c.cols[d]);
+int gemm_slots(const arwen_sht_gemm_config& c, int d) {
+  return c.grid[d] > 0 ? c.grid[d] : 256 * sht::gemm_blocks_per_cu(c.cols[d]);
 }
 
 // Cuts the work groups of one direction into panels (group x 64-row tile),
@@ -1241,7 +1240,7 @@ void plan_batch(arwen_sht_batch* B, const arwen_sht_job* jobs, int njobs) {
   }
   for (int d = 0; d < 2; ++d) {
     B->config.cols[d] = default_cols(d, B->groups[d], B->precision);
-    build_lists(d, B->groups[d], B->config.cols[d], gemm_slots(B, B->config, d), B->lists[d]);
+    build_lists(d, B->groups[d], B->config.cols[d], gemm_slots(B->config, d), B->lists[d]);
   }
   if (!g_setup_stream) hip_check(hipDeviceSynchronize(), "batch setup");
 }
@@ -1343,8 +1342,8 @@ void apply_config(arwen_sht_batch* B, const arwen_sht_gemm_config& c) {
   hip_check(hipDeviceSynchronize(), "config change");
   drop_graph(B);
   for (int d = 0; d < 2; ++d)
-    if (B->lists[d].bn != c.cols[d] || B->lists[d].slots != gemm_slots(B, c, d))
-      build_lists(d, B->groups[d], c.cols[d], gemm_slots(B, c, d), B->lists[d]);
+    if (B->lists[d].bn != c.cols[d] || B->lists[d].slots != gemm_slots(c, d))
+      build_lists(d, B->groups[d], c.cols[d], gemm_slots(c, d), B->lists[d]);
   B->config = c;
   hip_check(hipDeviceSynchronize(), "config upload");
 }

@@ -224,11 +224,11 @@ __device__ __forceinline__ void mfma_step(f32x4& acc, f32x4& acc2, const u32x4 (
 #undef SHT_MFMA_BF
 }
 
-// 32-column tiles fit three workgroups per CU (<= 168 VGPRs; fp32 four, <= 128),
-// 64- and 96-column ones two (the 96-column analysis tile's LDS, B tile plus step
-// list, is exactly half of the CU's 160 KB in bf16x6).
+// 32-column tiles fit three workgroups per CU (<= 168 VGPRs), 64- and 96-column
+// ones two (the 96-column analysis tile's LDS, B tile plus step list, is exactly
+// half of the CU's 160 KB in bf16x6).
 template <int MODE, int DIR, int BN, bool ACC2>
-__global__ void __launch_bounds__(256, gemm_blocks_per_cu(MODE == kFP32, BN)) legendre_gemm_kernel(GemmWork w) {
+__global__ void __launch_bounds__(256, gemm_blocks_per_cu(BN)) legendre_gemm_kernel(GemmWork w) {
   using C = GemmCfg<MODE, DIR, BN>;
   constexpr bool F32 = C::F32;
   constexpr int NP = C::NP, ROWB = C::ROWB, NB = C::NB;

@@ -223,7 +223,10 @@ constexpr int kGemmMaxSteps = 256;  // steps per panel incl. the null steps (LDS
                                      // the 96-column bf16x6 analysis leaves room for two blocks
                                      // per CU
 // Workgroups per CU the kernels are compiled for: the default persistent grid.
-constexpr int gemm_blocks_per_cu(bool f32, int bn) { return bn == 32 ? (f32 ? 4 : 3) : 2; }
+// (FP32 with 32 columns fits four; with 1024 queues, not 768, launches of 800
+// to 1600 items are 1-2% slower: T383 32 fields inverse 30.6 : 29.2 us, gradients
+// of 8 30.0 : 28.0.)
+constexpr int gemm_blocks_per_cu(int bn) { return bn == 32 ? 3 : 2; }
 
 struct GemmPanel {
   unsigned long long c[kMT];  // SYN: c[0] = waist block + r0 rows; ANA: packed block of order z + r0
