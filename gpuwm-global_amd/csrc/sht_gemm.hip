@@ -503,8 +503,10 @@ __global__ void __launch_bounds__(256, gemm_blocks_per_cu(BN)) legendre_gemm_ker
       if constexpr (DIR == 0) {
         // step j+1's B goes to the other buffer; the barrier orders it before
         // step j+1 reads it and after every read of this buffer two steps ago
-        // (after the MFMAs: among them, its wait for the loads would stall them)
-        __builtin_amdgcn_sched_barrier(0);
+        // (in the split modes after the MFMAs: among them, its wait for the
+        // loads would stall them; FP32's MFMAs are long, and its tile goes
+        // between them: launches of one item a workgroup 1-3% faster)
+        if constexpr (!F32) __builtin_amdgcn_sched_barrier(0);
         put_b(rb[R1], s ^ 1, q1.cmap);
         __syncthreads();
       } else if constexpr (R1 == 0) {
