@@ -1277,23 +1277,35 @@ int wave_rb(size_t lds8) { return lds8 <= kWaveLdsMax ? 8 : 4; }
 size_t gen_lds_bytes(int N, int rb) {
   return ((size_t)N + (size_t)rb * (2 * gen_span(N) + kSpanPad)) * sizeof(float2);
 }
-// Rows per block: the most, up to 8, that fit, or half as many where more than
-// 1.25 times the wavefronts then run on a CU (LDS in granules of 1280 bytes;
-// the kernels' 104 VGPRs let 16 run): occupancy is worth more than whole lines
-// of the waist from there on.  Wind of 32 levels, us and (wavefronts), at 8 : 4
-// : 2 rows: N = 576 126.9 (8) : 116.0 (12) : 124.2 (12); 640 163.3 (8) : 147.9
-// (12) : 183.4 (10); 704 194.0 (8) : 207.0 (8) : 208.5 (10); 1152 at 4 : 2 : 1
-// 412.1 (4) : 371.1 (6) : 425.4 (5).
-// (A single row needs 131 KB at N = 5120, the longest a plan accepts.)
-int gen_rb(int N) {
-  int best = 1, most = 0;
+// Rows per block for `rows` rows of each of `fields` fields: the most, up to 8,
+// that fit (a single row needs 131 KB at N = 5120, the longest a plan accepts);
+// where that takes more than one round of the blocks that are resident, the
+// number of least modelled time.  A CU holds as many blocks as fit its LDS (in
+// granules of 1280 bytes), up to 16 wavefronts (104 VGPRs); a round takes 8 + w
+// units, w the wavefronts on a CU (N = 640: 15.8 us with 8, 19.8 with 12); two
+// rows and one share the lines of the waist between blocks.  Winds, us a call
+// at 8 : 4 : 2 rows, the choice in brackets:
+//   N = 576, 32 levels 126.9 : [116.0] : 124.2; 640, 32 levels 163.3 : [147.9]
+//   : 183.4, 24 levels (T213) [95.1] : 105.7; 704, 32 levels [194.0] : 207.0 :
+//   208.5; 1088 [420.7] : 554.4 : 465.3; 1152 - : 412.1 : [371.1]
+// Launches of one round: 242, one level [44.4] : 50.3, but 320 [37.5] : 36.2.
+int gen_rb(int N, int rows, int fields) {
+  constexpr int kCus = 256;
+  int best = 0;
+  double least = 0.0;
   for (int rb = 8; rb >= 1; rb /= 2) {
     const size_t lds = (gen_lds_bytes(N, rb) + 1279) / 1280 * 1280;
-    const int waves = std::min(16, rb * (int)(kWaveLdsMax / lds));
-    if (4 * waves > 5 * most) {
-      most = waves;
+    const long long blocks = std::min<long long>(16 / rb, kWaveLdsMax / lds);
+    if (blocks < 1) continue;
+    const long long groups = (long long)fields * ((rows + rb - 1) / rb);
+    const long long rounds = (groups + blocks * kCus - 1) / (blocks * kCus);
+    const double line = rb == 1 ? 1.4 : rb == 2 ? 1.2 : 1.0;
+    const double cost = (double)(rounds * (8 + rb * blocks)) * line;
+    if (best == 0 || cost < least) {
       best = rb;
+      least = cost;
     }
+    if (best == rb && rounds <= 1) break;
   }
   return best;
 }
@@ -1567,7 +1579,7 @@ extern "C" hipError_t sht_launch_rfft_fold(const sht::FoldArgs* a, hipStream_t s
   }
   // any other N: one component per launch
   if (a->job.rowscale_hi || a->job.vector) return hipErrorInvalidValue;
-  const int rb = sht::gen_rb(a->fft.N);
+  const int rb = sht::gen_rb(a->fft.N, a->JHP, a->job.nfields);
   const int groups = a->job.nfields * (a->JHP / rb);
   if (groups == 0) return hipSuccess;
   return sht::launch_persistent(sht::rfft_fold_rows_kernel, groups, rb,
@@ -1606,7 +1618,7 @@ extern "C" hipError_t sht_launch_irfft_unfold(const sht::UnfoldArgs* a, hipStrea
     return e;
   }
   if (a->job.rowscale_hi) return hipErrorInvalidValue;  // order-dependent scales: wave path only
-  const int rb = sht::gen_rb(a->fft.N);
+  const int rb = sht::gen_rb(a->fft.N, a->JH, a->job.nfields);
   const int groups = a->job.nfields * ((a->JH + rb - 1) / rb);
   if (groups == 0) return hipSuccess;
   return sht::launch_persistent(sht::irfft_unfold_rows_kernel, groups, rb,

@@ -76,19 +76,20 @@ def test_vector_components_fold_one_at_a_time(nlon):
         assert rel_err(got, want) < tol
 
 
-@pytest.mark.parametrize("nlon", [558, 560, 698, 700, 1120, 1130, 1272, 1274])
-def test_lengths_either_side_of_a_change_of_rows_per_block(nlon):
-    """Eight rows a block up to 558 points, four from 560, eight from 700, two from
-    1130 and four from 1274; rows of several blocks and a remainder.
-    Tolerances as above."""
+@pytest.mark.parametrize("nlon,fields", [(144, 40), (576, 40), (144, 3), (640, 90), (1602, 90),
+                                         (704, 150), (1152, 90), (3072, 3), (5120, 2)])
+def test_eight_four_two_and_one_rows_per_block(nlon, fields):
+    """32 row pairs of as many fields as take 8, 8, 8, 4, 4, 2, 2, 2 and 1 rows per
+    block.  Tolerances as above."""
     from arwen_spectral import VorticityDivergenceOperator
 
-    o = OracleTransform.create(18, nlat=19, nlon=nlon, dealias_factor=1.0)
+    o = OracleTransform.create(18, nlat=63, nlon=nlon, dealias_factor=1.0)
     t = hip_transform(o, "float32")
     tol = _tol(nlon)
-    c, z, d = (red_spectrum(18, (3,), seed=s) for s in (nlon, nlon + 1, nlon + 2))
-    g32 = o.inverse(c).astype(np.float32)
-    assert rel_err(t.inverse(c), o.inverse(c)) < tol
+    c, z, d = (red_spectrum(18, (fields,), seed=s) for s in (nlon, nlon + 1, nlon + 2))
+    g = o.inverse(c)
+    g32 = g.astype(np.float32)
+    assert rel_err(t.inverse(c), g) < tol
     assert rel_err(t.forward(g32), o.forward(g32.astype(np.float64))) < tol
     v = VorticityDivergenceOperator(t)
     want = o.wind_from_vordiv(z, d)
