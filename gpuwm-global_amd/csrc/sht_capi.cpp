@@ -509,17 +509,22 @@ constexpr int kXcds = 8;  // MI355X: 8 XCDs x 32 CUs
 // by table reads and has enough of the larger tiles, else 32.  A tile reads
 // its table fragments through L1 once for its columns, so 64 halve that
 // traffic; they cost residency (two blocks per CU, not three) and padding.
-// Measured (us, 32 against 64 columns, synthesis / analysis):
-//   bf16x6  T383 160 columns 77.1/80.0 : 66.6/72.0, 256 columns 121/123 : 95/98
-//           T255 128 columns 24.7/27.6 : 22.0/25.5, 160 columns 32.1/32.5 : 30.0/34.1
-//           T383 80 columns (128 padded) 49.8/52.2 : 45.5/55.6
-//           T127 256 columns 17.0/17.5 : 16.6/19.5
-//   fp32    T383 256 columns 122/125 : 106/115, 128 columns 64.4/70.5 : 58.2/72.5,
-//           160 columns 78.9/78.9 : 77.3/81.7; T255 256 columns 49.5/54.4 : 43.0/54.1
-// so: tables from half of the eight 4 MB L2s up; in the split modes at most a
-// quarter of padding and as many tiles as run together (512), or in synthesis
-// more padding and twice the tiles; in FP32, whose MFMA time weighs more,
-// hardly any padding and two (synthesis) or four times as many tiles.
+// They also come in generations of 512, which a launch of few does not fill.
+// A call, us, 32 against 64 columns (64-column items, padding to whole tiles):
+//   bf16x6 synthesis  T383 wind 40 levels (1692, 1.2) 204 : 195, 32 (1128, 1)
+//     168 : 162, 16 (564, 1) 101 : 102; T255 gradients of 40 fields on 768
+//     longitudes (1536, 1.6) 99.3 : 97.3, on 512 (1024, 1.6) 60.8 : 65.2
+//   bf16x6 analysis   T383 vorticity, divergence 40 levels (1122, 1.2) 204 : 194,
+//     24 (748, 1.33) 144 : 136; T255 40 levels on 768 longitudes (555, 1.2)
+//     141 : 145, on 512 91.9 : 97.1, 64 on 768 (740, 1) 207 : 196
+//   fp32 synthesis    T383 gradients of 32 fields (1152, 1) 112 : 107, of 40
+//     (2304, 1.6) 148 : 156; T255 wind 64 levels on 768 longitudes (1536, 1)
+//     162 : 155, on 512 (1024, 1) 101 : 103
+//   fp32 analysis     T383 64 fields (774, 1) 118 : 118, 128 125 : 115 (kernel)
+// so: tables from half of the eight 4 MB L2s up; in the split modes about as many
+// items as run together with little or no padding, and more than two generations
+// (synthesis) or 700 items with more of it; in FP32, whose MFMA time weighs more,
+// more than two or four generations and hardly any padding.
 int default_cols(int dir, const std::vector<HostGroup>& groups, int precision) {
   const bool split = precision != ARWEN_SHT_FP32;
   long long tiles = 0, used = 0, wide = 0, table = 0;
@@ -535,9 +540,11 @@ int default_cols(int dir, const std::vector<HostGroup>& groups, int precision) {
       for (int z = 0; z < g.mcount; ++z)
         table += (long long)g.K[sg][z] * g.Arows[sg][z] * (long long)g.esz * pieces;
   }
-  const bool fits = split ? (4 * wide <= 5 * used && tiles >= 512) ||
-                                (dir == 0 && 5 * wide <= 8 * used && tiles >= 1024)
-                          : 10 * wide <= 11 * used && tiles >= (dir == 0 ? 1024 : 2048);
+  const bool fits = !split     ? 10 * wide <= 11 * used && tiles > (dir == 0 ? 1024 : 2047)
+                    : dir == 0 ? (4 * wide <= 5 * used && tiles >= 512) ||
+                                     (10 * wide <= 16 * used && tiles > 1024)
+                               : (20 * wide <= 21 * used && tiles >= 400) ||
+                                     (3 * wide <= 4 * used && tiles >= 700);
   return fits && table >= (16ll << 20) ? 64 : 32;
 }
 
