@@ -25,6 +25,14 @@ SPECTRAL_SOURCES = {"u": ("vorticity", "divergence"), "v": ("vorticity", "diverg
                     "psi": ("vorticity",), "chi": ("divergence",)}
 
 
+#: Member fields of a few MiB are launch-bound one by one: together they take a
+#: few launches (T127, 16 members, 80 fields of 5 MiB: 479 -> 230 us; T213, 20
+#: fields of 15 MiB: 133 us one by one, 145 together).
+_TOGETHER_BYTES = 8 << 20
+#: device copies of host (or converted) fields that wait to go together
+_HELD_BYTES = 32 << 20
+
+
 def _member_field(member, name):
     """A spectral field of a member: a mapping, a state, or a state with an
     ``atmosphere`` (the reference's ``ArwenGlobalState``)."""
@@ -98,23 +106,39 @@ class EnsembleSynthesis:
         members = list(members)
         if len(members) != self.members:
             raise ValueError(f"expected {self.members} members, got {len(members)}")
-        into, out_of = [], []
+        torch = self.transform.backend.xp
+        into, out_of, held = [], [], 0
+        slots = []  # per field: name, views per member, shape and bytes of one
+        for s, buf in self.inputs.items():
+            views = buf.unbind(0)
+            nbytes = views[0].numel() * views[0].element_size()
+            slots.append((s, views, views[0].shape, nbytes))
+
+        def flush():
+            nonlocal held
+            if into:
+                torch._foreach_copy_(into, out_of)
+            into.clear()
+            out_of.clear()
+            held = 0
+
         for k, member in enumerate(members):
-            for s, buf in self.inputs.items():
-                src = self.transform._spectral_tensor(_member_field(member, s))
-                if tuple(src.shape) != tuple(buf.shape[1:]):
+            for s, views, shape, nbytes in slots:
+                field = _member_field(member, s)
+                src = self.transform._spectral_tensor(field)
+                if src.shape != shape:
                     raise ValueError(f"member {k} field {s} has shape {tuple(src.shape)}, "
-                                     f"expected {tuple(buf.shape[1:])}")
-                into.append(buf[k])
+                                     f"expected {tuple(shape)}")
+                if nbytes > _TOGETHER_BYTES:
+                    views[k].copy_(src)
+                    continue
+                into.append(views[k])
                 out_of.append(src)
-        # fields of a few MiB are launch-bound one by one: together they take a
-        # few launches (T127, 16 members, 80 fields of 5 MiB: 479 -> 230 us;
-        # T213, 20 fields of 15 MiB: 133 us one by one, 145 together)
-        if max(t.numel() * t.element_size() for t in into) <= 8 << 20:
-            self.transform.backend.xp._foreach_copy_(into, out_of)
-        else:
-            for buf, src in zip(into, out_of):
-                buf.copy_(src)
+                if src is not field:  # a device copy of our own
+                    held += nbytes
+                    if held > _HELD_BYTES:
+                        flush()
+        flush()
 
     def run(self, *, graph: bool = False) -> dict:
         """Synthesize every member's grid fields; ``graph`` replays the batch

@@ -118,3 +118,34 @@ def test_state_objects_graph_replays_and_refusals(oracle):
         ens.load(states[:2])
     with pytest.raises(ValueError, match="unknown grid fields"):
         EnsembleSynthesis(tr, R, L, names=("w",))
+
+
+def test_load_holds_few_copies_of_host_members():
+    """Host members pass through the device a few fields at a time: no more
+    than the fields that wait together and the one being converted (complex128
+    first, so three times its bytes) are live beside the inputs."""
+    import torch
+
+    from arwen_spectral import EnsembleSynthesis
+    from arwen_spectral.ensemble import _HELD_BYTES, _TOGETHER_BYTES
+
+    o = OracleTransform.create(63, dealias_factor=1.0)
+    tr = hip_transform(o, "float32")
+    rng = np.random.default_rng(0)
+    for R, L in ((30, 60), (4, 300)):  # fields of 1.9 MiB and, one by one, 9.4 MiB
+        ens = EnsembleSynthesis(tr, R, L, ("theta", "qv"))
+        x = rng.standard_normal((L, 64, 64)) + 1j * rng.standard_normal((L, 64, 64))
+        members = [{"theta": x + k, "qv": x - k} for k in range(R)]
+        field = L * 64 * 64 * 8
+        assert 2 * R * field > 2 * (_HELD_BYTES + 4 * field) or field > _TOGETHER_BYTES
+        ens.load(members)  # the caching allocator's blocks exist
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        ens.load(members)
+        waiting = _HELD_BYTES + field if field <= _TOGETHER_BYTES else field
+        assert torch.cuda.max_memory_allocated() - before <= waiting + 3 * field + (4 << 20)
+        for k in (0, R // 2, R - 1):
+            for name, sign in (("theta", 1), ("qv", -1)):
+                assert np.array_equal(_np(ens.inputs[name][k]),
+                                      (x + sign * k).astype(np.complex64))
