@@ -12,6 +12,8 @@ replayable as a hipGraph.  The inverse Laplacian is fused into the pack.
 """
 from __future__ import annotations
 
+from bisect import bisect_right
+
 from .batch import TransformBatch
 from .transform import SphericalHarmonicTransform
 
@@ -109,10 +111,13 @@ class EnsembleSynthesis:
         torch = self.transform.backend.xp
         into, out_of, held = [], [], 0
         slots = []  # per field: name, views per member, shape and bytes of one
+        own = []    # first and past-the-end addresses of the inputs, in order
         for s, buf in self.inputs.items():
             views = buf.unbind(0)
             nbytes = views[0].numel() * views[0].element_size()
             slots.append((s, views, views[0].shape, nbytes))
+            own += (buf.data_ptr(), buf.data_ptr() + nbytes * self.members)
+        own.sort()
 
         def flush():
             nonlocal held
@@ -125,11 +130,15 @@ class EnsembleSynthesis:
         for k, member in enumerate(members):
             for s, views, shape, nbytes in slots:
                 field = _member_field(member, s)
+                # a view of the inputs themselves is copied in the order given
+                mine = isinstance(field, torch.Tensor) and bisect_right(own, field.data_ptr()) % 2
+                if mine:
+                    flush()
                 src = self.transform._spectral_tensor(field)
                 if src.shape != shape:
                     raise ValueError(f"member {k} field {s} has shape {tuple(src.shape)}, "
                                      f"expected {tuple(shape)}")
-                if nbytes > _TOGETHER_BYTES:
+                if mine or nbytes > _TOGETHER_BYTES:
                     views[k].copy_(src)
                     continue
                 into.append(views[k])

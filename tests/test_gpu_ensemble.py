@@ -149,3 +149,41 @@ def test_load_holds_few_copies_of_host_members():
             for name, sign in (("theta", 1), ("qv", -1)):
                 assert np.array_equal(_np(ens.inputs[name][k]),
                                       (x + sign * k).astype(np.complex64))
+
+
+def test_load_from_the_inputs_themselves_keeps_the_members_order():
+    """Members given as views of the stacked inputs are copied one after the
+    other: a shift by one member, and a later member that reads an earlier one."""
+    import torch
+
+    from arwen_spectral import EnsembleSynthesis
+
+    o = OracleTransform.create(31, dealias_factor=1.0)
+    tr = hip_transform(o, "float32")
+    R, L = 6, 40
+    ens = EnsembleSynthesis(tr, R, L, ("theta", "lnps"))
+    gen = torch.Generator(device="cuda").manual_seed(3)
+
+    def fresh(like):
+        return torch.view_as_complex(torch.randn((*like.shape, 2), generator=gen, device="cuda"))
+
+    names = {"theta": "theta", "log_surface_pressure": "log_surface_pressure"}
+    for trial in range(3):
+        for t in ens.inputs.values():
+            t.copy_(fresh(t))
+        new = {s: fresh(ens.inputs[s][0]) for s in names}
+        for source in (lambda t, k: t[k + 1] if k + 1 < R else None,       # forward shift
+                       lambda t, k: t[R - 1 - k],                          # reversal in place
+                       lambda t, k: t[0].mT if k else None):               # a strided view
+            want = {s: ens.inputs[s].clone() for s in names}
+            for s in names:
+                for k in range(R):  # one after the other
+                    src = source(want[s], k)
+                    want[s][k].copy_(new[s] if src is None else src)
+            members = []
+            for k in range(R):
+                members.append({s: new[s] if source(ens.inputs[s], k) is None
+                                else source(ens.inputs[s], k) for s in names})
+            ens.load(members)
+            for s in names:
+                assert torch.equal(ens.inputs[s], want[s])
