@@ -75,3 +75,27 @@ def test_few_field_analysis_row_tiles(T, nlat, nlon, counts, precision):
         out = torch.full((n, T + 1, T + 1), 7.0, device="cuda", dtype=torch.complex64)
         TransformBatch([("forward", t, f, out)]).run()
         assert torch.equal(t.forward(f), out), f"T{T} {n} fields"
+
+
+@pytest.mark.parametrize("precision", ["float32", "bf16x6", "bf16x3"])
+@pytest.mark.parametrize("T,nlat,nlon,counts", [(21, 33, 66, (1, 9, 72)), (64, 65, 192, (2, 13)),
+                                                (127, 128, 256, (1, 12, 18, 19))])
+def test_inverse_laplacian_has_the_grouped_bits(T, nlat, nlon, counts, precision):
+    """The C entry point's inverse Laplacian flag on a single synthesis (few
+    fields) against the batch job's."""
+    import ctypes
+
+    import torch
+
+    from arwen_spectral import SphericalHarmonicTransform, TransformBatch, _native
+
+    t = SphericalHarmonicTransform.create(T, nlat=nlat, nlon=nlon, dealias_factor=1.0,
+                                          precision=precision)
+    lib, vp = _native.load(), lambda x: ctypes.c_void_p(x.data_ptr())
+    for n in counts:
+        c = _red(torch, T, n, T + n)
+        want, got = (torch.empty(n, nlat, nlon, device="cuda") for _ in range(2))
+        TransformBatch([("inverse", t, c, want, {"inverse_laplacian": True})]).run()
+        _native.check(lib.arwen_sht_synthesis_about(t.plan_handle, vp(c), vp(got), n, None,
+                                                    _native.JOB_INVLAP, t.backend.stream()))
+        assert torch.equal(got, want), f"T{T} {n} fields"
