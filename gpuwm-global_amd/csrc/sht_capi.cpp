@@ -1204,6 +1204,34 @@ void bind_jobs(arwen_sht_batch* B) {
   for (auto& js : B->jobs) setup_job(B, js.get(), false);
 }
 
+// What a job may hold, whatever its plan.
+void check_job(const arwen_sht_job& J, int j) {
+  if (J.count < 0) fail(ARWEN_SHT_EINVAL, "job count must be >= 0");
+  const bool vec = J.op == ARWEN_SHT_OP_UV_FROM_VORDIV || J.op == ARWEN_SHT_OP_VORDIV_FROM_UV ||
+                   J.op == ARWEN_SHT_OP_VORDIV_FROM_WAIST;
+  const bool sgrad = J.op == ARWEN_SHT_OP_SYNTHESIS_GRADIENT;
+  const bool two_out = vec || J.op == ARWEN_SHT_OP_GRADIENT || sgrad;
+  const bool two_in = vec || J.op == ARWEN_SHT_OP_DIVERGENCE_FROM_WAIST;
+  if (J.op < ARWEN_SHT_OP_SYNTHESIS || J.op > ARWEN_SHT_OP_DIVERGENCE_FROM_WAIST)
+    fail(ARWEN_SHT_EINVAL, "unknown op " + std::to_string(J.op));
+  if (J.count > 0 && (!J.in0 || !J.out0 || (two_in && !J.in1) || (two_out && !J.out1) ||
+                      (sgrad && !J.out2)))
+    fail(ARWEN_SHT_EINVAL, "job " + std::to_string(j) + " is missing a buffer");
+  if (J.flags & ~(ARWEN_SHT_JOB_EXP | ARWEN_SHT_JOB_INVLAP))
+    fail(ARWEN_SHT_EINVAL, "job " + std::to_string(j) + " has unknown flags");
+  if ((J.flags & ARWEN_SHT_JOB_EXP) && J.op != ARWEN_SHT_OP_SYNTHESIS)
+    fail(ARWEN_SHT_EINVAL, "ARWEN_SHT_JOB_EXP applies to ARWEN_SHT_OP_SYNTHESIS only");
+  if ((J.flags & ARWEN_SHT_JOB_INVLAP) && (J.op != ARWEN_SHT_OP_SYNTHESIS || J.coeff_offset))
+    fail(ARWEN_SHT_EINVAL,
+         "ARWEN_SHT_JOB_INVLAP applies to ARWEN_SHT_OP_SYNTHESIS without a coeff_offset");
+  if (J.grid_offset && J.op != ARWEN_SHT_OP_ANALYSIS)
+    fail(ARWEN_SHT_EINVAL, "grid_offset applies to ARWEN_SHT_OP_ANALYSIS only");
+  if (J.coeff_offset && J.op != ARWEN_SHT_OP_ANALYSIS && J.op != ARWEN_SHT_OP_SYNTHESIS &&
+      !sgrad)
+    fail(ARWEN_SHT_EINVAL,
+         "coeff_offset applies to ARWEN_SHT_OP_ANALYSIS, _SYNTHESIS and _SYNTHESIS_GRADIENT only");
+}
+
 void plan_batch(arwen_sht_batch* B, const arwen_sht_job* jobs, int njobs) {
   if (njobs <= 0 || !jobs) fail(ARWEN_SHT_EINVAL, "a batch needs at least one job");
   hip_check(hipGetDevice(&B->device), "hipGetDevice");
@@ -1216,30 +1244,7 @@ void plan_batch(arwen_sht_batch* B, const arwen_sht_job* jobs, int njobs) {
       fail(ARWEN_SHT_EINVAL, "all plans of a batch must share one precision");
     if (P->device != B->device)
       fail(ARWEN_SHT_EINVAL, "job " + std::to_string(j) + "'s plan belongs to another device");
-    if (J.count < 0) fail(ARWEN_SHT_EINVAL, "job count must be >= 0");
-    const bool vec = J.op == ARWEN_SHT_OP_UV_FROM_VORDIV || J.op == ARWEN_SHT_OP_VORDIV_FROM_UV ||
-                     J.op == ARWEN_SHT_OP_VORDIV_FROM_WAIST;
-    const bool sgrad = J.op == ARWEN_SHT_OP_SYNTHESIS_GRADIENT;
-    const bool two_out = vec || J.op == ARWEN_SHT_OP_GRADIENT || sgrad;
-    const bool two_in = vec || J.op == ARWEN_SHT_OP_DIVERGENCE_FROM_WAIST;
-    if (J.op < ARWEN_SHT_OP_SYNTHESIS || J.op > ARWEN_SHT_OP_DIVERGENCE_FROM_WAIST)
-      fail(ARWEN_SHT_EINVAL, "unknown op " + std::to_string(J.op));
-    if (J.count > 0 && (!J.in0 || !J.out0 || (two_in && !J.in1) || (two_out && !J.out1) ||
-                        (sgrad && !J.out2)))
-      fail(ARWEN_SHT_EINVAL, "job " + std::to_string(j) + " is missing a buffer");
-    if (J.flags & ~(ARWEN_SHT_JOB_EXP | ARWEN_SHT_JOB_INVLAP))
-      fail(ARWEN_SHT_EINVAL, "job " + std::to_string(j) + " has unknown flags");
-    if ((J.flags & ARWEN_SHT_JOB_EXP) && J.op != ARWEN_SHT_OP_SYNTHESIS)
-      fail(ARWEN_SHT_EINVAL, "ARWEN_SHT_JOB_EXP applies to ARWEN_SHT_OP_SYNTHESIS only");
-    if ((J.flags & ARWEN_SHT_JOB_INVLAP) && (J.op != ARWEN_SHT_OP_SYNTHESIS || J.coeff_offset))
-      fail(ARWEN_SHT_EINVAL,
-           "ARWEN_SHT_JOB_INVLAP applies to ARWEN_SHT_OP_SYNTHESIS without a coeff_offset");
-    if (J.grid_offset && J.op != ARWEN_SHT_OP_ANALYSIS)
-      fail(ARWEN_SHT_EINVAL, "grid_offset applies to ARWEN_SHT_OP_ANALYSIS only");
-    if (J.coeff_offset && J.op != ARWEN_SHT_OP_ANALYSIS && J.op != ARWEN_SHT_OP_SYNTHESIS &&
-        !sgrad)
-      fail(ARWEN_SHT_EINVAL,
-           "coeff_offset applies to ARWEN_SHT_OP_ANALYSIS, _SYNTHESIS and _SYNTHESIS_GRADIENT only");
+    check_job(J, j);
     auto js = std::make_unique<JobState>();
     js->job = J;
     setup_job(B, js.get(), true);
@@ -1371,6 +1376,7 @@ int single_job(arwen_sht_plan* P, const arwen_sht_job& job, void* stream) {
     const int op = job.op, count = job.count;
     if (count < 0) fail(ARWEN_SHT_EINVAL, "count must be >= 0");
     if (count == 0) return;
+    check_job(job, 0);  // every call: a kept batch takes this one's buffers and flags
     std::lock_guard<std::mutex> lock(P->cache_mu);
     const auto key = std::make_tuple(op, count, stream);
     arwen_sht_batch* B = nullptr;

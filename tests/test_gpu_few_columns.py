@@ -99,3 +99,30 @@ def test_inverse_laplacian_has_the_grouped_bits(T, nlat, nlon, counts, precision
         _native.check(lib.arwen_sht_synthesis_about(t.plan_handle, vp(c), vp(got), n, None,
                                                     _native.JOB_INVLAP, t.backend.stream()))
         assert torch.equal(got, want), f"T{T} {n} fields"
+
+
+def test_a_later_single_operation_is_checked_like_the_first():
+    """The batch kept for an operation takes every call's buffers and flags:
+    what the first call refuses, the next one refuses too."""
+    import ctypes
+
+    import torch
+
+    from arwen_spectral import SphericalHarmonicTransform, _native
+
+    t = SphericalHarmonicTransform.create(21, dealias_factor=1.0)
+    lib = _native.load()
+    c = _red(torch, 21, 2, 1)
+    out = torch.empty(2, *t.grid.shape, device="cuda")
+    off = torch.ones(2, dtype=torch.complex64, device="cuda")
+    vp, s = lambda x: ctypes.c_void_p(x.data_ptr()), t.backend.stream()
+    call = lib.arwen_sht_synthesis_about
+    for _ in range(2):
+        assert call(t.plan_handle, vp(c), vp(out), 2, None, 0, s) == _native.OK
+        assert call(t.plan_handle, None, vp(out), 2, None, 0, s) == _native.EINVAL
+        assert call(t.plan_handle, vp(c), None, 2, None, 0, s) == _native.EINVAL
+        assert call(t.plan_handle, vp(c), vp(out), 2, None, 4, s) == _native.EINVAL
+        assert call(t.plan_handle, vp(c), vp(out), 2, vp(off), _native.JOB_INVLAP,
+                    s) == _native.EINVAL
+        assert call(t.plan_handle, vp(c), vp(out), 2, vp(off), _native.JOB_EXP, s) == _native.OK
+    torch.cuda.synchronize()
