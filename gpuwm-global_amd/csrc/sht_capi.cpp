@@ -687,8 +687,10 @@ void build_lists(int dir, const std::vector<HostGroup>& groups, int bn, int slot
   std::vector<sht::GemmItem> t(longest * queues.size());  // zero = none
   for (size_t b = 0; b < queues.size(); ++b)
     for (size_t k = 0; k < queues[b].size(); ++k) t[k * queues.size() + b] = queues[b][k];
-  // the kernel addresses the lists with 32-bit byte offsets
-  if (std::max(steps.size(), t.size()) >= (size_t(1) << 32) / sizeof(sht::GemmStep))
+  // the kernel addresses the lists with 32-bit byte offsets, the items up to
+  // four of a queue ahead (past the list: none)
+  if (std::max(steps.size(), t.size() + 4 * queues.size()) >=
+      (size_t(1) << 32) / sizeof(sht::GemmStep))
     fail(ARWEN_SHT_EINVAL, "too many operations for one GEMM work list");
   upload(out.panels, panels);
   upload(out.steps, steps);
