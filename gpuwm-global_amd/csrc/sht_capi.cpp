@@ -89,6 +89,10 @@ struct DevBuf {
     p = nullptr;
     bytes = 0;
   }
+  void swap(DevBuf& o) {
+    std::swap(p, o.p);
+    std::swap(bytes, o.bytes);
+  }
   ~DevBuf() { release(); }
   DevBuf(const DevBuf&) = delete;
   DevBuf& operator=(const DevBuf&) = delete;
@@ -443,6 +447,16 @@ struct GemmLists {
   int bn = 0;
   int slots = 0;  // the grid asked for
   int grid = 0;   // workgroups launched (at most `slots`)
+  void swap(GemmLists& o) {
+    panels.swap(o.panels);
+    steps.swap(o.steps);
+    items.swap(o.items);
+    std::swap(nitems, o.nitems);
+    std::swap(nsteps, o.nsteps);
+    std::swap(bn, o.bn);
+    std::swap(slots, o.slots);
+    std::swap(grid, o.grid);
+  }
 };
 
 struct JobState {
@@ -1355,9 +1369,16 @@ void apply_config(arwen_sht_batch* B, const arwen_sht_gemm_config& c) {
   // the lists are rebuilt while no launch of this batch is in flight
   hip_check(hipDeviceSynchronize(), "config change");
   drop_graph(B);
+  // both are there before either replaces the old ones: a failure leaves the
+  // batch as it was
+  GemmLists fresh[2];
+  bool change[2];
+  for (int d = 0; d < 2; ++d) {
+    change[d] = B->lists[d].bn != c.cols[d] || B->lists[d].slots != gemm_slots(c, d);
+    if (change[d]) build_lists(d, B->groups[d], c.cols[d], gemm_slots(c, d), fresh[d]);
+  }
   for (int d = 0; d < 2; ++d)
-    if (B->lists[d].bn != c.cols[d] || B->lists[d].slots != gemm_slots(c, d))
-      build_lists(d, B->groups[d], c.cols[d], gemm_slots(c, d), B->lists[d]);
+    if (change[d]) B->lists[d].swap(fresh[d]);
   B->config = c;
   hip_check(hipDeviceSynchronize(), "config upload");
 }
@@ -1686,10 +1707,8 @@ void build_sample_tables(arwen_sht_plan* P) {
   DevBuf r, dg;
   upload(r, rec);
   upload(dg, diag);
-  std::swap(P->sample_rec.p, r.p);
-  std::swap(P->sample_rec.bytes, r.bytes);
-  std::swap(P->sample_diag.p, dg.p);
-  std::swap(P->sample_diag.bytes, dg.bytes);
+  P->sample_rec.swap(r);
+  P->sample_diag.swap(dg);
 }
 }  // namespace
 
