@@ -22,9 +22,17 @@
 // for all loads at once.  Here a coefficient is loaded once per lane for PT
 // MFMAs and a basis value feeds CT.  T383, 30,000 points: 40 fields 11.25 ->
 // 7.10 ms in float64 (51 TFLOP/s; 62 is what a large FP64 matrix product
-// reaches), 9.18 -> 4.74 ms in float32 (bound by the FP64 recurrence); their
-// gradients 19.9 -> 19.1 and 19.5 -> 14.5 ms (the derivative's recurrence
-// runs beside two MFMAs a value); 3 fields at 300 points 2.84 -> 0.73 ms.
+// reaches), 9.18 -> 4.74 ms in float32 (bound by the FP64 recurrence); 3 fields
+// at 300 points 2.84 -> 0.73 ms.
+// Gradients and winds run the derivative's recurrence beside two MFMAs a value
+// (nine FP64 operations, not four), so there it counts as much: lanes that
+// share a point form the derivative of one degree each, the last odd column
+// tile runs alone, and one column tile of many points takes four point tiles,
+// whose lanes share no point.  Gradients, T383, 30,000 points, former kernel ->
+// every lane all derivatives and no tile alone -> here: 40 fields float64 19.9
+// -> 19.2 -> 16.1 ms, float32 19.6 -> 14.4 -> 12.1; 8 fields float64 4.26 ->
+// 4.76 -> 3.86; T127, 20 fields 1.40 -> 1.61 -> 1.31, 8 fields 0.51 -> 0.62 ->
+// 0.53.
 //
 // Precision: F32 = false accumulates in FP64; F32 = true rounds each basis
 // value to fp32 and accumulates an order's terms in fp32 before the FP64 sum
@@ -129,29 +137,34 @@ __device__ __forceinline__ void sample_store(int col, int p, int npts, int nout,
 // MFMA operands: lane l = (g = l / 16, q = l % 16); A holds point q of the
 // tile at degree n0 + g, B degree n0 + g at column q; accumulator register i
 // is point g + 4 i (FP64) or 4 g + i (fp32) at column q.
+template <int PT, int KIND, bool F32>
+struct SampleShared {
+  static constexpr int NP = 16 * PT;            // points of a wavefront
+  static constexpr int NB = KIND != 0 ? 2 : 1;  // bases: P, dP/dphi
+  // per wavefront: basis values [2 buffers][P, dP][degree][point], then
+  // cos and sin of the order's phase per point
+  typename SampleAcc<F32>::T A[4][2][NB][4][NP];
+  double E[4][2][NP];
+};
+
 template <int PT, int CT, int KIND, bool F32>
-__global__ void __launch_bounds__(256, 2) sample_kernel(
+__device__ __forceinline__ void sample_tiles(
+    SampleShared<PT, KIND, F32>& sh, int ct0,
     const typename SampleAcc<F32>::T* __restrict__ coef, const double* __restrict__ rec,
     const double* __restrict__ diag, const double* __restrict__ sin_lat,
-    const double* __restrict__ cos_lat, const double* __restrict__ lon, SampleCuts cuts, int T,
-    int npts, int ldc, int nout, double radius, double* __restrict__ out0,
+    const double* __restrict__ cos_lat, const double* __restrict__ lon, const SampleCuts& cuts,
+    int T, int npts, int ldc, int nout, double radius, double* __restrict__ out0,
     double* __restrict__ out1, double* __restrict__ partial) {
   using Acc = typename SampleAcc<F32>::T;
   using D = typename SampleAcc<F32>::D;
   constexpr bool GRAD = KIND != 0;
-  constexpr int NP = 16 * PT;              // points of this wavefront
-  constexpr int NB = GRAD ? 2 : 1;         // bases: P, dP/dphi
-  // per wavefront: basis values [2 buffers][P, dP][degree][point], then
-  // cos and sin of the order's phase per point
-  __shared__ Acc sA[4][2][NB][4][NP];
-  __shared__ double sE[4][2][NP];
+  constexpr int NP = 16 * PT, NB = GRAD ? 2 : 1;
+  auto& sA = sh.A;
+  auto& sE = sh.E;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int g = lane >> 4, q = lane & 15;
   const int p0 = ((int)blockIdx.x * 4 + wv) * NP;
   if (p0 >= npts) return;  // wave-uniform; no block barrier in this kernel
-  // the last group of column tiles starts early enough to be whole: its first
-  // tiles may be another group's too, with the same bits
-  const int ct0 = min((int)blockIdx.y * CT, ldc / 8 - CT);
   const int r = blockIdx.z;
   const int m0 = cuts.m[r], m1 = cuts.m[r + 1];
   const long long K = (long long)(T + 1) * (T + 2) / 2;
@@ -209,45 +222,53 @@ __global__ void __launch_bounds__(256, 2) sample_kernel(
     // degrees m and m + 1 have their own rules; TAIL: degrees past T are 0
     auto basis = [&](auto FIRST, auto TAIL, int j, int buf) {
       constexpr bool first = decltype(FIRST)::value, tail = decltype(TAIL)::value;
-      double P[4], dP[4];
-      double ra[4], rb[4], rc[4];
+      // the lanes that share a point form its four values of P each, and
+      // between them those of dP and the LDS writes
+      constexpr int SHARE = 64 / NP, EACH = 4 / SHARE;
+      const int part = lane / NP;
+      double P[4], rc[EACH];
+      double ra[4], rb[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         const long long k = k0 + (tail ? min(j + u, len - 1) : j + u);
         ra[u] = rec_a[k];
         rb[u] = rec_b[k];
-        rc[u] = GRAD ? rec_c[k] : 0.0;
       }
+      if constexpr (GRAD)
+#pragma unroll
+        for (int e = 0; e < EACH; ++e) {
+          const int u = (SHARE > 1 ? part * EACH : 0) + e;
+          rc[e] = rec_c[k0 + (tail ? min(j + u, len - 1) : j + u)];
+        }
+      double below = prev;  // P one degree below this lane's first
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         double v;
         if (first && u == 0) v = dg;
         else if (first && u == 1) v = diag_g[m] * x * dg;
         else v = ra[u] * (x * prev - rb[u] * prev2);
-        double d = 0.0;
-        if constexpr (GRAD) {
-          const double nn = (double)(m + j + u);
-          if (first && u == 0) d = m >= 1 ? rd * (nn * x * dg) : 0.0;
-          else d = rd * (nn * x * v - rc[u] * prev);
-        }
+        if constexpr (GRAD)
+          if (u > 0 && u % EACH == 0) below = part * EACH == u ? prev : below;
         prev2 = prev;
         prev = v;
         P[u] = tail && j + u >= len ? 0.0 : v;
-        dP[u] = tail && j + u >= len ? 0.0 : d;
       }
-      // the lanes that share a point write its four degrees between them
-      constexpr int SHARE = 64 / NP, EACH = 4 / SHARE;
-      const int part = lane / NP;
 #pragma unroll
       for (int e = 0; e < EACH; ++e) {
-        double v = P[e], d = dP[e];
+        double v = P[e];
 #pragma unroll
-        for (int h = 1; h < SHARE; ++h) {
-          v = part == h ? P[h * EACH + e] : v;
-          d = part == h ? dP[h * EACH + e] : d;
-        }
+        for (int h = 1; h < SHARE; ++h) v = part == h ? P[h * EACH + e] : v;
         sA[wv][buf][0][part * EACH + e][mine] = (Acc)v;
-        if constexpr (GRAD) sA[wv][buf][NB - 1][part * EACH + e][mine] = (Acc)d;
+        if constexpr (GRAD) {
+          // at degree m the second term is 0 (rec_c and P below); past T the
+          // basis value is 0 and so is the derivative
+          const int u = (SHARE > 1 ? part * EACH : 0) + e;
+          double d = rd * ((double)(m + j + u) * x * v - rc[e] * below);
+          if (first && u == 0 && m == 0) d = 0.0;
+          if (tail) d = j + u < len ? d : 0.0;
+          sA[wv][buf][NB - 1][part * EACH + e][mine] = (Acc)d;
+          below = v;
+        }
       }
     };
     auto lds_sync = [] {  // this wavefront's LDS accesses, in order
@@ -367,6 +388,28 @@ __global__ void __launch_bounds__(256, 2) sample_kernel(
       }
 }
 
+template <int PT, int CT, int KIND, bool F32>
+__global__ void __launch_bounds__(256, 2) sample_kernel(
+    const typename SampleAcc<F32>::T* __restrict__ coef, const double* __restrict__ rec,
+    const double* __restrict__ diag, const double* __restrict__ sin_lat,
+    const double* __restrict__ cos_lat, const double* __restrict__ lon, SampleCuts cuts, int T,
+    int npts, int ldc, int nout, double radius, double* __restrict__ out0,
+    double* __restrict__ out1, double* __restrict__ partial) {
+  __shared__ SampleShared<PT, KIND, F32> sh;
+  const int tiles = ldc / 8, ct0 = (int)blockIdx.y * CT;
+  if constexpr (KIND != 0 && CT == 2) {
+    if (ct0 + CT > tiles) {  // block-uniform: one tile is left
+      sample_tiles<PT, 1, KIND, F32>(sh, ct0, coef, rec, diag, sin_lat, cos_lat, lon, cuts, T,
+                                     npts, ldc, nout, radius, out0, out1, partial);
+      return;
+    }
+  }
+  // the last group of column tiles starts early enough to be whole: its first
+  // tiles may be another group's too, with the same bits
+  sample_tiles<PT, CT, KIND, F32>(sh, min(ct0, tiles - CT), coef, rec, diag, sin_lat, cos_lat, lon,
+                                  cuts, T, npts, ldc, nout, radius, out0, out1, partial);
+}
+
 // Adds the R parts' sums of each (column, point) in part order and stores
 // the outputs; one thread per (column or column pair, point).
 template <int KIND>
@@ -427,8 +470,9 @@ hipError_t launch_sample_tile(const sht::SampleArgs& a, hipStream_t s) {
 // registers of two wavefronts per SIMD hold (five for values, two for the two
 // bases of gradients and winds) feed the most MFMAs per basis value and
 // coefficient; fewer points or columns take smaller tiles, so that the launch
-// still has a wavefront for each of the chip's 1024 SIMDs.  ct is the even
-// share of the column tiles between the groups, so it is never above their
+// still has a wavefront for each of the chip's 1024 SIMDs.  One column tile of
+// derivatives takes four point tiles from two wavefronts per SIMD up.  ct is the
+// even share of the column tiles between the groups, so it is never above their
 // number: a group wider than all of them would begin at a negative column.
 struct SampleTile {
   int pt, ct;
@@ -439,6 +483,8 @@ SampleTile sample_tile(int kind, int ldc, int npts, int parts) {
   const int ct = (int)((tiles + groups - 1) / groups);
   const long long waves2 = ((long long)npts + 31) / 32 * groups * parts;
   const long long waves1 = ((long long)npts + 15) / 16 * groups * parts;
+  const long long waves4 = ((long long)npts + 63) / 64 * groups * parts;
+  if (kind != 0 && ct == 1 && waves4 >= 2048) return {4, 1};
   if (waves2 >= 2048 || (waves2 >= 1024 && ct >= 2)) return {2, ct};
   if (waves1 >= 1024 && ct >= 2) return {1, ct};
   return {1, 1};
@@ -460,6 +506,8 @@ hipError_t launch_sample_kind(const sht::SampleArgs& a, hipStream_t s) {
     SHT_TILE(2, 3);
     SHT_TILE(2, 4);
     SHT_TILE(2, 5);
+  } else {
+    SHT_TILE(4, 1);
   }
 #undef SHT_TILE
   return hipErrorInvalidValue;

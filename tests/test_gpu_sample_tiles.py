@@ -128,3 +128,32 @@ def test_two_to_five_column_tiles_of_one_point_tile(T, points, precision):
     assert np.max(np.abs(tiles[:, some].cpu().numpy() - want)) < tol * np.max(np.abs(want))
     for count in (17, 24, 25, 32, 33):
         assert torch.equal(call(fields[:count]), tiles[:count]), count
+
+
+@pytest.mark.parametrize("T,points,count", [(127, 16400, 3), (127, 16321, 8), (127, 4100, 20),
+                                            (31, 33000, 17), (21, 131080, 1)])
+@pytest.mark.parametrize("kind", ["gradient", "wind"])
+@pytest.mark.parametrize("precision", list(TOL))
+def test_derivatives_at_many_points(T, points, count, kind, precision):
+    """Four point tiles of one column tile (orders of every remainder, points of
+    the last block missing), and a last column tile alone: the oracle's values
+    at some points, the last ones among them, and the bits of a few points
+    alone.  Tolerances as above; winds carry the fp32 rounding of psi and chi."""
+    from arwen_spectral import sampling
+
+    o = OracleTransform.create(T, dealias_factor=1.0)
+    t = hip_transform(o, "float32")
+    lat, lon = _points(points)
+    n = (count + 1) // 2 if kind == "wind" else count
+    fields = [_fields(T, n, 5), _fields(T, n, 6)][:2 if kind == "wind" else 1]
+    fn = {"gradient": (sampling.sample_gradient, osamp.sample_gradient),
+          "wind": (sampling.sample_wind, osamp.sample_wind)}[kind]
+    some = np.r_[0:16, points - 40:points]
+    got = fn[0](t, *fields, lat, lon, precision=precision)
+    want = fn[1](o, *(f.astype(np.complex128) for f in fields), lat[some], lon[some])
+    few = fn[0](t, *fields, lat[some], lon[some], precision=precision)
+    tol = max(TOL[precision], (T + 1) * 6e-8 if precision == "float32" else 0.0,
+              2e-6 if kind == "wind" else 0.0)
+    for g, w, f in zip(got, want, few):
+        assert np.max(np.abs(g[:, some] - w)) < tol * np.max(np.abs(w))
+        assert np.array_equal(g[:, some], f)
