@@ -25,6 +25,7 @@
 #include <algorithm>
 #include <map>
 #include <mutex>
+#include <tuple>
 #include <type_traits>
 #include <utility>
 
@@ -1217,10 +1218,11 @@ int wave_L(int N) {
 // device at once (registers and LDS, from the runtime's occupancy query, at
 // most 8 per CU), capped by the number of groups.  A grid larger than what is
 // resident runs its surplus blocks after the first ones finish, which leaves
-// the CUs half idle at the end.  The query is cached per (kernel, LDS size).
+// the CUs half idle at the end.  The query is cached per (kernel, threads, LDS
+// size): the row kernels run with several block sizes.
 int persistent_blocks(const void* kernel, int threads, int groups, size_t lds_bytes) {
   static std::mutex mu;
-  static std::map<std::pair<const void*, size_t>, int> cache;
+  static std::map<std::tuple<const void*, int, size_t>, int> cache;
   int dev = 0, cus = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
@@ -1229,7 +1231,7 @@ int persistent_blocks(const void* kernel, int threads, int groups, size_t lds_by
   int per_cu = 0;
   {
     std::lock_guard<std::mutex> lock(mu);
-    const auto key = std::make_pair(kernel, lds_bytes);
+    const auto key = std::make_tuple(kernel, threads, lds_bytes);
     const auto it = cache.find(key);
     if (it != cache.end()) {
       per_cu = it->second;
