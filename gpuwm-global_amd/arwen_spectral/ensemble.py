@@ -29,7 +29,9 @@ SPECTRAL_SOURCES = {"u": ("vorticity", "divergence"), "v": ("vorticity", "diverg
 
 #: Member fields of a few MiB are launch-bound one by one: together they take a
 #: few launches (T127, 16 members, 80 fields of 5 MiB: 479 -> 230 us; T213, 20
-#: fields of 15 MiB: 133 us one by one, 145 together).
+#: fields of 15 MiB: 133 us one by one, 145 together).  The largest field decides
+#: for all: beside larger ones the few small fields take one block of a joint
+#: copy each (T213, 2 members, two ln ps of 0.4 MB: 21 us together, 6 apart).
 _TOGETHER_BYTES = 8 << 20
 #: device copies of host (or converted) fields that wait to go together
 _HELD_BYTES = 32 << 20
@@ -118,6 +120,7 @@ class EnsembleSynthesis:
             slots.append((s, views, views[0].shape, nbytes))
             own += (buf.data_ptr(), buf.data_ptr() + nbytes * self.members)
         own.sort()
+        together = max(slot[3] for slot in slots) <= _TOGETHER_BYTES
 
         def flush():
             nonlocal held
@@ -138,7 +141,7 @@ class EnsembleSynthesis:
                 if src.shape != shape:
                     raise ValueError(f"member {k} field {s} has shape {tuple(src.shape)}, "
                                      f"expected {tuple(shape)}")
-                if mine or nbytes > _TOGETHER_BYTES:
+                if mine or not together:
                     views[k].copy_(src)
                     continue
                 into.append(views[k])

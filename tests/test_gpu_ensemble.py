@@ -187,3 +187,25 @@ def test_load_from_the_inputs_themselves_keeps_the_members_order():
             ens.load(members)
             for s in names:
                 assert torch.equal(ens.inputs[s], want[s])
+
+
+@pytest.mark.parametrize("L,calls", [(40, 1), (300, 0)])  # fields of 1.3 and 9.4 MiB
+def test_the_largest_field_decides_how_members_are_copied(monkeypatch, L, calls):
+    """Small members go in one joint copy; beside large fields the small ones
+    are copied one by one as well."""
+    import torch
+
+    from arwen_spectral import EnsembleSynthesis
+
+    o = OracleTransform.create(63, dealias_factor=1.0)
+    ens = EnsembleSynthesis(hip_transform(o, "float32"), 2, L, ("theta", "lnps"))
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    members = [{s: torch.randn(buf.shape[1:], generator=gen, dtype=buf.dtype, device="cuda")
+                for s, buf in ens.inputs.items()} for _ in range(2)]
+    joint, copy = [], torch._foreach_copy_
+    monkeypatch.setattr(torch, "_foreach_copy_", lambda a, b: (joint.append(len(a)), copy(a, b)))
+    ens.load(members)
+    assert len(joint) == calls
+    for k, member in enumerate(members):
+        for s, buf in ens.inputs.items():
+            assert torch.equal(buf[k], member[s])
