@@ -370,8 +370,9 @@ constexpr int fold_waves_per_simd() {
 // of a vector level together.  A group is kWaveBlock consecutive rows of one
 // field (JHP is a multiple of 32): each wavefront folds its row's spectrum
 // into registers and parks the values in its LDS span, then the block writes
-// every (column, m-tile, parity) run of RB rows x 4 orders as one piece.  Blocks are persistent: while a group is transformed, the rows of
-// the block's next group are already being loaded into registers.
+// every (column, m-tile, parity) run of RB rows x 4 orders as one piece.
+// Blocks are persistent: while a group is transformed, the rows of the block's
+// next group are already being loaded into registers.
 template <int L, int F, int kWaveBlock>
 __global__ void __launch_bounds__(64 * kWaveBlock, (fold_waves_per_simd<L, F, kWaveBlock>()))
     rfft_fold_wave_kernel(FoldArgs a) {
@@ -493,6 +494,29 @@ __global__ void __launch_bounds__(64 * kWaveBlock, (fold_waves_per_simd<L, F, kW
   }
 }
 
+// The waist runs of a row group come through bounds-checked buffer loads off
+// one descriptor (a column pair, from row i0 on): an offset is one 32-bit
+// register held across the groups, and a thread without a run reads past the
+// extent (0, no access).  Loads from pointers could have their addresses formed
+// in the loads' own result registers, and then each waited for the one before
+// it: fp32 unfold, T767, 160 fields 568 -> 450 us, T511, 40 fields 65.8 -> 58.9;
+// T383 (no such waits) 49.8 us either way.
+typedef __attribute__((ext_vector_type(4))) float f4;
+constexpr unsigned kNoRun = ~15u;
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t waist_rows(const float* column, int ldw, int i0) {
+  // uniform, but not seen as such: without this a loop over the wavefront's
+  // values surrounds every load (T383 49.3 -> 50.8 us)
+  const unsigned long long at = reinterpret_cast<unsigned long long>(column + kMT * i0);
+  const unsigned lo = __builtin_amdgcn_readfirstlane((int)at);
+  const unsigned hi = __builtin_amdgcn_readfirstlane((int)(at >> 32));
+  return __builtin_amdgcn_make_buffer_rsrc(
+      reinterpret_cast<void*>(((unsigned long long)hi << 32) | lo), 0,
+      __builtin_amdgcn_readfirstlane(8 * ldw - 4 * kMT * i0), 0x00020000);
+}
+__device__ __forceinline__ f4 load_run(__amdgpu_buffer_rsrc_t rows, unsigned off) {
+  return __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(rows, (int)off, 0, 0));
+}
+
 // Synthesis: one wavefront per (field, folded row).  A group is kWaveBlock
 // consecutive rows of one field: the block reads every (column, m-tile,
 // parity) run of RB rows x 4 orders of the waist as one piece and hands each
@@ -506,7 +530,6 @@ __global__ void __launch_bounds__(64 * kWaveBlock,
   extern __shared__ float2 lds[];
   constexpr int N = 64 * L, SP = wave_span<L>();
   static_assert(kMT == 4, "a row's four orders are one 16-byte vector");
-  typedef __attribute__((ext_vector_type(4))) float f4;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   constexpr int WS = SP + kSpanPad;  // span stride per wavefront
   float2* tw = lds;
@@ -524,7 +547,8 @@ __global__ void __launch_bounds__(64 * kWaveBlock,
   // parity; consecutive lanes take one run's rows (16 bytes each).  Where a
   // run sits relative to the group's first row, in the waist and in LDS,
   // is the same for every group, so it is worked out once:
-  //   waist  W + c ldw + 4 i0 + roff[r],  roff = (e >> 1) ldw + 4 ((2 mt + (e & 1)) JHP + ww)
+  //   waist  W + c ldw + 4 i0, and roff[r] bytes on,
+  //          roff = 4 ((e >> 1) ldw + 4 ((2 mt + (e & 1)) JHP + ww))
   //   LDS    span ww, float 4 (e MT + mt)
   // (the waist layout W[c][m/4][p][i][m%4]); rvalid bit r marks r < 4 MT.
   constexpr int RU = (4 * (N / 8 + 1) + 63) / 64;  // 4 MT <= N/2 + 4 runs
@@ -537,15 +561,16 @@ __global__ void __launch_bounds__(64 * kWaveBlock,
     const bool ok = rn < 4 * MT;
     const unsigned e = ok ? (unsigned)(rn / MT) : 0u, mt = ok ? (unsigned)(rn % MT) : 0u;
     rvalid |= (ok ? 1u : 0u) << r;
-    roff[r] = (e >> 1) * (unsigned)a.job.ldw + 4u * ((2u * mt + (e & 1u)) * (unsigned)a.JHP + ww);
+    roff[r] = 4u * ((e >> 1) * (unsigned)a.job.ldw + 4u * ((2u * mt + (e & 1u)) * (unsigned)a.JHP + ww));
+    if (!ok) roff[r] = kNoRun;
     loff[r] = (unsigned)(2 * wave_tw<L>() + 2 * ww * WS) + 4u * (e * (unsigned)MT + mt);
   }
   auto load_runs = [&](int grp) {
     const int fld = grp / JH4, i0 = (grp % JH4) * kWaveBlock;
-    const float* base = W + (size_t)(a.job.col0 + a.job.fstride * fld) * a.job.ldw + 4 * i0;
+    const __amdgpu_buffer_rsrc_t rows = waist_rows(
+        W + (size_t)(a.job.col0 + a.job.fstride * fld) * a.job.ldw, a.job.ldw, i0);
 #pragma unroll
-    for (int r = 0; r < RU; ++r)
-      if (rvalid & (1u << r)) run[r] = *reinterpret_cast<const f4*>(base + roff[r]);
+    for (int r = 0; r < RU; ++r) run[r] = load_run(rows, roff[r]);
   };
   load_runs(g);
   fill_wave_twiddles<L>(tw, a.fft.tw);
@@ -742,7 +767,6 @@ __global__ void __launch_bounds__(64 * kWaveBlock) irfft_unfold_wave64_kernel(Un
   extern __shared__ double2 lds_d[];
   constexpr int N = 64 * L, SP = wave_span<L>();
   static_assert(kMT == 4, "a row's four orders are one 16-byte vector");
-  typedef __attribute__((ext_vector_type(4))) float f4;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   constexpr int WS = SP + kSpanPad;  // span stride per wavefront, double2
   double2* tw = lds_d;
@@ -768,15 +792,16 @@ __global__ void __launch_bounds__(64 * kWaveBlock) irfft_unfold_wave64_kernel(Un
     const bool ok = rn < 4 * MT;
     const unsigned e = ok ? (unsigned)(rn / MT) : 0u, mt = ok ? (unsigned)(rn % MT) : 0u;
     rvalid |= (ok ? 1u : 0u) << r;
-    roff[r] = (e >> 1) * (unsigned)a.job.ldw + 4u * ((2u * mt + (e & 1u)) * (unsigned)a.JHP + ww);
+    roff[r] = 4u * ((e >> 1) * (unsigned)a.job.ldw + 4u * ((2u * mt + (e & 1u)) * (unsigned)a.JHP + ww));
+    if (!ok) roff[r] = kNoRun;
     loff[r] = (unsigned)(4 * wave_tw<L>() + 4 * ww * WS) + 4u * (e * (unsigned)MT + mt);
   }
   auto load_runs = [&](int grp) {
     const int fld = grp / JH4, i0 = (grp % JH4) * kWaveBlock;
-    const float* base = W + (size_t)(a.job.col0 + a.job.fstride * fld) * a.job.ldw + 4 * i0;
+    const __amdgpu_buffer_rsrc_t rows = waist_rows(
+        W + (size_t)(a.job.col0 + a.job.fstride * fld) * a.job.ldw, a.job.ldw, i0);
 #pragma unroll
-    for (int r = 0; r < RU; ++r)
-      if (rvalid & (1u << r)) run[r] = *reinterpret_cast<const f4*>(base + roff[r]);
+    for (int r = 0; r < RU; ++r) run[r] = load_run(rows, roff[r]);
   };
   load_runs(g);
   fill_wave_twiddles<L>(tw, a.fft.tw64);
