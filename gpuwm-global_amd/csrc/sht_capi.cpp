@@ -119,13 +119,19 @@ void upload(DevBuf& buf, const std::vector<T>& host) {
   }
 }
 
-// Passes of the row FFT kernels for scalar fields: primes above 13 first, largest first (the
-// first pass of such a radix shares its sums between outputs and has no
-// twiddles), then the radices 2..16 of least modelled cost.  A pass costs its
+// Passes of the row FFT kernels for scalar fields: primes above 13 first,
+// largest first (the first pass of such a radix shares its sums between outputs
+// and has no twiddles), then the radices 2..16 of least modelled cost.  A pass costs its
 // LDS round trip (~100 wave instructions) plus, per round of 64 butterflies,
 // ~20 R for addresses, twiddles and LDS accesses and its DFT (direct for 5,
 // 7, 11, 13, ~5 R log2 R otherwise); with N = 1152 this takes 12 x 12 x 8
 // over 4 x 4 x 4 x 2 x 3 x 3.
+// Rounding: fewer passes round less, direct sums of 5..13 a little more.  In a
+// float32 emulation over 345 row lengths the FFT's rms error is 0.92 of the
+// passes 4, 2, 3 and direct sums' at the median and 1.08 at most (above 1.0 at
+// 21 lengths; no other order of the same radices does better).  On the device,
+// whole transforms: inverse 0.98 at the median, 1.02 at most; forward 0.97 and
+// 1.08.
 double pass_cost(int n, int r) {
   const int rounds = (n / r + 63) / 64;
   double dft = 5.0 * r * std::log2((double)r);
@@ -813,7 +819,9 @@ void add_ana_group(std::vector<HostGroup>& b, const arwen_sht_plan* P, int mb, i
 // the scalar operations, while their time stays below the grouped path's.
 // That grows with the fields and, through the gathers and the k chain of one
 // wavefront, with the square (synthesis) or the cube (analysis, whose results
-// leave in 8-byte pieces) of K = ceil((T+1)/64) k-chunks.  GPU time of a call
+// leave in 8-byte pieces) of K = ceil((T+1)/64) k-chunks.  A batch keeps the
+// grouped path whatever its jobs' sizes: there one launch serves all jobs of a
+// direction, and the lines below were measured for calls of one job.  GPU time of a call
 // either side of the lines, grouped -> few-column, us (float32; bf16x6 alike):
 //   synthesis, fields K^2 <= 72:   T127 16 fields 17.1 -> 13.1, T255 4 21.8 ->
 //     17.7, T383 2 31.8 -> 28.9
@@ -2082,17 +2090,24 @@ int arwen_sht_batch_autotune(arwen_sht_batch* B, void* stream, int reps,
       // split accumulators, is a candidate only where they are off.
       const bool wide = B->precision == ARWEN_SHT_FP32 || !B->config.split_acc;
       const std::vector<int> cols = wide ? std::vector<int>{32, 64, 96} : std::vector<int>{32, 64};
-      // one generation of resident blocks, or more that the hardware deals
-      const int grids[2] = {0, 256 * 8};
+      // one generation of resident blocks, or more, whose shorter queues the
+      // hardware deals as blocks end: best where the launch is long (bf16x6,
+      // 96 columns, synthesis + analysis ms at 0 / 2048 / 8192 / 32768: 32 x
+      // T383 4.85 / 5.29 / 5.08 / 4.57; 4 x T767 + 8 x T383 + 16 x T127 5.08 /
+      // 5.22 / 4.78 / 4.78; T767 1.11 / 1.06 / 1.10 / 1.10)
+      const int grids[5] = {0, 256 * 8, 256 * 16, 256 * 32, 256 * 128};
       for (int d = 0; d < 2; ++d) {
         if (B->lists[d].nitems == 0) continue;
         float best_ms = 0.f;
         for (int bn : cols) {
+          int timed = -1;  // workgroups of the last launch timed
           for (int gr : grids) {
             arwen_sht_gemm_config c = best;
             c.cols[d] = bn;
             c.grid[d] = gr;
             apply_config(B, c);
+            if (B->lists[d].grid == timed) continue;  // a queue for each item already
+            timed = B->lists[d].grid;
             hip_check(launch_gemm(B, d, s), "autotune warm-up");
             hip_check(hipEventRecord(e0, s), "hipEventRecord");
             for (int r = 0; r < reps; ++r) hip_check(launch_gemm(B, d, s), "autotune launch");

@@ -97,6 +97,24 @@ def test_schedule_configs_and_autotune_are_bit_identical(oracles, T, precision):
         assert torch.equal(v, ref[k]), ("autotuned", tuned, k)
 
 
+@pytest.mark.parametrize("precision", ["float32", "bf16x6"])
+def test_queues_of_any_length_are_bit_identical(oracles, precision):
+    """From one item a queue (more workgroups than items) to all of an XCD's
+    items in one queue, as the autotuner's grids give at other sizes."""
+    import torch
+
+    o = oracles[63]
+    _, batch, bufs = _round_trip(o, precision)
+    _run(batch)
+    ref = _outputs(bufs)
+    for grid in ((8192, 32768), (32768, 4096), (8, 8)):
+        batch.set_config(grid=grid)
+        assert batch.config()["grid"] == list(grid)
+        _run(batch)
+        for k, v in _outputs(bufs).items():
+            assert torch.equal(v, ref[k]), (grid, k)
+
+
 @pytest.mark.parametrize("T", [21, 63])
 def test_shared_accumulator_stays_within_tolerance(oracles, T):
     import torch
