@@ -530,24 +530,30 @@ constexpr int kXcds = 8;  // MI355X: 8 XCDs x 32 CUs
 // its table fragments through L1 once for its columns, so 64 halve that
 // traffic; they cost residency (two blocks per CU, not three) and padding.
 // They also come in generations of 512, which a launch of few does not fill.
-// A call, us, 32 against 64 columns (64-column items, padding to whole tiles):
-//   bf16x6 synthesis  T383 wind 40 levels (1692, 1.2) 204 : 195, 32 (1128, 1)
-//     168 : 162, 16 (564, 1) 101 : 102; T255 gradients of 40 fields on 768
-//     longitudes (1536, 1.6) 99.3 : 97.3, on 512 (1024, 1.6) 60.8 : 65.2
-//   bf16x6 analysis   T383 vorticity, divergence 40 levels (1122, 1.2) 204 : 194,
-//     24 (748, 1.33) 144 : 136; T255 40 levels on 768 longitudes (555, 1.2)
-//     141 : 145, on 512 91.9 : 97.1, 64 on 768 (740, 1) 207 : 196
-//   fp32 synthesis    T383 gradients of 32 fields (1152, 1) 112 : 107, of 40
-//     (2304, 1.6) 148 : 156; T255 wind 64 levels on 768 longitudes (1536, 1)
-//     162 : 155, on 512 (1024, 1) 101 : 103
+// What counts of the padding is what 64-column tiles have more of than
+// 32-column ones (80 columns: 128 against 96).  A call, us, 32 against 64
+// columns (64-column items, padded columns over the 32-column tiles'):
+//   bf16x6 synthesis  T383 60 fields (1152, 1) 114 : 103, 40 (1152, 1.33) 78.0 :
+//     78.3, gradients of 40 (2304, 1.33) 184 : 174, wind 40 levels (1692, 1.2)
+//     204 : 194; T287 wind 40 levels (1296, 1.2) 132 : 126; gradients of 40
+//     fields (1.33), T191 on 576 longitudes (1152) 90.3 : 96.3, T255 on 768
+//     (1536) 131 : 126; T255 60 fields (512, 1) 46.1 : 46.5
+//   bf16x6 analysis   T383 20 fields (384, 1) 49.9 : 47.0, vorticity, divergence
+//     40 levels (1128, 1.2) 205 : 195, 24 (752, 1.33) 141 : 136; T223 60 levels
+//     (640, 1) 129 : 120; T255 on 768 longitudes 40 levels (558, 1.2) 142 : 145
+//   fp32 synthesis    T383 gradients of 32 fields (1152, 1) 136 : 131, of 40
+//     (2304, 1.33) 178 : 185; T255 gradients of 64 (1024, 1) 112 : 109; T191 on
+//     576 longitudes, 20 MB of tables, wind 64 levels (1152, 1) 132 : 135
 //   fp32 analysis     T383 64 fields (774, 1) 118 : 118, 128 125 : 115 (kernel)
-// so: tables from half of the eight 4 MB L2s up; in the split modes about as many
-// items as run together with little or no padding, and more than two generations
-// (synthesis) or 700 items with more of it; in FP32, whose MFMA time weighs more,
-// more than two or four generations and hardly any padding.
+// so: tables from half of the eight 4 MB L2s up; in the split modes, with no
+// more padding about as many items as run together, with more of it more than
+// two generations (synthesis) or 700 (analysis); in FP32, whose MFMA time
+// weighs more, two generations (and tables of 24 MB) or four and hardly any
+// padding at all.  Over 2,336 calls of T106 to T383 this is 0.1% above the
+// better of the two at the mean and at most 4% above 32 columns.
 int default_cols(int dir, const std::vector<HostGroup>& groups, int precision) {
   const bool split = precision != ARWEN_SHT_FP32;
-  long long tiles = 0, used = 0, wide = 0, table = 0;
+  long long tiles = 0, used = 0, wide = 0, narrow = 0, table = 0;
   const int pieces = split ? (precision == ARWEN_SHT_BF16X6 ? 3 : 2) : 1;
   for (const HostGroup& g : groups) {
     int rows = 0;
@@ -556,15 +562,18 @@ int default_cols(int dir, const std::vector<HostGroup>& groups, int precision) {
     tiles += panels * nt;
     used += panels * g.N;
     wide += panels * nt * 64;
+    narrow += panels * ((g.N + 31) / 32) * 32;
     for (int sg = 0; sg < g.nseg; ++sg)
       for (int z = 0; z < g.mcount; ++z)
         table += (long long)g.K[sg][z] * g.Arows[sg][z] * (long long)g.esz * pieces;
   }
-  const bool fits = !split     ? 10 * wide <= 11 * used && tiles > (dir == 0 ? 1024 : 2047)
-                    : dir == 0 ? (4 * wide <= 5 * used && tiles >= 512) ||
-                                     (10 * wide <= 16 * used && tiles > 1024)
-                               : (20 * wide <= 21 * used && tiles >= 400) ||
-                                     (3 * wide <= 4 * used && tiles >= 700);
+  const bool same = 50 * wide <= 51 * narrow;  // hardly more padding than 32-column tiles
+  const bool fits =
+      !split     ? 10 * wide <= 11 * used &&
+                       (dir == 0 ? tiles >= 1024 && table >= (24ll << 20) : tiles > 2047)
+      : dir == 0 ? (same && tiles >= 512) || (4 * wide <= 5 * narrow && tiles >= 1200) ||
+                       (3 * wide <= 4 * narrow && tiles >= 1300)
+                 : (same && tiles >= 380) || (3 * wide <= 4 * used && tiles >= 700);
   return fits && table >= (16ll << 20) ? 64 : 32;
 }
 
