@@ -3,12 +3,12 @@
 Drop-in for the reference's ``arwen_global.spectral.sampling``
 (src/arwen_global/spectral/sampling.py): same functions, arguments, error
 conditions and result layout ``(*lead, *point_shape)`` float64.  Every call
-is one pack and one launch of ``libarwen_sht.so``'s point sampler: one lane
-per point runs the FP64 normalized recurrence (the reference's operand
-order) and multiply-adds a tile of fields' coefficients into per-order
-amplitudes; nothing the size of the reference's (2K x points) basis is
-materialised, so ``chunk_points`` only bounds a launch and never the
-arithmetic of a point.
+is one pack and one launch of ``libarwen_sht.so``'s point sampler (and the
+ordered sum of its parts): a wavefront runs the FP64 normalized recurrence of
+16 or more points (the reference's operand order) and multiplies it into tiles
+of fields' coefficients on the matrix cores, one amplitude per order; nothing
+the size of the reference's (2K x points) basis is materialised, so
+``chunk_points`` only bounds a launch and never the arithmetic of a point.
 """
 from __future__ import annotations
 

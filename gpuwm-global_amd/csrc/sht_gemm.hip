@@ -37,12 +37,14 @@
 // workgroup its queue, an item's LDS list ends with the next item's first
 // three steps (null steps, extent 0, where there is none), so the last trip's
 // loads are the next item's, and they are in flight while the outputs are
-// stored.  What bounds the launch is what it moves: the tables and data once
-// from memory, and 12 KB of table per 64-column step through L1; without
-// MFMAs it takes the same time.  T383 bf16x6, 160 columns, 64-column tiles:
-// 69.4 / 77.5 us (synthesis / analysis) with a prologue of 4-5 us per tile
-// (panel, list, first tiles, each waited on) and list order, 66.6 / 72.0 us
-// here; 96-column analysis 78.4 -> 69.5 us.
+// stored.  The split synthesis is bound by what it moves (12 KB of table per
+// step reach each block's registers through L1, for the tables once from
+// memory) and by the loads' latency, not by its MFMAs: with every MFMA
+// replaced by one vector operation on its operands it takes the same time
+// (T383 wind, 160 columns, 64-column tiles: 62.4 against 62.2 us).  The same
+// launch and its analysis took 69.4 / 77.5 us with a prologue of 4-5 us per
+// tile (panel, list, first tiles, each waited on) and list order, 66.6 / 72.0
+// us from the queues on the same card; 96-column analysis 78.4 -> 69.5 us.
 //
 // LDS B tiles are unpadded rows of 32 k, one row per column (128 bytes fp32,
 // 64 bytes per bf16 piece), whose 16-byte chunks are XOR-swizzled by row, so

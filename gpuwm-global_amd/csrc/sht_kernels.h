@@ -249,7 +249,7 @@ static_assert(sizeof(GemmItem) == 32 && sizeof(GemmPanel) == 64, "as the kernel 
 static_assert(sizeof(GemmStep) == 32, "GemmStep is one 8-dword scalar load");
 
 // One grouped-GEMM launch: precision mode, direction (0 SYN, 1 ANA), column
-// tile (32 or 64), separate accumulators for the small split products.
+// tile (32, 64 or 96), separate accumulators for the small split products.
 struct GemmLaunch {
   int mode, dir, bn, acc2;
   const GemmPanel* panels;

@@ -37,11 +37,13 @@
 // Bound: the phases of a wavefront in turn, its loads, its MFMAs (their time
 // at full rate is a third of the call at 40 levels) and its stores; with every
 // MFMA taken out the solve is 32 us, near the HBM time of its planes.
-// Measured at T383, 40 levels (former form, matrix rows against register
-// columns by fma): solve 79 -> 48 us, apply 100 -> 57, tendencies 47 -> 37,
-// half map 215 -> 79.  A wavefront of 8 orders (real and imaginary parts in
-// one tile, six wavefronts per SIMD instead of four) takes 66 and 101 us for
-// solve and half map: its loads and stores are 64-byte pieces.
+// Measured at T383 (former form, matrix rows against register columns by fma
+// -> here; us a call, events around many; by card): 40 levels solve 79 ->
+// 47-50, apply 100 -> 56-60, tendencies 47 -> 37-39, half map 215 -> 76-80; 64
+// levels here 116, 139, 85 and 200.  A wavefront of 8 orders (real and
+// imaginary parts in one tile, six wavefronts per SIMD instead of four) takes
+// 66 and 101 us for solve and half map: its loads and stores are 64-byte
+// pieces.
 #include <algorithm>
 
 #include "sht_kernels.h"
@@ -313,10 +315,9 @@ hipError_t launch_vertical(const sht::VerticalArgs& a, hipStream_t s) {
   const size_t lds = (size_t)slots * sht::vertical_slot<NT>() * sizeof(float);
   const int T1 = a.T + 1;
   // Wavefronts (16 orders each) per block: eight, which share one copy of the
-  // matrices, or as many as the degree has orders for.  At T383: four take
-  // 52 (solve) and 90 us (half map) at 40 levels and 70 and 175 us at 64,
-  // eight 52 and 82, 64 and 108; five or six spread unevenly over a CU's four
-  // SIMDs (62-73 us).  From 32 levels on, also eight where a degree has fewer
+  // matrices, or as many as the degree has orders for.  At T383, 40 levels:
+  // four take 52 (solve) and 90 us (half map), eight 52 and 82 on the same
+  // card; five or six spread unevenly over a CU's four SIMDs (62-73 us).  From 32 levels on, also eight where a degree has fewer
   // orders (T <= 63): the others only stage, most of the time of such a launch
   // (half map, T31: 40 levels 24.3 -> 19.0 us a call, 64 levels 53.9 -> 32.5).
   const int waves = T1 <= 64 && NT >= 3 ? 8 : std::min(8, (T1 + 15) / 16);

@@ -362,7 +362,7 @@ typedef struct arwen_sht_gemm_config {
 int arwen_sht_batch_get_config(const arwen_sht_batch* batch, arwen_sht_gemm_config* out);
 int arwen_sht_batch_set_config(arwen_sht_batch* batch, const arwen_sht_gemm_config* config);
 /* Autotuner: times each direction's GEMM launch `reps` times on `stream` for
- * every column tile and grid, keeps the fastest and returns it in `out`
+ * every column tile and several grids, keeps the fastest and returns it in `out`
  * (optional).  Synchronizes; overwrites the batch's intermediate buffers. */
 int arwen_sht_batch_autotune(arwen_sht_batch* batch, void* stream, int reps,
                              arwen_sht_gemm_config* out);
